@@ -1022,8 +1022,63 @@ __global__ __launch_bounds__(WG) void k_rp_sym(const F *__restrict__ x, int64_t 
 }
 
 // ---------------------------------------------------------------- k_rr
+// Recurrences of one 32-row block of a lane's column (packed ranks R) for
+// every threshold, over the pairs i <= j of the segment.  Pair weight: 2 if
+// i < j, 1 if i == j.  non[t] collects the block's non-recurrent and
+// uncounted steps (one bit count per threshold; blk32 is the 32 steps of every
+// block counted so far, so blk32 - non[t] pairs recur with i < j): rows on or
+// below the diagonal, past the segment or of a column past N_c are forced to
+// the largest rank.  Diagonal elements, in the blocks that hold any, are
+// counted straight into acc (LDS).
+template <int TG>
+__device__ __forceinline__ void count_block(const uint32_t (&R)[8], uint32_t (&non)[TG], uint32_t &blk32, int nt,
+                                            int64_t i0, int64_t ie, int64_t j0, int64_t j, bool jv,
+                                            unsigned long long *acc) {
+    constexpr int B = rank_bits<TG>();
+    const int64_t nr64 = ie - i0;
+    const uint32_t mrow = nr64 >= BLK ? 0xFFFFFFFFu : ((1u << nr64) - 1u);
+    const bool diag = i0 + BLK > j0;   // the block reaches the band's diagonal (wave-uniform)
+    const int64_t du = j - i0;         // step index of the diagonal element
+    uint32_t mup = jv ? mrow : 0u;
+    if (diag) mup &= du >= BLK ? 0xFFFFFFFFu : (du <= 0 ? 0u : ((1u << du) - 1u));
+    uint32_t Pl[B];
+    {
+        rank_planes<B>(R, Pl, 0xFFFFFFFFu, ~mup);
+        const GeTree<B> G(Pl);
+        blk32 += BLK;
+#pragma unroll
+        for (int t = 0; t < TG; t++)
+            if (t < nt) non[t] += __popc(G.ge(t + 1));
+    }
+    if (diag) {
+        const uint32_t mdg = (jv && du >= 0 && du < BLK) ? (1u << du) & mrow : 0u;
+        rank_planes<B>(R, Pl, 0xFFFFFFFFu, ~mdg);
+        const GeTree<B> G(Pl);
+#pragma unroll
+        for (int t = 0; t < TG; t++)
+            if (t < nt) {
+                const unsigned long long w = __builtin_amdgcn_ballot_w64(G.ge(t + 1) != 0xFFFFFFFFu);
+                if (w && (threadIdx.x & (WAVE - 1)) == 0) atomicAdd(&acc[t], (unsigned long long)__popcll(w));
+            }
+    }
+}
+
+// The lane counts of an item, added to the workgroup's totals.
+template <int TG>
+__device__ __forceinline__ void count_item(const uint32_t (&non)[TG], uint32_t blk32, int nt,
+                                           unsigned long long *acc) {
+#pragma unroll
+    for (int t = 0; t < TG; t++) {
+        if (t < nt) {
+            unsigned long long v = 2ull * (blk32 - non[t]);
+            for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+            if ((threadIdx.x & (WAVE - 1)) == 0 && v) atomicAdd(&acc[t], v);
+        }
+    }
+}
+
 // Work item = (band of 64 columns, row segment q) over rows i <= max column
-// of the band.  Pair weight: 2 if i < j, 1 if i == j, 0 otherwise.
+// of the band.
 template <typename F, int NORM, int TG>
 __global__ __launch_bounds__(WG) void k_rr(const F *__restrict__ x, int64_t nc, int tau, int m, Bounds<F, TG> S,
                                            int nt, const LutEntry<F> *__restrict__ lut, LutParams P, int seg_len,
@@ -1038,7 +1093,6 @@ __global__ __launch_bounds__(WG) void k_rr(const F *__restrict__ x, int64_t nc, 
     __syncthreads();
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
-    constexpr int B = rank_bits<TG>();
 
     for (int64_t item = (int64_t)blockIdx.x * WAVES + wave; item < nitems; item += (int64_t)gridDim.x * WAVES) {
         const int2 it = items[item];
@@ -1049,9 +1103,9 @@ __global__ __launch_bounds__(WG) void k_rr(const F *__restrict__ x, int64_t nc, 
         const int64_t ib = (int64_t)it.y * seg_len;
         const int64_t ie = ib + seg_len < rows ? ib + seg_len : rows;
 
-        uint32_t c2[TG], c1[TG];
+        uint32_t non[TG], blk32 = 0;
 #pragma unroll
-        for (int t = 0; t < TG; t++) c2[t] = c1[t] = 0;
+        for (int t = 0; t < TG; t++) non[t] = 0;
 
         for (int64_t i0 = ib; i0 < ie; i0 += BLK) {
             F s[BLK];
@@ -1067,32 +1121,9 @@ __global__ __launch_bounds__(WG) void k_rr(const F *__restrict__ x, int64_t nc, 
             }
             uint32_t R[8];
             pack_ranks<F, TG>(s, R, lut_s, P, bnd_s, nt);
-            uint32_t Pl[B];
-            rank_planes<B>(R, Pl);
-            const GeTree<B> G(Pl);
-            // rows i0+u with u < nrow are in the segment; weight 2 for i < j, 1 for i == j
-            const int64_t nr64 = ie - i0;
-            const uint32_t mrow = nr64 >= BLK ? 0xFFFFFFFFu : ((1u << nr64) - 1u);
-            const int64_t du = j - i0;   // step index of the diagonal element
-            const uint32_t mup = !jv ? 0u : (du >= BLK ? 0xFFFFFFFFu : (du <= 0 ? 0u : ((1u << du) - 1u)));
-            const uint32_t mdg = (jv && du >= 0 && du < BLK) ? (1u << du) : 0u;
-#pragma unroll
-            for (int t = 0; t < TG; t++) {
-                if (t < nt) {
-                    const uint32_t w = ~G.ge(t + 1) & mrow;
-                    c2[t] += __popc(w & mup);
-                    c1[t] += __popc(w & mdg);
-                }
-            }
+            count_block<TG>(R, non, blk32, nt, i0, ie, j0, j, jv, acc);
         }
-#pragma unroll
-        for (int t = 0; t < TG; t++) {
-            if (t < nt) {
-                unsigned long long v = 2ull * c2[t] + c1[t];
-                for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
-                if (lane == 0 && v) atomicAdd(&acc[t], v);
-            }
-        }
+        count_item<TG>(non, blk32, nt, acc);
     }
     __syncthreads();
     for (int e = threadIdx.x; e < nt; e += WG)
@@ -1247,13 +1278,15 @@ __device__ __forceinline__ MxScale mx_scale(const unsigned int *__restrict__ nma
 
 // n_i = sum_k x[i + k tau]^2 (fp64, rounded to fp32); entries nc .. nc+127 = 0.
 // nmax_bits: atomic max of the float bits (non-negative floats order as uints;
-// NaN bits are above +inf, so a NaN norm forces the all-exact fallback).
+// NaN bits are above +inf, so a NaN norm forces the all-exact fallback), one
+// per workgroup of NRT threads.
+constexpr int NRT = 256;
 template <typename F>
-__global__ void k_norms(const F *__restrict__ x, int64_t nc, int tau, int m, float *__restrict__ nrm,
-                        unsigned int *__restrict__ nmax_bits) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc + 2 * WAVE) return;
+__global__ __launch_bounds__(NRT) void k_norms(const F *__restrict__ x, int64_t nc, int tau, int m,
+                                               float *__restrict__ nrm, unsigned int *__restrict__ nmax_bits) {
+    const int64_t i = (int64_t)blockIdx.x * NRT + threadIdx.x;
     float v = 0.f;
+    uint32_t top = 0u;
     if (i < nc) {
         double a = 0.0;
         for (int k = 0; k < m; k++) {
@@ -1262,9 +1295,17 @@ __global__ void k_norms(const F *__restrict__ x, int64_t nc, int tau, int m, flo
         }
         v = (float)a;
         const float mag = fabsf(v);
-        atomicMax(nmax_bits, __float_as_uint(mag > 1e30f || mag != mag ? __int_as_float(0x7F800000) : mag));
+        top = __float_as_uint(mag > 1e30f || mag != mag ? __int_as_float(0x7F800000) : mag);
     }
-    nrm[i] = v;
+    if (i < nc + 2 * WAVE) nrm[i] = v;
+    __shared__ uint32_t wtop[NRT / WAVE];
+    for (int off = WAVE / 2; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
+    if ((threadIdx.x & (WAVE - 1)) == 0) wtop[threadIdx.x / WAVE] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < NRT / WAVE; w++) top = max(top, wtop[w]);
+        if (top) atomicMax(nmax_bits, top);
+    }
 }
 
 // Byte table.  Bucket without any bound within E_max of its value range:
@@ -1648,6 +1689,71 @@ __device__ __forceinline__ void tile_row_norms(const float *__restrict__ nrm, in
     }
 }
 
+// Ranks of one 32-row block against the band's 64 columns (both Gram tiles;
+// windows in Wn), exact: R holds the lane's own column j0 + lane in the scan's
+// packed layout.  nb: rows of the block that belong to the segment.  rowm:
+// this lane's elements on those rows; flw0, flw1: the tiles' flagged elements
+// (mx_tile layout) and amb: the elements re-decided in exact order (for the
+// decision counters).
+template <typename F, int TG, int G>
+__device__ __forceinline__ void mx_block(const MxWin<2> &Wn, const float *const (&pa)[8], const F *__restrict__ x,
+                                         const float *__restrict__ nrm, int64_t i0, int64_t j0, int nb, int64_t nc,
+                                         int tau, int m, int nt, const uint8_t *lut_s, const MxParams &P,
+                                         const MxScale &Z, const float *bnd_s, const F *bndx, uint32_t (&R)[8],
+                                         uint32_t &rowm, uint32_t &flw0, uint32_t &flw1, uint32_t &amb) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int col = lane & 31;
+    const int h = lane >> 5;
+    float ni[16];
+    tile_row_norms(nrm, i0, h, ni);
+    // real rows of this lane's elements (rows past the segment are
+    // padding); all of them but in a segment's last block
+    rowm = 0xFFFFu;
+    if (nb < BLK) {
+        rowm = 0u;
+#pragma unroll
+        for (int e = 0; e < 16; e++) rowm |= ((8 * (e >> 2) + 4 * h + (e & 3)) < nb ? 1u : 0u) << e;
+    }
+    uint32_t Rr[8], fm = 0u;
+    {
+        const floatx16 acc = gram_tile<2, 0, G>(Wn, pa, col, h, m, tau);
+        uint32_t Rq[4], f;
+        tile_ranks(acc, ni, nrm[j0 + col], lut_s, P, Z, bnd_s, Rq, f, flw0);
+#pragma unroll
+        for (int c = 0; c < 4; c++) Rr[c] = Rq[c];
+        if (j0 + col < nc) fm |= f & rowm;
+    }
+    {
+        const floatx16 acc = gram_tile<2, 1, G>(Wn, pa, col, h, m, tau);
+        uint32_t Rq[4], f;
+        tile_ranks(acc, ni, nrm[j0 + 32 + col], lut_s, P, Z, bnd_s, Rq, f, flw1);
+#pragma unroll
+        for (int c = 0; c < 4; c++) Rr[4 + c] = Rq[c];
+        if (j0 + 32 + col < nc) fm |= (f & rowm) << 16;
+    }
+    amb = fm;
+    // exact re-decision of the ambiguous elements by their own lane
+    while (fm) {
+        const uint32_t b = __builtin_ctz(fm);
+        fm &= fm - 1u;
+        const uint32_t e = b & 15u, p = b >> 4;
+        const F sx = exact_sqdist<F>(x, i0 + 4 * h + 8 * (e >> 2) + (e & 3), j0 + 32 * p + col, tau, m);
+        const uint32_t rk = rank_direct<F, TG>(sx, bndx, nt);
+        const uint32_t c = 4 * p + (e & 3), sh = 8 * (e >> 2), keep = ~(0xFFu << sh), val = rk << sh;
+#pragma unroll
+        for (int cc = 0; cc < 8; cc++)
+            if (c == (uint32_t)cc) Rr[cc] = (Rr[cc] & keep) | val;
+    }
+    // one swap per register: half 0 keeps tile 0 rows 8g+c and gets
+    // tile 0 rows 8g+4+c from its partner; half 1 the same for tile 1
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const auto sw = __builtin_amdgcn_permlane32_swap(Rr[c], Rr[4 + c], false, false);
+        R[c] = sw[0];
+        R[4 + c] = sw[1];
+    }
+}
+
 // ---------------------------------------------------------------- k_lam_mx
 // LAM pass of the MFMA form.  Work item = (band of 64 columns, row segment).
 // Per 32-row block two 32x32 Gram tiles (columns j0..j0+31, then j0+32..j0+63)
@@ -1761,34 +1867,9 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
             const bool more = i0 + BLK < ie;
             pre0 = more && lane < rspan ? x[i0 + BLK + lane] : 0.f;
             pre1 = more && lane + WAVE < rspan ? x[i0 + BLK + WAVE + lane] : 0.f;
-            float ni[16];
-            tile_row_norms(nrm, i0, h, ni);
-            // real rows of this lane's elements (rows past the segment are
-            // padding); all of them but in a segment's last block
-            uint32_t rowm = 0xFFFFu;
-            if (nb < BLK) {
-                rowm = 0u;
-#pragma unroll
-                for (int e = 0; e < 16; e++) rowm |= ((8 * (e >> 2) + 4 * h + (e & 3)) < nb ? 1u : 0u) << e;
-            }
-            uint32_t Rr[8], fm = 0u;
-            uint32_t flw0, flw1;
-            {
-                const floatx16 acc = gram_tile<2, 0, G>(Wn, pa, col, h, m, tau);
-                uint32_t Rq[4], f;
-                tile_ranks(acc, ni, nrm[j0 + col], lut_s, P, Z, bnd_s, Rq, f, flw0);
-#pragma unroll
-                for (int c = 0; c < 4; c++) Rr[c] = Rq[c];
-                if (j0 + col < nc) fm |= f & rowm;
-            }
-            {
-                const floatx16 acc = gram_tile<2, 1, G>(Wn, pa, col, h, m, tau);
-                uint32_t Rq[4], f;
-                tile_ranks(acc, ni, nrm[j0 + 32 + col], lut_s, P, Z, bnd_s, Rq, f, flw1);
-#pragma unroll
-                for (int c = 0; c < 4; c++) Rr[4 + c] = Rq[c];
-                if (j0 + 32 + col < nc) fm |= (f & rowm) << 16;
-            }
+            uint32_t R[8], rowm, flw0, flw1, amb;
+            mx_block<F, TG, G>(Wn, pa, x, nrm, i0, j0, nb, nc, tau, m, nt, lut_s, P, Z, bnd_s, bndx, R, rowm, flw0, flw1,
+                               amb);
             if constexpr (STATS) {
                 // flag words to element bits (element e <-> bit 8(e>>2) + (e&3))
                 uint32_t e0 = 0, e1 = 0;
@@ -1800,28 +1881,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
                 const uint32_t v0 = j0 + col < nc ? rowm : 0u, v1 = j0 + 32 + col < nc ? rowm : 0u;
                 st_rank += __builtin_popcount(v0) + __builtin_popcount(v1);
                 st_flag += __builtin_popcount(e0 & v0) + __builtin_popcount(e1 & v1);
-                st_exact += __builtin_popcount(fm);
-            }
-            // exact re-decision of the ambiguous elements by their own lane
-            while (fm) {
-                const uint32_t b = __builtin_ctz(fm);
-                fm &= fm - 1u;
-                const uint32_t e = b & 15u, p = b >> 4;
-                const F sx = exact_sqdist<F>(x, i0 + 4 * h + 8 * (e >> 2) + (e & 3), j0 + 32 * p + col, tau, m);
-                const uint32_t rk = rank_direct<F, TG>(sx, bndx, nt);
-                const uint32_t c = 4 * p + (e & 3), sh = 8 * (e >> 2), keep = ~(0xFFu << sh), val = rk << sh;
-#pragma unroll
-                for (int cc = 0; cc < 8; cc++)
-                    if (c == (uint32_t)cc) Rr[cc] = (Rr[cc] & keep) | val;
-            }
-            // one swap per register: half 0 keeps tile 0 rows 8g+c and gets
-            // tile 0 rows 8g+4+c from its partner; half 1 the same for tile 1
-            uint32_t R[8];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const auto sw = __builtin_amdgcn_permlane32_swap(Rr[c], Rr[4 + c], false, false);
-                R[c] = sw[0];
-                R[4 + c] = sw[1];
+                st_exact += __builtin_popcount(amb);
             }
             if (tiles) store_tile(tiles, i0 / BLK, band, nbands, R);
             if constexpr (SCAN) {
@@ -1846,6 +1906,84 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
         if (st_flag) atomicAdd(&stats[1], (unsigned long long)st_flag);
         if (st_exact) atomicAdd(&stats[2], (unsigned long long)st_exact);
     }
+}
+
+// ---------------------------------------------------------------- k_rr_mx
+// RR asked alone, MFMA form: the pairs i <= j ranked as in k_lam_mx (mx_block)
+// and counted as in k_rr (count_block), nothing stored.  Bound by VALU issue:
+// ranking about 10 and counting 2 + 2 T / 32 lane-operations a pair, against
+// 3m + 8 of the exact sums.  The threshold search at N_c = 65,536, m = 16 (one
+// pass of 3 thresholds, four of 31): 15.3 ms with k_rr, 6.4 ms with this.  fp32
+// and fp64 input as in k_lam_mx.
+template <typename F, int TG>
+__global__ __launch_bounds__(WG) RQA_WPE_MX(false) void k_rr_mx(
+    const F *__restrict__ x, const float *__restrict__ nrm, const unsigned int *__restrict__ nmax_bits, int64_t nc,
+    int tau, int m, Bounds<float, TG> S, Bounds<F, TG> SX, int nt, const uint8_t *__restrict__ lut, MxParams P,
+    int seg_len, const int2 *__restrict__ items, int64_t nitems, unsigned long long *__restrict__ counts) {
+    __shared__ unsigned long long acc[TG];
+    __shared__ uint8_t lut_s[NBX_LAM];
+    __shared__ float bnd_s[NBND];
+    __shared__ F bndx_s[sizeof(F) == 8 ? NBND : 1];
+    __shared__ MxWin<2> win[WAVES];
+    for (int e = threadIdx.x; e < TG; e += WG) acc[e] = 0;
+    for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
+    if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, nt, S.s);
+    if constexpr (sizeof(F) == 8)
+        if (threadIdx.x < NBND) bndx_s[threadIdx.x] = (int)threadIdx.x < nt ? SX.s[threadIdx.x] : (F)__builtin_inf();
+    const F *bndx;
+    if constexpr (sizeof(F) == 8)
+        bndx = bndx_s;
+    else
+        bndx = bnd_s;
+    __syncthreads();
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = wave_id();
+    const int col = lane & 31;
+    const int h = lane >> 5;
+    const int rspan = 32 + (m - 1) * tau;   // <= MXW (checked by the host)
+    const int cspan = 64 + (m - 1) * tau;   // <= MXW + 32
+    MxWin<2> &Wn = win[wave];
+    float *rw = Wn.rw, *cw = Wn.cw;
+    mx_win_init(Wn, lane);
+    const float *pa[8];
+    gram_addrs(Wn, col, h, m, tau, pa);
+    const MxScale Z = mx_scale(nmax_bits, P);
+
+    for (int64_t item = (int64_t)blockIdx.x * WAVES + wave; item < nitems; item += (int64_t)gridDim.x * WAVES) {
+        const int2 it = items[item];
+        const int64_t j0 = (int64_t)it.x * WAVE;
+        const int64_t j = j0 + lane;
+        const bool jv = j < nc;
+        const int64_t rows = min(j0 + WAVE, nc);
+        const int64_t ib = (int64_t)it.y * seg_len;
+        const int64_t ie = min(ib + (int64_t)seg_len, rows);
+        uint32_t non[TG], blk32 = 0;
+#pragma unroll
+        for (int t = 0; t < TG; t++) non[t] = 0;
+
+        // windows as in k_lam_mx: columns once per item, rows one block ahead
+        for (int e = lane; e < cspan; e += WAVE) cw[e] = hl_word((float)x[j0 + e] * Z.s);
+        float pre0 = lane < rspan ? x[ib + lane] : 0.f;
+        float pre1 = lane + WAVE < rspan ? x[ib + WAVE + lane] : 0.f;
+        for (int64_t i0 = ib; i0 < ie; i0 += BLK) {
+            const int nb = ie - i0 < BLK ? (int)(ie - i0) : BLK;
+            wave_sync();
+            if (lane < rspan) rw[lane] = hl_word(pre0 * Z.s);
+            if (lane + WAVE < rspan) rw[WAVE + lane] = hl_word(pre1 * Z.s);
+            wave_sync();
+            const bool more = i0 + BLK < ie;
+            pre0 = more && lane < rspan ? x[i0 + BLK + lane] : 0.f;
+            pre1 = more && lane + WAVE < rspan ? x[i0 + BLK + WAVE + lane] : 0.f;
+            uint32_t R[8], rowm, flw0, flw1, amb;
+            mx_block<F, TG, GRAM_HILO>(Wn, pa, x, nrm, i0, j0, nb, nc, tau, m, nt, lut_s, P, Z, bnd_s, bndx, R, rowm,
+                                       flw0, flw1, amb);
+            count_block<TG>(R, non, blk32, nt, i0, ie, j0, j, jv, acc);
+        }
+        count_item<TG>(non, blk32, nt, acc);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < nt; e += WG)
+        if (acc[e]) glob_add(&counts[e], acc[e]);
 }
 
 // ---------------------------------------------------------------- k_rp_mx

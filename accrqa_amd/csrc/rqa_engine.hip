@@ -937,12 +937,34 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
     if (want_rr && !want_lam) {
         fill_zero(counts, 32, st);
         const int64_t ni = c.n_items_rr;
-        prof_begin("k_rr", st);
-        hipLaunchKernelGGL((rqa::k_rr<F, NORM, TG>), dim3(grid_for(rqa::k_rr<F, NORM, TG>, ni, c.ncu)), dim3(rqa::WG), 0,
-                           st, dx, nc, tau, m,
-                           B, nt, d_lut, P, L, (const int2 *)c.items_rr.p, ni, counts);
-        prof_end(st);
-        HIP_TRY(hipGetLastError());
+        bool done = false;
+        if constexpr (NORM == 1) {
+            if (use_mfma<F>(1, m, tau)) {
+                rqa::Bounds<float, TG> Bf;
+                for (int t = 0; t < TG; t++) Bf.s[t] = (float)B.s[t];
+                const rqa::MxParams MP = mx_params(Bf.s, nt, m, rqa::NBX_LAM, sizeof(F) == 8 ? 4 : 0);
+                if ((e = ensure(c.lut8, rqa::NBX_LAM))) return e;
+                hipLaunchKernelGGL((rqa::k_mx_lut<TG>), dim3((MP.nb + 255) / 256), dim3(256), 0, st, Bf, nt, MP,
+                                   (const unsigned int *)c.nmax.p, (uint8_t *)c.lut8.p);
+                HIP_TRY(hipGetLastError());
+                prof_begin("k_rr_mx", st);
+                hipLaunchKernelGGL((rqa::k_rr_mx<F, TG>), dim3(grid_for(rqa::k_rr_mx<F, TG>, ni, c.ncu)),
+                                   dim3(rqa::WG), 0, st, dx, (const float *)c.nrm.p, (const unsigned int *)c.nmax.p,
+                                   nc, tau, m, Bf, B, nt, (const uint8_t *)c.lut8.p, MP, L,
+                                   (const int2 *)c.items_rr.p, ni, counts);
+                prof_end(st);
+                HIP_TRY(hipGetLastError());
+                done = true;
+            }
+        }
+        if (!done) {
+            prof_begin("k_rr", st);
+            hipLaunchKernelGGL((rqa::k_rr<F, NORM, TG>), dim3(grid_for(rqa::k_rr<F, NORM, TG>, ni, c.ncu)),
+                               dim3(rqa::WG), 0, st, dx, nc, tau, m, B, nt, d_lut, P, L,
+                               (const int2 *)c.items_rr.p, ni, counts);
+            prof_end(st);
+            HIP_TRY(hipGetLastError());
+        }
     }
 
     if (want_lam || want_det) {
@@ -1265,8 +1287,8 @@ int run_block(const F *dx, size_t n, int tau, int emb, const F *thr, int T, cons
         if ((e = ensure(c.nmax, 256))) return e;
         fill_zero((unsigned long long *)c.nmax.p, 1, st);
         const int64_t nthr = nc + 2 * rqa::WAVE;
-        hipLaunchKernelGGL((rqa::k_norms<F>), dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, st, dx, nc,
-                           tau, emb, (float *)c.nrm.p, (unsigned int *)c.nmax.p);
+        hipLaunchKernelGGL((rqa::k_norms<F>), dim3((unsigned)((nthr + rqa::NRT - 1) / rqa::NRT)), dim3(rqa::NRT), 0, st,
+                           dx, nc, tau, emb, (float *)c.nrm.p, (unsigned int *)c.nmax.p);
         HIP_TRY(hipGetLastError());
     }
 
@@ -1526,8 +1548,8 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
             if ((e = ensure(c.lut8, rqa::NBX_LAM))) return e;
             fill_zero((unsigned long long *)c.nmax.p, 1, st);
             const int64_t nthr = nc + 2 * rqa::WAVE;
-            hipLaunchKernelGGL((rqa::k_norms<F>), dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, st, dx, nc, tau,
-                               emb, (float *)c.nrm.p, (unsigned int *)c.nmax.p);
+            hipLaunchKernelGGL((rqa::k_norms<F>), dim3((unsigned)((nthr + rqa::NRT - 1) / rqa::NRT)), dim3(rqa::NRT), 0, st,
+                               dx, nc, tau, emb, (float *)c.nrm.p, (unsigned int *)c.nmax.p);
             HIP_TRY(hipGetLastError());
             rqa::Bounds<float, 4> Bf;
             for (int t = 0; t < 4; t++) Bf.s[t] = (float)b;
