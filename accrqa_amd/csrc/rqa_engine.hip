@@ -1118,6 +1118,33 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
         if (nc > 1) {
             const int64_t ni = c.n_items_det;
             bool done = false;
+            if constexpr (NORM == 1) {
+                // DET asked alone, MFMA form: rank the upper triangle once into
+                // the tile store (when it fits) and scan the tiles, instead of
+                // three Gram tiles per two of pairs and a scan at three waves
+                // per SIMD (k_det_mx): N = 100,003, m = 32, 16 thresholds,
+                // 9.0 -> 6.4 ms.
+                if (!tiles && !want_lam && g_split == 0 && use_mfma<F>(1, m, tau) && tile_store_fits(nc)) {
+                    rqa::Bounds<float, TG> Bf;
+                    for (int t = 0; t < TG; t++) Bf.s[t] = (float)B.s[t];
+                    const rqa::MxParams MP = mx_params(Bf.s, nt, m, rqa::NBX_LAM, sizeof(F) == 8 ? 4 : 0);
+                    if ((e = ensure(c.tiles, tile_store_bytes(nc)))) return e;
+                    if ((e = ensure(c.lut8, rqa::NBX_LAM))) return e;
+                    tiles = (uint8_t *)c.tiles.p;
+                    hipLaunchKernelGGL((rqa::k_mx_lut<TG>), dim3((MP.nb + 255) / 256), dim3(256), 0, st, Bf, nt, MP,
+                                       (const unsigned int *)c.nmax.p, (uint8_t *)c.lut8.p);
+                    HIP_TRY(hipGetLastError());
+                    const rqa::LamWork RW{(const int2 *)c.items_lamv.p, c.n_items_lamv, nseg, 2 * nseg};
+                    const unsigned g = grid_for(rqa::k_lam_mx<F, TG, false>, RW.nitems, c.ncu);
+                    prof_begin("k_lam_mx", st);
+                    hipLaunchKernelGGL((rqa::k_lam_mx<F, TG, false>), dim3(g), dim3(rqa::WG), 0, st, dx,
+                                       (const float *)c.nrm.p, (const unsigned int *)c.nmax.p, nc, tau, m, Bf, B, nt,
+                                       (const uint8_t *)c.lut8.p, MP, L, RW, hist, carry, (uint32_t *)c.priv.p, tiles,
+                                       (unsigned long long *)nullptr);
+                    prof_end(st);
+                    HIP_TRY(hipGetLastError());
+                }
+            }
             if (tiles) {
                 const int64_t nig = c.n_items_dets;
                 const size_t pd = lds_cap_pad(rqa::k_det_scan<TG>, g_scan_waves);
