@@ -145,7 +145,7 @@ FORM_AUTO, FORM_EXACT, FORM_MFMA = 0, 1, 2
 
 def set_form(form):
     """Euclidean distance form: FORM_AUTO (MFMA Gram + exact recheck for
-    m >= 8), FORM_EXACT (exact VALU sums only) or FORM_MFMA (MFMA form wherever
+    m >= 8, m >= 4 for plots of bytes with N_c > 16384), FORM_EXACT (exact VALU sums only) or FORM_MFMA (MFMA form wherever
     it applies: fp32 input, and fp64 input in the LAM pass with the Gram of
     the series rounded to fp32 and an fp64 recheck).  The Gram runs on FP16
     matrix cores with each sample split into two halves (hi/lo).  Results are identical; only
@@ -217,10 +217,9 @@ def set_rp_wide(on):
 
 
 def set_rp_sym(on):
-    """Recurrence plot of bytes, both forms: the upper triangle only, each
-    64 x 64 square stored mirrored as well, where N_c % 16 == 0 and the plot
-    is 16-byte aligned (default on), or every element.  The plots are
-    identical."""
+    """Recurrence plot of bytes, both forms: whole rows of a block stored 16
+    bytes a lane, mirrored squares where that is faster (default on), or one
+    store per decision.  The plots are identical."""
     e = load().accrqa_amd_set_rp_sym(1 if on else 0)
     if e:
         raise AccrqaError(e, "set_rp_sym")

@@ -885,36 +885,48 @@ __global__ __launch_bounds__(WG) void k_rp4(const F *__restrict__ x, int64_t nc,
 // ---------------------------------------------------------------- plot squares
 // The recurrence plot is symmetric bit for bit: s_ij and s_ji are the same
 // sums, since (a - b)^2 = (b - a)^2 and |a - b| = |b - a| exactly, and every
-// form decides the reference's s.  The symmetric kernels (k_rp_sym,
-// k_rp_mx_sym) decide the 64 x 64 squares with g <= J only (rows 64g..,
-// columns 64J..) and store each one as is
-// and mirrored (out[64J.., 64g..]), both as 16-byte row stores staged in
-// the wave's LDS:
-//   D, one 32-row block of the square, row-major (32 rows x 64 bytes),
-//     stored after each block;
-//   T, the mirror, one row per column of the square (64 rows x 64 bytes),
-//     stored after the square's two blocks, except on the diagonal (g == J),
-//     where D covers the square.
-// Rows of both are padded to 80 bytes, so the 16-byte accesses of eight
-// consecutive rows fall on all 32 banks.  The host takes these kernels only
-// where N_c % 16 == 0 and the plot is 16-byte aligned: then every 16-byte
-// store lies inside one row of the plot, and one is made only when its row
-// and first column are below N_c.  Decisions of rows or columns past N_c
-// come from the zero padding of the series and are not stored.
-struct RpStage {
-    static constexpr int RS = 80;   // bytes per row of D and T
-    uint8_t d[BLK * RS];
-    uint8_t t[WAVE * RS];
+// form decides the reference's s.  The square kernels (k_rp_sq, k_rp_mx_sq)
+// decide the S x S squares with g <= J only (rows Sg.., columns SJ..), one
+// workgroup of S threads per square, and store each one as is and mirrored
+// (out[SJ.., Sg..]).  Any N_c, any address of the plot.
+//
+// Decisions travel through LDS as bits, one word per 32 rows of a column
+// (mc, the mirror's rows) and, transposed in registers, one word per 32
+// columns of a row (mr): S^2 / 4 bytes for both orders, so a square is wide
+// enough for its row runs to cover whole 128-byte lines.  A byte table turns
+// eight bits into eight bytes at the store, 16 bytes a lane, S consecutive
+// bytes of a row per S / 16 lanes.
+//
+// Bound by the stores: N_c = 65,536, m = 3: 0.88 ms with S = 256 (4.9 TB/s; the
+// stores alone, in this order, 0.78; a plain fill 0.63), 1.35 ms with the former
+// 64-squares of bytes.  Small squares serve plots that the last-level cache
+// holds (rp_shape in rqa_engine.hip has the rule and its measurements).
+template <int S>
+struct RpBits {
+    static constexpr int CS = S + 4;   // word row stride: the eight words of a row fall on different banks
+    uint32_t mc[S / 32 * CS];          // word w of column j at w * CS + j
+    uint32_t mr[S / 32 * CS];          // word w of row i at w * CS + i
+    uint2 tab[256];                    // byte -> its eight bits as bytes
 };
 
-// Work item it -> square (g, J).  Squares go in groups of 16 x 16 (rows
-// 1024G.., columns 1024H.., G <= H, group number H (H + 1) / 2 + G; square
-// (g, J) = (16G + (it % 256) / 16, 16H + it % 16)), so that the waves at work
-// at one time store their rows in runs of 1,024 bytes rather than 64
-// (measured: groups of 8 and 32 were slower).  False for the squares of a
-// group below the diagonal or past the last band.
-constexpr int RP_GROUP = 16;
-__device__ __forceinline__ bool rp_square(int64_t it, int64_t nbands, int64_t &g, int64_t &J) {
+template <int S>
+__device__ __forceinline__ void rp_table(RpBits<S> &M) {
+    for (int v = threadIdx.x; v < 256; v += S)
+        M.tab[v] = make_uint2(((v & 15) * 0x00204081u) & 0x01010101u, ((v >> 4) * 0x00204081u) & 0x01010101u);
+}
+
+// Square of a workgroup: squares go in groups of RP_GROUP x RP_GROUP (group
+// (G, H), G <= H, number H (H + 1) / 2 + G), and workgroups are numbered XCD
+// by XCD (workgroup b goes to XCD b % 8), so that the two squares that share
+// a 128-byte line at their common edge are stored by one XCD's L2 at about
+// the same time.  False for squares below the diagonal or past the last.
+constexpr int RP_GROUP = 4;
+__host__ __device__ inline int64_t rp_items(int64_t nsq) {
+    const int64_t ng = (nsq + RP_GROUP - 1) / RP_GROUP;
+    return (ng * (ng + 1) / 2 * (RP_GROUP * RP_GROUP) + 7) / 8 * 8;
+}
+__device__ __forceinline__ bool rp_square(int64_t nsq, int64_t &g, int64_t &J) {
+    const int64_t it = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
     const int64_t grp = it / (RP_GROUP * RP_GROUP);
     const int loc = (int)(it - grp * (RP_GROUP * RP_GROUP));
     int64_t H = (int64_t)((__builtin_sqrt(8.0 * (double)grp + 1.0) - 1.0) * 0.5);
@@ -922,103 +934,234 @@ __device__ __forceinline__ bool rp_square(int64_t it, int64_t nbands, int64_t &g
     while ((H + 1) * (H + 2) / 2 <= grp) H++;
     g = RP_GROUP * (grp - H * (H + 1) / 2) + loc / RP_GROUP;
     J = RP_GROUP * H + loc % RP_GROUP;
-    return g <= J && J < nbands;
+    return g <= J && J < nsq;
 }
 
-// The wave's first work item: its slot among the grid's waves, numbered XCD
-// by XCD.  Workgroups go to the eight XCDs in turn (workgroup b to XCD
-// b % 8), so with a grid of a multiple of 8 workgroups (the host rounds it)
-// the squares of one group are taken by waves of one XCD, whose L2 then
-// sees both halves of every 128-byte line the group stores.
-__device__ __forceinline__ int64_t rp_first_item(int wave) {
-    if (gridDim.x % 8) return (int64_t)blockIdx.x * WAVES + wave;
-    return ((int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8) * WAVES + wave;
+// 32 x 32 bit transpose within each half of the wave: lane r's bit c trades
+// places with lane c's bit r, in five exchanges (16 and 8: whole bytes, one
+// byte permute each; 4, 2, 1: a rotate and a bit select).
+__device__ __forceinline__ uint32_t bit_transpose(uint32_t x) {
+    const uint32_t lane = threadIdx.x;
+    {
+        const auto sw = __builtin_amdgcn_permlane16_swap(x, x, false, false);   // both rows of 16: even, odd
+        x = __builtin_amdgcn_perm(sw[1], sw[0], (lane & 16) ? 0x07060302u : 0x05040100u);
+    }
+    {
+        const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);   // lane ^ 8
+        x = __builtin_amdgcn_perm(y, x, (lane & 8) ? 0x03070105u : 0x06020400u);
+    }
+    auto stage = [&](uint32_t y, uint32_t s, uint32_t m) {
+        const bool up = lane & s;
+        const uint32_t r = __builtin_amdgcn_alignbit(y, y, up ? s : 32 - s);
+        const uint32_t k = up ? ~m : m;
+        x = (x & k) | (r & ~k);
+    };
+    uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, false);   // lane ^ 7
+    y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)y, 0x1B, 0xF, 0xF, false);             // then ^ 3
+    stage(y, 4, 0x0F0F0F0Fu);
+    stage((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false), 2, 0x33333333u);
+    stage((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false), 1, 0x55555555u);
+    return x;
 }
 
-// Work items of a plot of nbands bands: whole groups of squares.
-__host__ __device__ inline int64_t rp_items(int64_t nbands) {
-    const int64_t ng = (nbands + RP_GROUP - 1) / RP_GROUP;
-    return ng * (ng + 1) / 2 * (RP_GROUP * RP_GROUP);
-}
+// 16 bytes at any address: one global store, whatever the row's alignment.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
 
-// D to out[i0 + row][j0 + 16 ch ..]: lane -> row (lane >> 2) + 16s, ch = lane & 3.
-__device__ __forceinline__ void rp_store_block(const RpStage &S, int lane, int64_t i0, int64_t j0, int64_t nc,
-                                               char *__restrict__ out) {
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-        const int row = (lane >> 2) + 16 * s, ch = lane & 3;
-        const uint4 v = *(const uint4 *)(S.d + row * RpStage::RS + 16 * ch);
-        const int64_t i = i0 + row, jc = j0 + 16 * ch;
-        if (i < nc && jc < nc) *(uint4 *)(out + i * nc + jc) = v;
+// Rows r0 .. r0+S-1, columns c0 .. c0+S-1 of the plot from the row words w.
+template <int S>
+__device__ __forceinline__ void rp_store(const uint32_t *w, const uint2 *tab, int64_t r0, int64_t c0, int64_t nc,
+                                         char *__restrict__ out) {
+    constexpr int CH = S / 16;   // 16-byte chunks of a row
+    constexpr int CS = RpBits<S>::CS;
+    const int c = threadIdx.x % CH, rr = threadIdx.x / CH;
+    const int64_t left = nc - (c0 + 16 * c);   // columns of the plot from this chunk on
+    if (left <= 0) return;
+    const uint32_t *src = w + (c >> 1) * CS + rr;
+    char *dst = out + (r0 + rr) * nc + c0 + 16 * c;
+    const int64_t rows = nc - (r0 + rr);
+    const int sh = 16 * (c & 1);
+    if (left >= 16) {
+#pragma unroll 4
+        for (int k = 0; k < S / 16; k++) {
+            if (16 * k >= rows) return;
+            const uint32_t v = src[16 * k] >> sh;
+            const uint2 a = tab[v & 0xFFu], b = tab[(v >> 8) & 0xFFu];
+            *(u32x4_any *)(dst + (int64_t)(16 * k) * nc) = (u32x4_any){a.x, a.y, b.x, b.y};
+        }
+    } else {
+#pragma clang loop vectorize(disable) unroll(disable)
+        for (int k = 0; k < S / 16 && 16 * k < rows; k++) {
+            const uint32_t v = src[16 * k] >> sh;
+#pragma clang loop vectorize(disable) unroll(disable)
+            for (int e = 0; e < (int)left; e++) dst[(int64_t)(16 * k) * nc + e] = (char)((v >> e) & 1u);
+        }
     }
 }
 
-// T to out[j0 + row][r0 + 16 ch ..]: lane -> row (lane >> 2) + 16s, ch = lane & 3.
-__device__ __forceinline__ void rp_store_mirror(const RpStage &S, int lane, int64_t j0, int64_t r0, int64_t nc,
-                                                char *__restrict__ out) {
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        const int row = (lane >> 2) + 16 * s, ch = lane & 3;
-        const uint4 v = *(const uint4 *)(S.t + row * RpStage::RS + 16 * ch);
-        const int64_t jr = j0 + row, ic = r0 + 16 * ch;
-        if (jr < nc && ic < nc) *(uint4 *)(out + jr * nc + ic) = v;
-    }
+// w = 2 w + [s <= b] (a NaN s counts as not recurrent): the compare's lane
+// mask is the carry of one add.
+__device__ __forceinline__ void push_le(uint32_t &w, float s, float b) {
+    asm("v_cmp_le_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(s), "v"(b) : "vcc");
+}
+__device__ __forceinline__ void push_le(uint32_t &w, double s, double b) {
+    asm("v_cmp_le_f64 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(s), "v"(b) : "vcc");
 }
 
-// ---------------------------------------------------------------- k_rp_sym
-// The symmetric recurrence plot in the exact form, bytes: per 32-row block
-// of a square, lane = column, the sums of k_rp; the lane's 32 decisions,
-// four rows per word, go to D one byte at a time and to T as two 16-byte
-// LDS stores.  Reads are k_rp's.
-template <typename F, int NORM>
-__global__ __launch_bounds__(WG) void k_rp_sym(const F *__restrict__ x, int64_t nc, int tau, int m, F bound,
-                                               char *__restrict__ out) {
-    __shared__ __attribute__((aligned(16))) RpStage stg[WAVES];
-    constexpr int RS = RpStage::RS;
+// ---------------------------------------------------------------- k_rp_sq
+// The recurrence plot of bytes in the exact form, squares: wave w takes the
+// columns 64w .. 64w+63 (lane = column) of every 32-row block; row samples
+// are wave-uniform (scalar) loads, the first RPK column samples stay in
+// registers.  Columns past N_c read the last one (not stored).
+template <typename F, int NORM, int S>
+__global__ __launch_bounds__(S) void k_rp_sq(const F *__restrict__ x, int64_t nc, int tau, int m, F bound,
+                                             char *__restrict__ out) {
+    __shared__ RpBits<S> M;
+    constexpr int RPK = 4;
+    int64_t g, J;
+    if (!rp_square((nc + S - 1) / S, g, J)) return;
+    rp_table<S>(M);
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
-    RpStage &S = stg[wave];
-    const int64_t nbands = (nc + WAVE - 1) / WAVE;
-    const int64_t nsq = rp_items(nbands);
-    for (int64_t it = rp_first_item(wave); it < nsq; it += (int64_t)gridDim.x * WAVES) {
-        int64_t g, J;
-        if (!rp_square(it, nbands, g, J)) continue;
-        const int64_t j0 = J * WAVE, r0 = g * WAVE;
-        const int64_t j = j0 + lane;
-        for (int k = 0; k < 2; k++) {
-            const int64_t i0 = r0 + BLK * k;
+    const int64_t r0 = g * S, c0 = J * S;
+    const int jl = wave * WAVE + lane;
+    const F *xj = x + min(c0 + jl, nc - 1);
+    F xk[RPK];
+#pragma unroll
+    for (int k = 0; k < RPK; k++) xk[k] = xj[(int64_t)(k < m ? k : 0) * tau];
+    for (int b = 0; b < S / BLK; b++) {
+        const int64_t i0 = r0 + BLK * b;
+        uint32_t w = 0u;
+        if (i0 < nc) {
+            F s[BLK];
+#pragma unroll
+            for (int u = 0; u < BLK; u++) s[u] = F(0);
+#pragma unroll
+            for (int k = 0; k < RPK; k++) {
+                if (k < m) {
+                    const F *xr = x + i0 + (int64_t)k * tau;
+#pragma unroll
+                    for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xk[k]);
+                }
+            }
+            for (int k = RPK; k < m; k++) {
+                const F xv = xj[(int64_t)k * tau];
+                const F *xr = x + i0 + (int64_t)k * tau;
+#pragma unroll
+                for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xv);
+            }
+#pragma unroll
+            for (int u = BLK - 1; u >= 0; u--) push_le(w, s[u], bound);
+        }
+        // lanes 0-31 / 32-63: the block's words of 32-column group 2 wave / 2 wave + 1
+        M.mc[b * RpBits<S>::CS + jl] = w;
+        M.mr[(2 * wave + (lane >> 5)) * RpBits<S>::CS + BLK * b + (lane & 31)] = bit_transpose(w);
+    }
+    __syncthreads();
+    rp_store<S>(M.mr, M.tab, r0, c0, nc, out);
+    if (g < J) rp_store<S>(M.mc, M.tab, c0, r0, nc, out);
+}
+
+// ---------------------------------------------------------------- k_rp_row
+// The recurrence plot of bytes, every element: a workgroup takes R rows of C
+// columns, row words only, and stores runs of C bytes.  For rows that do not
+// start on 128-byte lines: runs of 1,024 unaligned bytes reach 4.7-6 TB/s, the
+// mirrored runs of 256 bytes 2.6-3 (N_c = 30,011, m = 3: 0.23 ms; 0.35 ms with
+// 256-squares, 0.42-0.53 with one store per decision).
+template <int R, int C>
+struct RpRows {
+    static constexpr int CS = R + 1;   // word row stride (odd: the words of a row on different banks)
+    uint32_t mr[C / 32 * CS];          // word w of row i at w * CS + i
+    uint2 tab[256];
+};
+
+// The workgroup's block: blocks along a row first, numbered XCD by XCD.
+template <int R, int C>
+__device__ __forceinline__ bool rp_block(int64_t nc, int64_t &r0, int64_t &c0) {
+    const int64_t ncb = (nc + C - 1) / C;
+    const int64_t it = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    r0 = it / ncb * R;
+    c0 = it % ncb * C;
+    return r0 < nc;
+}
+template <int R, int C>
+int64_t rp_blocks(int64_t nc) {
+    return ((nc + R - 1) / R * ((nc + C - 1) / C) + 7) / 8 * 8;
+}
+
+template <int R, int C>
+__device__ __forceinline__ void rp_store_rows(const RpRows<R, C> &M, int64_t r0, int64_t c0, int64_t nc,
+                                              char *__restrict__ out) {
+    constexpr int CH = C / 16, RP = WG / CH;   // 16-byte chunks of a row, rows per pass
+    const int c = threadIdx.x % CH, rr = threadIdx.x / CH;
+    const int64_t left = nc - (c0 + 16 * c);
+    if (left <= 0) return;
+    const uint32_t *src = M.mr + (c >> 1) * RpRows<R, C>::CS + rr;
+    char *dst = out + (r0 + rr) * nc + c0 + 16 * c;
+    const int64_t rows = nc - (r0 + rr);
+    const int sh = 16 * (c & 1);
+    if (left >= 16) {
+#pragma unroll 4
+        for (int k = 0; k < R / RP; k++) {
+            if (RP * k >= rows) return;
+            const uint32_t v = src[RP * k] >> sh;
+            const uint2 a = M.tab[v & 0xFFu], b = M.tab[(v >> 8) & 0xFFu];
+            *(u32x4_any *)(dst + (int64_t)(RP * k) * nc) = (u32x4_any){a.x, a.y, b.x, b.y};
+        }
+    } else {
+#pragma clang loop vectorize(disable) unroll(disable)
+        for (int k = 0; k < R / RP && RP * k < rows; k++) {
+            const uint32_t v = src[RP * k] >> sh;
+#pragma clang loop vectorize(disable) unroll(disable)
+            for (int e = 0; e < (int)left; e++) dst[(int64_t)(RP * k) * nc + e] = (char)((v >> e) & 1u);
+        }
+    }
+}
+
+template <typename F, int NORM, int R, int C>
+__global__ __launch_bounds__(WG) void k_rp_row(const F *__restrict__ x, int64_t nc, int tau, int m, F bound,
+                                               char *__restrict__ out) {
+    __shared__ RpRows<R, C> M;
+    constexpr int RPK = 4;
+    int64_t r0, c0;
+    if (!rp_block<R, C>(nc, r0, c0)) return;
+    for (int v = threadIdx.x; v < 256; v += WG)
+        M.tab[v] = make_uint2(((v & 15) * 0x00204081u) & 0x01010101u, ((v >> 4) * 0x00204081u) & 0x01010101u);
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = wave_id();
+    for (int q = wave; q < C / WAVE; q += WAVES) {
+        if (c0 + q * WAVE >= nc) break;
+        const F *xj = x + min(c0 + q * WAVE + lane, nc - 1);
+        F xk[RPK];
+#pragma unroll
+        for (int k = 0; k < RPK; k++) xk[k] = xj[(int64_t)(k < m ? k : 0) * tau];
+        for (int b = 0; b < R / BLK; b++) {
+            const int64_t i0 = r0 + BLK * b;
             if (i0 >= nc) break;
             F s[BLK];
 #pragma unroll
             for (int u = 0; u < BLK; u++) s[u] = F(0);
-            F xj = x[j];
-            for (int kk = 0; kk < m; kk++) {
-                const F xjn = x[j + (int64_t)(kk + 1 < m ? kk + 1 : kk) * tau];
-                const F *xr = x + i0 + (int64_t)kk * tau;
 #pragma unroll
-                for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xj);
-                xj = xjn;
+            for (int k = 0; k < RPK; k++) {
+                if (k < m) {
+                    const F *xr = x + i0 + (int64_t)k * tau;
+#pragma unroll
+                    for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xk[k]);
+                }
             }
-            // byte c of word q: row 4q + c
-            uint32_t w[8];
+            for (int k = RPK; k < m; k++) {
+                const F xv = xj[(int64_t)k * tau];
+                const F *xr = x + i0 + (int64_t)k * tau;
 #pragma unroll
-            for (int q = 0; q < 8; q++) {
-                w[q] = 0u;
-#pragma unroll
-                for (int c = 0; c < 4; c++) w[q] |= (s[4 * q + c] <= bound ? 1u : 0u) << (8 * c);
+                for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xv);
             }
-            wave_sync();   // the last block's D and the last square's T are stored
-            uint8_t *dd = S.d + lane;
+            uint32_t w = 0u;
 #pragma unroll
-            for (int u = 0; u < BLK; u++) dd[u * RS] = (uint8_t)(w[u >> 2] >> (8 * (u & 3)));
-            uint4 *tt = (uint4 *)(S.t + lane * RS + 32 * k);
-            tt[0] = make_uint4(w[0], w[1], w[2], w[3]);
-            tt[1] = make_uint4(w[4], w[5], w[6], w[7]);
-            wave_sync();
-            rp_store_block(S, lane, i0, j0, nc, out);
+            for (int u = BLK - 1; u >= 0; u--) push_le(w, s[u], bound);
+            M.mr[(2 * q + (lane >> 5)) * RpRows<R, C>::CS + BLK * b + (lane & 31)] = bit_transpose(w);
         }
-        if (g < J) rp_store_mirror(S, lane, j0, r0, nc, out);
     }
+    __syncthreads();
+    rp_store_rows<R, C>(M, r0, c0, nc, out);
 }
 
 // ---------------------------------------------------------------- k_rr
@@ -1220,7 +1363,6 @@ __global__ __launch_bounds__(WG) void k_fp64_diag(const float *__restrict__ x, i
 // is then decided exactly.
 constexpr int NBX = 16384;       // byte buckets of the MFMA rank table (LDS), DET pass
 constexpr int NBX_LAM = 32768;   // the same for the LAM pass (which has the LDS to spare)
-constexpr int NBX_RP = 4096;     // the same for the symmetric plot (four workgroups per CU)
 constexpr int MXW = 128;     // LDS row window: 32 + (m-1)*tau samples at most
 constexpr int NBND = 64;     // bound slots reachable by a 6-bit table index
 
@@ -2063,104 +2205,315 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(false) void k_rp_mx(const float *__r
 }
 #endif
 
-// ---------------------------------------------------------------- k_rp_mx_sym
-// The symmetric recurrence plot (squares as in k_rp_sym) in the MFMA form.
-// Each 32-row block of a square is decided as in k_rp_mx; with one bound
-// every final rank is 0 or 1, so four elements' decisions (rank 0 -> 1) are
-// their rank word XOR 0x01010101.  D gets each lane's column one byte at a
-// time.  For T, byte q of rank word c is row 8q + 4h + c of the lane's
-// column: a byte transpose of the four words and one cross-half swap per
-// two words leave half 0 with rows 0..15 and half 1 with rows 16..31, one
-// 16-byte LDS store per tile.  Windows read what k_rp_mx reads.
-#ifndef RQA_HELPERS_ONLY
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_rp_mx_sym(
-    const float *__restrict__ x, const float *__restrict__ nrm, const unsigned int *__restrict__ nmax_bits,
-    int64_t nc, int tau, int m, float bound, const uint8_t *__restrict__ lut, MxParams P, char *__restrict__ out) {
-    __shared__ uint8_t lut_s[NBX_RP];
-    __shared__ float bnd_s[NBND];
-    __shared__ MxWin<2> win[WAVES];
-    __shared__ __attribute__((aligned(16))) RpStage stg[WAVES];
-    for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
-    if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, 1, &bound);
-    __syncthreads();
-    constexpr int RS = RpStage::RS;
+// ---------------------------------------------------------------- k_rp_mx_sq
+// The recurrence plot in the MFMA form (fp32, Euclidean), squares as in
+// k_rp_sq.  With one bound no table is needed: per element
+//   d = c2 g + (n_i + (n_j - B)),
+// recurrent iff d < 0 unless |d| <= E_max, the error bound at the largest
+// norm; a tile with such an element in some lane takes each element's own
+// E_ij, and what is still ambiguous is re-summed in exact order by its lane.
+// Against s~ - B of the table form, n_j - B and the sum round once more:
+// at most 2u (n_i + n_j + B) with u = 2^-24, and where B > 4 (n_i + n_j), so
+// B > 2 s, |d| exceeds that and E_ij by far; the host adds RP_EXTRA_U = 12 u
+// to the coefficient cE for B <= 4 (n_i + n_j).  Non-finite or huge norms
+// make E_max infinite: every pair is then decided exactly.
+//
+// Wave w takes the rows 64w .. 64w+63 in two 32-row tiles, each against the
+// square's column tiles two at a time.  A lane's 16 signs of a tile go into
+// one word by shifts through the sign bit (rows 8q + 4h + c of its column at
+// bits 8q + c), and one cross-half swap of the two tiles' words leaves each
+// lane with all 32 rows of one column.
+//
+// About 4 lane-operations an element plus the matrix cores, against about 12
+// with the byte table: N_c = 65,536, m = 16: 1.45 -> 0.93 ms (4.6 TB/s).
+constexpr int RP_EXTRA_U = 12;
+
+template <int S>
+struct RpWin {
+    static constexpr int W = S + MXW - 32;   // samples of a square's rows or columns
+    uint32_t rw[W], cw[W];                   // window words (hl_word)
+    float nr[S], nj[S];                      // norms of the rows and columns
+};
+
+template <int S>
+__global__ __launch_bounds__(S) __attribute__((amdgpu_waves_per_eu(4))) void k_rp_mx_sq(const float *__restrict__ x, const float *__restrict__ nrm,
+                                                const unsigned int *__restrict__ nmax_bits, int64_t nc, int tau,
+                                                int m, float bound, MxParams P, char *__restrict__ out) {
+    __shared__ RpBits<S> M;
+    __shared__ __align__(16) RpWin<S> Wn;
+    int64_t g, J;
+    if (!rp_square((nc + S - 1) / S, g, J)) return;
+    rp_table<S>(M);
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
     const int col = lane & 31;
     const int h = lane >> 5;
-    const int rspan = 32 + (m - 1) * tau;   // <= MXW (checked by the host)
-    const int cspan = 64 + (m - 1) * tau;
-    MxWin<2> &Wn = win[wave];
-    float *rw = Wn.rw, *cw = Wn.cw;
-    mx_win_init(Wn, lane);
-    const float *pa[8];
-    gram_addrs(Wn, col, h, m, tau, pa);
+    const int64_t r0 = g * S, c0 = J * S;
+    const int span = S + (m - 1) * tau;   // <= RpWin::W (checked by the host)
+    const int64_t n = nc + (int64_t)(m - 1) * tau;
     const MxScale Z = mx_scale(nmax_bits, P);
-    RpStage &S = stg[wave];
-    const int64_t nbands = (nc + WAVE - 1) / WAVE;
-    const int64_t nsq = rp_items(nbands);
-    for (int64_t it = rp_first_item(wave); it < nsq; it += (int64_t)gridDim.x * WAVES) {
-        int64_t g, J;
-        if (!rp_square(it, nbands, g, J)) continue;
-        const int64_t j0 = J * WAVE, r0 = g * WAVE;
-        wave_sync();
-        for (int e = lane; e < cspan; e += WAVE) cw[e] = hl_word(x[j0 + e] * Z.s);
-        for (int k = 0; k < 2; k++) {
-            const int64_t i0 = r0 + BLK * k;
-            if (i0 >= nc) break;
-            for (int e = lane; e < rspan; e += WAVE) rw[e] = hl_word(x[i0 + e] * Z.s);
-            wave_sync();
-            float ni[16];
-            tile_row_norms(nrm, i0, h, ni);
+    const float nmax = __uint_as_float(*nmax_bits);
+    float emax = (P.cE * 2.0f * nmax + Z.dE) * 1.0001f;
+    if (!(nmax <= 1e30f)) emax = __int_as_float(0x7F800000);
+    for (int e = threadIdx.x; e < span; e += S) {
+        Wn.rw[e] = __float_as_uint(hl_word(r0 + e < n ? x[r0 + e] * Z.s : 0.f));
+        Wn.cw[e] = __float_as_uint(hl_word(c0 + e < n ? x[c0 + e] * Z.s : 0.f));
+    }
+    {
+        const int e = threadIdx.x;
+        Wn.nr[e] = r0 + e < nc ? nrm[r0 + e] : 0.f;
+        Wn.nj[e] = c0 + e < nc ? nrm[c0 + e] : 0.f;
+    }
+    __syncthreads();
+
+    constexpr uint32_t SH = 0x05040100u, SL = 0x07060302u;
+    // window offset of dimension k0 + 8h + t; the row operands of dimensions
+    // past m are 0, so the column operands there may be anything finite
+    auto offs = [&](int k0, int t) { const int k = k0 + 8 * h + t; return col + (k < m ? k * tau : 0); };
+    for (int r = 0; r < 2; r++) {
+        const int rb = wave * WAVE + BLK * r;
+        if (r0 + rb >= nc) {   // no such rows: their words are 0
+#pragma unroll 1
+            for (int p = 0; p < S / BLK; p++) {
+                if (h == 0) M.mc[(rb / BLK) * RpBits<S>::CS + BLK * p + col] = 0u;
+                if (h == 1) M.mr[p * RpBits<S>::CS + rb + col] = 0u;
+            }
+            continue;
+        }
+        float ni[16];
+        tile_row_norms(Wn.nr, rb, h, ni);
+        uint32_t a[8], b[8];
+        auto load_a = [&](int k0) {
 #pragma unroll
-            for (int p = 0; p < 2; p++) {
-                const floatx16 acc = p == 0 ? gram_tile<2, 0>(Wn, pa, col, h, m, tau) : gram_tile<2, 1>(Wn, pa, col, h, m, tau);
-                uint32_t Rq[4], fm, flw;
-                tile_ranks(acc, ni, nrm[j0 + 32 * p + col], lut_s, P, Z, bnd_s, Rq, fm, flw);
-                const int64_t j = j0 + 32 * p + col;
-                // exact re-decision of the ambiguous elements by their own lane
-                uint32_t f = j < nc ? fm : 0u;
-                while (f) {
-                    const uint32_t e = __builtin_ctz(f);
-                    f &= f - 1u;
-                    const int64_t i = i0 + 8 * (e >> 2) + 4 * h + (e & 3);
+            for (int t = 0; t < 8; t++) {
+                const uint32_t v = Wn.rw[rb + offs(k0, t)];
+                a[t] = k0 + 8 * h + t < m ? v : 0u;
+            }
+        };
+        load_a(0);
+        const halfx8 ah = hl_halves<SH>(a), al = hl_halves<SL>(a);
+        int o0[8];
+#pragma unroll
+        for (int t = 0; t < 8; t++) o0[t] = offs(0, t);
+        auto gram = [&](int cb) {
+            floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (m <= 16) {
+#pragma unroll
+                for (int t = 0; t < 8; t++) b[t] = Wn.cw[cb + o0[t]];
+                const halfx8 bh = hl_halves<SH>(b);
+                acc = mfma16(al, bh, acc);
+                acc = mfma16(ah, hl_halves<SL>(b), acc);
+                return mfma16(ah, bh, acc);
+            }
+            // small products of every chunk, then h.h chunk by chunk
+            auto load = [&](int k0) {
+                load_a(k0);
+#pragma unroll
+                for (int t = 0; t < 8; t++) b[t] = Wn.cw[cb + offs(k0, t)];
+            };
+            for (int k0 = 0; k0 < m; k0 += 16) {
+                load(k0);
+                acc = mfma16(hl_halves<SL>(a), hl_halves<SH>(b), acc);
+                acc = mfma16(hl_halves<SH>(a), hl_halves<SL>(b), acc);
+            }
+            for (int k0 = 0; k0 < m; k0 += 16) {
+                load(k0);
+                acc = mfma16(hl_halves<SH>(a), hl_halves<SH>(b), acc);
+            }
+            return acc;
+        };
+        // signs of a tile's 16 elements as a word: row 8q + 4h + c at bit 8q + c
+        auto decide = [&](floatx16 acc, int cb) -> uint32_t {
+            const float nj = Wn.nj[cb + col], njb = nj - bound;
+            float lo = __int_as_float(0x7F800000);
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[e] = fmaf(Z.c2, acc[e], ni[e] + njb);
+#pragma unroll
+            for (int e = 0; e < 16; e += 2) lo = fminf(lo, fminf(fabsf(acc[e]), fabsf(acc[e + 1])));
+            uint32_t w = 0u;
+#pragma unroll
+            for (int q = 3; q >= 0; q--) {
+                w <<= 4;
+#pragma unroll
+                for (int c = 3; c >= 0; c--) w = __builtin_amdgcn_alignbit(w, __float_as_uint(acc[4 * q + c]), 31);
+            }
+            if (__builtin_amdgcn_ballot_w64(!(lo > emax)) != 0ull) {
+                const int64_t j = c0 + cb + col;
+                uint32_t fm = 0u;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const float E = fmaf(P.cE, ni[e] + nj, Z.dE);
+                    fm |= (!(fabsf(acc[e]) > E) ? 1u : 0u) << (8 * (e >> 2) + (e & 3));
+                }
+                if (j >= nc) fm = 0u;
+                while (fm) {
+                    const uint32_t e = __builtin_ctz(fm);   // row e + 4h of the tile
+                    fm &= fm - 1u;
+                    const int64_t i = r0 + rb + 4 * h + e;
                     if (i < nc) {
-                        const float sx = exact_sqdist<float>(x, i, j, tau, m);
-                        const uint32_t rk = rank_direct<float, 1>(sx, bnd_s, 1);
-                        const uint32_t sh = 8 * (e >> 2), c = e & 3;
-                        Rq[c] = (Rq[c] & ~(0xFFu << sh)) | (rk << sh);
+                        const uint32_t in = exact_sqdist<float>(x, i, j, tau, m) <= bound ? 1u : 0u;
+                        w = (w & ~(1u << e)) | (in << e);
                     }
                 }
-                uint32_t Dw[4];
-#pragma unroll
-                for (int c = 0; c < 4; c++) Dw[c] = Rq[c] ^ 0x01010101u;
-                // D: element e is row 8(e>>2) + 4h + (e&3), column 32p + col
-                uint8_t *dd = S.d + 4 * h * RS + 32 * p + col;
-#pragma unroll
-                for (int e = 0; e < 16; e++) dd[(8 * (e >> 2) + (e & 3)) * RS] = (uint8_t)(Dw[e & 3] >> (8 * (e >> 2)));
-                // T: byte q of Dw[c] is row 8q + 4h + c; word q of the
-                // transpose holds rows 8q + 4h .. 8q + 4h + 3
-                const uint32_t lo01 = __builtin_amdgcn_perm(Dw[1], Dw[0], 0x05010400u);
-                const uint32_t hi01 = __builtin_amdgcn_perm(Dw[1], Dw[0], 0x07030602u);
-                const uint32_t lo23 = __builtin_amdgcn_perm(Dw[3], Dw[2], 0x05010400u);
-                const uint32_t hi23 = __builtin_amdgcn_perm(Dw[3], Dw[2], 0x07030602u);
-                const uint32_t w0 = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-                const uint32_t w1 = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-                const uint32_t w2 = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-                const uint32_t w3 = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
-                // half 0 then holds rows 0..15 of its column, half 1 rows 16..31
-                const auto s02 = __builtin_amdgcn_permlane32_swap(w0, w2, false, false);
-                const auto s13 = __builtin_amdgcn_permlane32_swap(w1, w3, false, false);
-                *(uint4 *)(S.t + (32 * p + col) * RS + 32 * k + 16 * h) = make_uint4(s02[0], s02[1], s13[0], s13[1]);
             }
-            wave_sync();
-            rp_store_block(S, lane, i0, j0, nc, out);
-            wave_sync();
+            return w;
+        };
+#pragma unroll 1
+        for (int p = 0; p < S / BLK; p += 2) {
+            const floatx16 g0 = gram(BLK * p), g1 = gram(BLK * p + BLK);
+            const uint32_t w0 = decide(g0, BLK * p), w1 = decide(g1, BLK * p + BLK);
+            // half 0: column tile p, half 1: column tile p + 1; words of rows 8q + c, then 8q + 4 + c
+            const auto sw = __builtin_amdgcn_permlane32_swap(w0, w1, false, false);
+            const uint32_t w = sw[0] | (sw[1] << 4);
+            M.mc[(rb / BLK) * RpBits<S>::CS + BLK * (p + h) + col] = w;
+            M.mr[(p + h) * RpBits<S>::CS + rb + col] = bit_transpose(w);
         }
-        if (g < J) rp_store_mirror(S, lane, j0, r0, nc, out);
     }
+    __syncthreads();
+    rp_store<S>(M.mr, M.tab, r0, c0, nc, out);
+    if (g < J) rp_store<S>(M.mc, M.tab, c0, r0, nc, out);
 }
-#endif
+
+// ---------------------------------------------------------------- k_rp_mx_row
+// k_rp_mx_sq's decisions for the blocks of k_rp_row.  The matrix product is
+// taken the other way round (element = column, lane = row), so a lane's signs
+// are its row's bits and no transpose is needed.
+template <int R, int C>
+struct RpRowWin {
+    uint32_t rw[R + MXW - 32], cw[C + MXW - 32];   // window words (hl_word)
+    float nr[R], nj[C], njb[C];                    // norms of the rows, of the columns, columns less the bound
+};
+
+template <int R, int C>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_rp_mx_row(
+    const float *__restrict__ x, const float *__restrict__ nrm, const unsigned int *__restrict__ nmax_bits, int64_t nc,
+    int tau, int m, float bound, MxParams P, char *__restrict__ out) {
+    __shared__ RpRows<R, C> M;
+    __shared__ __align__(16) RpRowWin<R, C> Wn;
+    int64_t r0, c0;
+    if (!rp_block<R, C>(nc, r0, c0)) return;
+    for (int v = threadIdx.x; v < 256; v += WG)
+        M.tab[v] = make_uint2(((v & 15) * 0x00204081u) & 0x01010101u, ((v >> 4) * 0x00204081u) & 0x01010101u);
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = wave_id();
+    const int col = lane & 31;
+    const int h = lane >> 5;
+    const int64_t n = nc + (int64_t)(m - 1) * tau;
+    const MxScale Z = mx_scale(nmax_bits, P);
+    const float nmax = __uint_as_float(*nmax_bits);
+    float emax = (P.cE * 2.0f * nmax + Z.dE) * 1.0001f;
+    if (!(nmax <= 1e30f)) emax = __int_as_float(0x7F800000);
+    for (int e = threadIdx.x; e < C + (m - 1) * tau; e += WG)   // <= C + MXW - 32 (checked by the host)
+        Wn.cw[e] = __float_as_uint(hl_word(c0 + e < n ? x[c0 + e] * Z.s : 0.f));
+    for (int e = threadIdx.x; e < R + (m - 1) * tau; e += WG)
+        Wn.rw[e] = __float_as_uint(hl_word(r0 + e < n ? x[r0 + e] * Z.s : 0.f));
+    for (int e = threadIdx.x; e < C; e += WG) {
+        const float v = c0 + e < nc ? nrm[c0 + e] : 0.f;
+        Wn.nj[e] = v;
+        Wn.njb[e] = v - bound;
+    }
+    if (threadIdx.x < R) Wn.nr[threadIdx.x] = r0 + threadIdx.x < nc ? nrm[r0 + threadIdx.x] : 0.f;
+    __syncthreads();
+
+    constexpr uint32_t SH = 0x05040100u, SL = 0x07060302u;
+    // window offset of dimension k0 + 8h + t; the row operands of dimensions
+    // past m are 0, so the column operands there may be anything finite
+    auto offs = [&](int k0, int t) { const int k = k0 + 8 * h + t; return col + (k < m ? k * tau : 0); };
+    int o0[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) o0[t] = offs(0, t);
+#pragma unroll 1
+    for (int r = 0; r < R / BLK; r++) {
+        const int rb = BLK * r;
+        if (r0 + rb >= nc) break;
+        uint32_t a[8], b[8];
+        auto load_b = [&](int k0) {
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                const uint32_t v = Wn.rw[rb + offs(k0, t)];
+                b[t] = k0 + 8 * h + t < m ? v : 0u;
+            }
+        };
+        load_b(0);
+        const halfx8 bh = hl_halves<SH>(b), bl = hl_halves<SL>(b);
+        const float ni = Wn.nr[rb + col];
+        auto gram = [&](int cb) {
+            floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (m <= 16) {
+#pragma unroll
+                for (int t = 0; t < 8; t++) a[t] = Wn.cw[cb + o0[t]];
+                const halfx8 ah = hl_halves<SH>(a);
+                acc = mfma16(hl_halves<SL>(a), bh, acc);
+                acc = mfma16(ah, bl, acc);
+                return mfma16(ah, bh, acc);
+            }
+            // small products of every chunk, then h.h chunk by chunk
+            auto load = [&](int k0) {
+                load_b(k0);
+#pragma unroll
+                for (int t = 0; t < 8; t++) a[t] = Wn.cw[cb + offs(k0, t)];
+            };
+            for (int k0 = 0; k0 < m; k0 += 16) {
+                load(k0);
+                acc = mfma16(hl_halves<SL>(a), hl_halves<SH>(b), acc);
+                acc = mfma16(hl_halves<SH>(a), hl_halves<SL>(b), acc);
+            }
+            for (int k0 = 0; k0 < m; k0 += 16) {
+                load(k0);
+                acc = mfma16(hl_halves<SH>(a), hl_halves<SH>(b), acc);
+            }
+            return acc;
+        };
+        // signs of a tile's 16 elements as a word: column 8q + 4h + c at bit 8q + c
+        auto decide = [&](floatx16 acc, int cb) -> uint32_t {
+            float nb[16];
+            tile_row_norms(Wn.njb, cb, h, nb);
+            float lo = __int_as_float(0x7F800000);
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[e] = fmaf(Z.c2, acc[e], ni + nb[e]);
+#pragma unroll
+            for (int e = 0; e < 16; e += 2) lo = fminf(lo, fminf(fabsf(acc[e]), fabsf(acc[e + 1])));
+            uint32_t w = 0u;
+#pragma unroll
+            for (int q = 3; q >= 0; q--) {
+                w <<= 4;
+#pragma unroll
+                for (int c = 3; c >= 0; c--) w = __builtin_amdgcn_alignbit(w, __float_as_uint(acc[4 * q + c]), 31);
+            }
+            if (__builtin_amdgcn_ballot_w64(!(lo > emax)) != 0ull) {
+                const int64_t i = r0 + rb + col;
+                uint32_t fm = 0u;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const float E = fmaf(P.cE, ni + Wn.nj[cb + 8 * (e >> 2) + 4 * h + (e & 3)], Z.dE);
+                    fm |= (!(fabsf(acc[e]) > E) ? 1u : 0u) << (8 * (e >> 2) + (e & 3));
+                }
+                if (i >= nc) fm = 0u;
+                while (fm) {
+                    const uint32_t e = __builtin_ctz(fm);   // column e + 4h of the tile
+                    fm &= fm - 1u;
+                    const int64_t j = c0 + cb + 4 * h + e;
+                    if (j < nc) {
+                        const uint32_t in = exact_sqdist<float>(x, i, j, tau, m) <= bound ? 1u : 0u;
+                        w = (w & ~(1u << e)) | (in << e);
+                    }
+                }
+            }
+            return w;
+        };
+#pragma unroll 1
+        for (int p = 2 * wave; p < C / BLK; p += 2 * WAVES) {
+            if (c0 + BLK * p >= nc) break;
+            const floatx16 g0 = gram(BLK * p), g1 = gram(BLK * p + BLK);
+            const uint32_t w0 = decide(g0, BLK * p), w1 = decide(g1, BLK * p + BLK);
+            // half 0: column tile p, half 1: column tile p + 1; columns 8q + c, then 8q + 4 + c
+            const auto sw = __builtin_amdgcn_permlane32_swap(w0, w1, false, false);
+            M.mr[(p + h) * RpRows<R, C>::CS + rb + col] = sw[0] | (sw[1] << 4);
+        }
+    }
+    __syncthreads();
+    rp_store_rows<R, C>(M, r0, c0, nc, out);
+}
 
 // ---------------------------------------------------------------- k_lam_vscan
 // The column part of LAM in the split form, read back from the rank tiles

@@ -105,10 +105,9 @@ int g_gram = 0;
 // stores align) or one (k_rp; accrqa_amd_set_rp_wide(0)).
 bool g_rp_wide = true;
 
-// Recurrence plot of bytes: the upper triangle, each 64 x 64 square stored
-// mirrored as well (k_rp_mx_sym, k_rp_sym; where N_c % 16 == 0 and the plot
-// is 16-byte aligned), or every element (k_rp_mx, k_rp4, k_rp;
-// accrqa_amd_set_rp_sym(0)).
+// Recurrence plot of bytes: decisions as bits through LDS, the upper triangle
+// in squares stored mirrored as well or every element in rows (rp_shape), or
+// one store per decision (k_rp_mx, k_rp4, k_rp; accrqa_amd_set_rp_sym(0)).
 bool g_rp_sym = true;
 
 // The split form's DET tile scan on the context's second stream, beside the
@@ -1555,6 +1554,73 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
     return E_OK;
 }
 
+// Shape of a plot's work.  Measured (MI355X, bytes, m = 3 exact unless said):
+//   SMALL  blocks of 32 x 256, every element: enough workgroups for a small
+//          plot (N_c = 1,500: 4.8 us, 64-squares 8.0; 4,000: 9.6 and 9.2)
+//   SQ64   64-squares, mirrored: while the plot fits the 256 MB last-level
+//          cache its short mirrored runs merge there (12,000: 30 us, 256-squares
+//          36, rows 41; 20,000: 140, 128, 102)
+//   SQ256  256-squares, mirrored: large plots whose rows start on 128-byte
+//          lines, so every run is whole lines (65,536: 0.88 ms, rows 1.03)
+//   ROWS   blocks of 64 (MFMA, large: 128) x 1,024, every element: other large
+//          plots, where the runs' partial lines cost more than the second
+//          half's decisions (30,011: 225 us, 256-squares 346), as long as the
+//          decisions are cheap: the MFMA form in one chunk of 16 dimensions
+//          (m = 16: 265 and 379 us, m = 32: 617 and 490), or at most 15 VALU
+//          operations an element (m = 5: 318 and 346 us, m = 6: 372 and 351)
+enum { RP_SMALL, RP_SQ64, RP_SQ256, RP_ROWS };
+int rp_shape(int64_t nc, const void *out, bool cheap) {
+    if (nc <= 3072) return RP_SMALL;
+    if (nc <= 16384) return RP_SQ64;
+    if (nc % 128 == 0 && (uintptr_t)out % 128 == 0) return RP_SQ256;
+    return cheap ? RP_ROWS : RP_SQ256;
+}
+
+unsigned rp_grid(int64_t nc, int64_t S) { return (unsigned)rqa::rp_items((nc + S - 1) / S); }
+
+template <typename F, int NORM>
+void rp_launch_exact(int shape, const F *dx, int64_t nc, int tau, int m, F b, char *out, hipStream_t st) {
+    switch (shape) {
+        case RP_SMALL:
+            hipLaunchKernelGGL((rqa::k_rp_row<F, NORM, 32, 256>), dim3((unsigned)rqa::rp_blocks<32, 256>(nc)),
+                               dim3(rqa::WG), 0, st, dx, nc, tau, m, b, out);
+            break;
+        case RP_SQ64:
+            hipLaunchKernelGGL((rqa::k_rp_sq<F, NORM, 64>), dim3(rp_grid(nc, 64)), dim3(64), 0, st, dx, nc, tau, m, b,
+                               out);
+            break;
+        case RP_SQ256:
+            hipLaunchKernelGGL((rqa::k_rp_sq<F, NORM, 256>), dim3(rp_grid(nc, 256)), dim3(256), 0, st, dx, nc, tau, m,
+                               b, out);
+            break;
+        default:
+            hipLaunchKernelGGL((rqa::k_rp_row<F, NORM, 64, 1024>), dim3((unsigned)rqa::rp_blocks<64, 1024>(nc)),
+                               dim3(rqa::WG), 0, st, dx, nc, tau, m, b, out);
+            break;
+    }
+}
+
+void rp_launch_mx(int shape, const float *dx, int64_t nc, int tau, int m, float b, const rqa::MxParams &P, char *out,
+                  hipStream_t st) {
+    const float *nrm = (const float *)g_ctx.nrm.p;
+    const unsigned int *nmax = (const unsigned int *)g_ctx.nmax.p;
+    auto sq = [&](auto kern, int S) {
+        hipLaunchKernelGGL(kern, dim3(rp_grid(nc, S)), dim3(S), 0, st, dx, nrm, nmax, nc, tau, m, b, P, out);
+    };
+    auto row = [&](auto kern, int64_t blocks) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(rqa::WG), 0, st, dx, nrm, nmax, nc, tau, m, b, P, out);
+    };
+    switch (shape) {
+        case RP_SMALL: row(rqa::k_rp_mx_row<32, 256>, rqa::rp_blocks<32, 256>(nc)); break;
+        case RP_SQ64: sq(rqa::k_rp_mx_sq<64>, 64); break;
+        case RP_SQ256: sq(rqa::k_rp_mx_sq<256>, 256); break;
+        default:
+            if (nc > 24576) row(rqa::k_rp_mx_row<128, 1024>, rqa::rp_blocks<128, 1024>(nc));
+            else row(rqa::k_rp_mx_row<64, 1024>, rqa::rp_blocks<64, 1024>(nc));
+            break;
+    }
+}
+
 // The recurrence plot of one (tau, emb, threshold) into d_out (N_c x N_c
 // elements of O, row-major), from the padded series dx.  A threshold that
 // never recurs (negative or NaN) gets bound -1, below every s.
@@ -1566,13 +1632,19 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
     const bool never = never_recurs(b);
     if (never) b = F(-1);
     const int64_t nblk = ((nc + rqa::BLK - 1) / rqa::BLK) * ((nc + rqa::WAVE - 1) / rqa::WAVE);
+    const bool sym = sizeof(O) == 1 && g_rp_sym;
     if constexpr (sizeof(F) == 4 && sizeof(O) == 1) {
-        if (!never && dist == 1 && use_mfma<F>(1, emb, tau)) {
-            // MFMA form: norms, the one-bound byte table, then the plot
+        // With one bound the MFMA form pays from m = 4 on large plots (65,536, m = 4:
+        // 0.95 ms either way, m = 6: 0.94 against 1.09; 30,011, m = 4: 253 us against
+        // 283); small ones would pay for the norms' launches
+        const bool mx = use_mfma<F>(1, emb, tau) ||
+                        (sym && nc > 16384 && emb >= 4 && use_mfma<F>(1, std::max(emb, 8), 0) &&
+                         (int64_t)(emb - 1) * tau <= rqa::MXW - 32);
+        if (!never && dist == 1 && mx) {
+            // MFMA form: norms, then the plot (every element: with its one-bound byte table)
             int e;
             if ((e = ensure(c.nrm, ((size_t)nc + 2 * rqa::WAVE) * sizeof(float)))) return e;
             if ((e = ensure(c.nmax, 256))) return e;
-            if ((e = ensure(c.lut8, rqa::NBX_LAM))) return e;
             fill_zero((unsigned long long *)c.nmax.p, 1, st);
             const int64_t nthr = nc + 2 * rqa::WAVE;
             hipLaunchKernelGGL((rqa::k_norms<F>), dim3((unsigned)((nthr + rqa::NRT - 1) / rqa::NRT)), dim3(rqa::NRT), 0, st,
@@ -1580,21 +1652,16 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
             HIP_TRY(hipGetLastError());
             rqa::Bounds<float, 4> Bf;
             for (int t = 0; t < 4; t++) Bf.s[t] = (float)b;
-            // the upper triangle, each square stored mirrored as well, where
-            // its 16-byte stores align
-            const bool sym = g_rp_sym && nc % 16 == 0 && (uintptr_t)d_out % 16 == 0;
-            const rqa::MxParams MP = mx_params(Bf.s, 1, emb, sym ? rqa::NBX_RP : rqa::NBX_LAM);
-            hipLaunchKernelGGL((rqa::k_mx_lut<4>), dim3((MP.nb + 255) / 256), dim3(256), 0, st, Bf, 1, MP,
-                               (const unsigned int *)c.nmax.p, (uint8_t *)c.lut8.p);
-            HIP_TRY(hipGetLastError());
             if (sym) {
-                const int64_t nbands = (nc + rqa::WAVE - 1) / rqa::WAVE;
-                const unsigned g = xcd_round(grid_for(rqa::k_rp_mx_sym, rqa::rp_items(nbands), c.ncu));
-                prof_begin("k_rp_mx_sym", st);
-                hipLaunchKernelGGL(rqa::k_rp_mx_sym, dim3(g), dim3(rqa::WG), 0, st, (const float *)dx,
-                                   (const float *)c.nrm.p, (const unsigned int *)c.nmax.p, nc, tau, emb, (float)b,
-                                   (const uint8_t *)c.lut8.p, MP, (char *)d_out);
+                prof_begin("k_rp_mx_sq", st);
+                rp_launch_mx(rp_shape(nc, d_out, emb <= 16), (const float *)dx, nc, tau, emb, (float)b,
+                             mx_params(Bf.s, 1, emb, rqa::NBX_LAM, rqa::RP_EXTRA_U), (char *)d_out, st);
             } else {
+                const rqa::MxParams MP = mx_params(Bf.s, 1, emb, rqa::NBX_LAM);
+                if ((e = ensure(c.lut8, rqa::NBX_LAM))) return e;
+                hipLaunchKernelGGL((rqa::k_mx_lut<4>), dim3((MP.nb + 255) / 256), dim3(256), 0, st, Bf, 1, MP,
+                                   (const unsigned int *)c.nmax.p, (uint8_t *)c.lut8.p);
+                HIP_TRY(hipGetLastError());
                 const unsigned g = grid_for(rqa::k_rp_mx, nblk, c.ncu);
                 prof_begin("k_rp_mx", st);
                 hipLaunchKernelGGL(rqa::k_rp_mx, dim3(g), dim3(rqa::WG), 0, st, (const float *)dx,
@@ -1607,27 +1674,20 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
             return E_OK;
         }
     }
-    const uintptr_t oa = (uintptr_t)d_out;
     if constexpr (sizeof(O) == 1) {
-        // the upper triangle, each square stored mirrored as well
-        if (g_rp_sym && nc % 16 == 0 && oa % 16 == 0) {
-            const int64_t nsq = rqa::rp_items((nc + rqa::WAVE - 1) / rqa::WAVE);
-            prof_begin("k_rp_sym", st);
-            if (dist == 1) {
-                const unsigned g = xcd_round(grid_for(rqa::k_rp_sym<F, 1>, nsq, c.ncu));
-                hipLaunchKernelGGL((rqa::k_rp_sym<F, 1>), dim3(g), dim3(rqa::WG), 0, st, dx, nc, tau, emb, b,
-                                   (char *)d_out);
-            } else {
-                const unsigned g = xcd_round(grid_for(rqa::k_rp_sym<F, 2>, nsq, c.ncu));
-                hipLaunchKernelGGL((rqa::k_rp_sym<F, 2>), dim3(g), dim3(rqa::WG), 0, st, dx, nc, tau, emb, b,
-                                   (char *)d_out);
-            }
+        if (sym) {
+            const int ops = (dist == 1 ? 3 : 2) * emb * (sizeof(F) == 8 ? 2 : 1);
+            const int shape = rp_shape(nc, d_out, ops <= 15);
+            prof_begin("k_rp_sq", st);
+            if (dist == 1) rp_launch_exact<F, 1>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
+            else rp_launch_exact<F, 2>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
             prof_end(st);
             HIP_TRY(hipGetLastError());
             prof_collect(st);
             return E_OK;
         }
     }
+    const uintptr_t oa = (uintptr_t)d_out;
     // four columns per lane when its 4-element stores align
     if (g_rp_wide && nc % 4 == 0 && oa % (sizeof(O) == 1 ? 4 : 16) == 0) {
         constexpr int R4 = rqa::rp4_rows<F>();

@@ -613,8 +613,8 @@ def config4_batched(accrqa_amd):
 def rp_bench(accrqa_amd, torch, x, thr, reps=3):
     """accrqa_RP through the device entry point, series and plot in HBM, on a
     65,536-row plot (4.3 GB of bytes) of the default workload's series, at
-    m = 16 (k_rp_mx_sym, the MFMA form) and m = 3 (k_rp_sym, the exact form),
-    both deciding the upper triangle and storing each 64 x 64 square
+    m = 16 (k_rp_mx_sq, the MFMA form) and m = 3 (k_rp_sq, the exact form),
+    both deciding the upper triangle and storing each 256 x 256 square
     mirrored as well, tau = 1, Euclidean; one byte per element written,
     priced against 8 TB/s.  `every_element_form_ms` is the plot with every
     element decided (accrqa_amd_set_rp_sym(0): k_rp_mx, or k_rp4 with four

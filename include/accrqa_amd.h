@@ -193,8 +193,8 @@ int accrqa_amd_rp_device_f64(const double *d_input, size_t data_size, int tau, i
                              int distance_type, char *d_output, void *stream);
 
 /* Form of the Euclidean distance (no counterpart in the reference, which has
- * one form per platform).  0 = automatic: the MFMA form for emb >= 8, exact
- * VALU sums otherwise; 1 = exact VALU sums only; 2 = MFMA form wherever it
+ * one form per platform).  0 = automatic: the MFMA form for emb >= 8 (emb >= 4
+ * for plots of bytes with N_c > 16384), exact VALU sums otherwise; 1 = exact VALU sums only; 2 = MFMA form wherever it
  * applies (Euclidean norm; fp32 input, and fp64 input in the LAM pass, whose
  * Gram then runs on the series rounded to fp32).  The MFMA form computes
  * |x_i|^2 + |x_j|^2 - 2 x_i.x_j with the Gram tile on FP16 matrix cores
@@ -242,18 +242,19 @@ int accrqa_amd_mx_stats_read(unsigned long long *counts);
  * Returns 0 or an Accrqa_Error code. */
 int accrqa_amd_mfma16_probe(const uint16_t *a, const uint16_t *b, const float *c, float *d);
 
-/* Recurrence plot, exact form (tuning aid, no counterpart in the reference):
- * 1 (the default) gives each lane four adjacent columns, so every store
+/* Recurrence plot of ints, and of bytes with accrqa_amd_set_rp_sym(0), exact
+ * form (tuning aid, no counterpart in the reference): 1 (the default) gives each lane four adjacent columns, so every store
  * writes 256 consecutive elements, where N_c % 4 == 0 and the plot's address
  * aligns those stores; 0 keeps one column per lane.  The plots are identical.
  * Returns 0 or ERR_INVALID_ARGUMENT. */
 int accrqa_amd_set_rp_wide(int on);
 
 /* Recurrence plot of bytes, both forms (tuning aid, no counterpart in the
- * reference): 1 (the default) decides the upper triangle only and stores
- * each 64 x 64 square mirrored as well, where N_c % 16 == 0 and the plot is
- * 16-byte aligned (every store is then 16 bytes of one row); 0 decides every
- * element.  The plots are identical.  Returns 0 or ERR_INVALID_ARGUMENT. */
+ * reference): 1 (the default) stores whole rows of a block 16 bytes a lane,
+ * the upper triangle decided once and stored mirrored as well where that is
+ * faster, for any N_c and address; 0 makes one store per decision (or per four,
+ * accrqa_amd_set_rp_wide).  The plots are identical.  Returns 0 or
+ * ERR_INVALID_ARGUMENT. */
 int accrqa_amd_set_rp_sym(int on);
 
 /* Waves per SIMD of the three tile scans (tuning aid, no counterpart in the
