@@ -123,15 +123,15 @@ ChunkPlan plan_chunk(const std::vector<SBlock<F>> &blocks, size_t s0, size_t s1,
 
 // ---------------------------------------------------------------- autotuner
 // k_batch comes in instantiations that differ in the waves per SIMD their
-// register allocation must allow (the compiler's choice, 4, 5, 6).  The first
+// register allocation must allow (the compiler's choice, 4, 5).  The first
 // call of a (precision, norm, threshold group) with at least TUNE_MIN_PAIRS
 // pair decisions in its first chunk runs that chunk once with each
 // instantiation, timed with HIP events, and keeps the fastest for the rest of
 // the process; every run recomputes the chunk from zeroed histograms, so the
 // results are those of any one run.  accrqa_amd_batch_report() gives the
 // choices.
-constexpr int NVAR = 4;
-constexpr int VAR_WPE[NVAR] = {1, 4, 5, 6};
+constexpr int NVAR = 3;
+constexpr int VAR_WPE[NVAR] = {1, 4, 5};
 constexpr double TUNE_MIN_PAIRS = 2e9;
 
 struct TuneEntry {
@@ -150,7 +150,6 @@ auto with_variant(int var, Fn &&f) {
     switch (var) {
         case 1: return f(rqa::k_batch<F, NORM, TG, 4>);
         case 2: return f(rqa::k_batch<F, NORM, TG, 5>);
-        case 3: return f(rqa::k_batch<F, NORM, TG, 6>);
         default: return f(rqa::k_batch<F, NORM, TG, 1>);
     }
 }

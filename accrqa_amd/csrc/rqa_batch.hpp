@@ -11,10 +11,10 @@
 // the persistent grid finish together whatever the mix of lengths.
 //
 // Decisions, ranks and the word-level line scan are those of the large-N
-// kernels (dim_step, pack_ranks, rank_planes, GeTree, consume; exact-order
+// kernels (dim_step, pack_ranks, scan_core; exact-order
 // sums, rqa_device.hpp), so every histogram is the reference's bit for bit.
 // Each wave keeps the run-length histogram of its current (problem, kind) in
-// its own LDS (lengths < BLCAP) and adds it to the problem's u32 histogram in
+// its own LDS (lengths < blcap) and adds it to the problem's u32 histogram in
 // HBM when it moves on; longer runs go straight to HBM.  The bucket table of
 // the ranks is built per wave from the problem's sorted bounds.
 #pragma once
@@ -25,14 +25,14 @@ namespace rqa {
 constexpr int BMAX_NC = 65535;   // u32 bins cannot overflow: every count is below N_c^2 < 2^32
 constexpr int BNB = 128;         // bucket table entries per wave
 constexpr int BWIN = 256;        // DET column window per wave (samples)
-// Run lengths below BLCAP go to the wave's LDS histogram.  Smaller than the
-// large-N kernels' LCAP: a wave's LDS (histogram with a spare bin per lane and
-// row, table, window) is 6.0 KB for 8 thresholds, so LDS allows 6 waves per
-// SIMD, above what the registers allow; the short series of a batch rarely
-// have runs this long.
-constexpr int BLCAP = 64;
-constexpr int BNSPARE = WAVE;               // spare bins per row, one per lane
-constexpr int BLROW = BLCAP + BNSPARE;      // LDS words per threshold row
+// Run lengths below blcap() go to the wave's LDS histogram, whose rows end in
+// NONES bins for the runs of one step (scan_core's dense form): 6.7 KB a wave
+// with the table and the window at 8 thresholds, so LDS allows 6 waves per
+// SIMD, above what the registers allow.
+template <int TG>
+constexpr int blcap() { return TG <= 8 ? 128 : 64; }
+template <int TG>
+constexpr int blrow() { return lrow<NONES, blcap<TG>()>(); }
 
 // One problem: a series at x + xoff (n = N_c + (m-1) tau samples, followed
 // by at least PAD zeros in the batch buffer), one (tau, emb), nt <= TG live
@@ -65,7 +65,7 @@ __device__ __forceinline__ unsigned long long bkey_at(double, unsigned long long
 
 // The bucket table of rank_of for sorted non-negative bounds b[0 .. nt), built
 // by the 64 lanes of one wave: bucket bk covers high key bits
-// [base + bk<<sh, base + (bk+1)<<sh); the last bucket lies past the largest
+// [(qlo + bk)<<sh, (qlo + bk + 1)<<sh); the last bucket lies past the largest
 // bound.  Entry: the key of the first bound at or above the bucket's start
 // (all-ones if none), the number of bounds below the start, and a flag if the
 // bucket holds two or more bounds (pack_ranks then counts directly).
@@ -73,14 +73,14 @@ template <typename F, int TG>
 __device__ __forceinline__ LutParams batch_lut(const F *b, int nt, LutEntry<F> *lut) {
     const int lane = threadIdx.x & (WAVE - 1);
     LutParams P;
-    P.base = bkey_hi(b[0]);
-    const uint32_t range = bkey_hi(b[nt - 1]) - P.base;
+    const uint32_t klo = bkey_hi(b[0]), khi = bkey_hi(b[nt - 1]);
     int sh = 0;
-    while ((range >> sh) > (uint32_t)(BNB - 2)) sh++;
+    while ((khi >> sh) - (klo >> sh) > (uint32_t)(BNB - 2)) sh++;
     P.sh = sh;
-    P.nb = (int)(range >> sh) + 2;
+    P.qlo = klo >> sh;
+    P.nb = (int)((khi >> sh) - P.qlo) + 2;
     for (int bk = lane; bk < P.nb; bk += WAVE) {
-        const unsigned long long s_hi = (unsigned long long)P.base + ((unsigned long long)bk << sh);
+        const unsigned long long s_hi = (unsigned long long)(P.qlo + (uint32_t)bk) << sh;
         const auto start = bkey_at(F(0), s_hi);
         const auto end = bkey_at(F(0), s_hi + (1ull << sh));
         int r_lo = 0, inside = 0;
@@ -104,43 +104,26 @@ __device__ __forceinline__ LutParams batch_lut(const F *b, int nt, LutEntry<F> *
 // Per-wave LDS of the batched kernel.
 template <typename F, int TG>
 struct BatchWave {
-    uint32_t lh[TG * BLROW];   // run lengths < BLCAP of the current (problem, kind), row t at t * BLROW
+    uint32_t lh[TG * blrow<TG>()];   // run lengths < blcap of the current (problem, kind), row t at t * blrow
     LutEntry<F> lut[BNB];
     F bnd[TG];
     F win[BWIN];
 };
 
-// The word scan of one 32-step block for every threshold of the group, with
-// runs that start at the sequence's first step counted like any other (the
-// sequence is never cut) and runs of BLCAP or more added to row t of `hrow`
-// (u32) straight away.
+// The word scan of one 32-step block for every threshold of the group (the
+// form by the data, as in scan_words), with runs that start at the sequence's
+// first step counted like any other (the sequence is never cut) and runs of
+// blcap() or more added to row t of `hrow` (u32) straight away.
 template <int TG>
 __device__ __forceinline__ void batch_scan(const uint32_t (&R)[8], uint32_t keep, uint32_t force,
-                                           uint32_t (&run)[TG], int nt, uint32_t *lh, uint32_t spare,
-                                           uint32_t *hrow, int64_t hs) {
-    constexpr int B = rank_bits<TG>();
-    uint32_t Pl[B];
-    rank_planes<B>(R, Pl, keep, force);
-    const GeTree<B> G(Pl);
-    bool lead_in = true;
-#pragma unroll
-    for (int t = 0; t < TG; t++) {
-        if (t < nt) {
-            const uint32_t nw = G.ge(t + 1);
-            if (lead_in) {
-                if (__builtin_amdgcn_ballot_w64((~nw | run[t]) != 0u) == 0ull) continue;
-                lead_in = false;
-            }
-            uint32_t *lht = lh + t * BLROW;
-            consume<BLCAP>(
-                nw, run[t], spare, [&](uint32_t b) { lds_inc(&lht[b + 1]); },
-                [&](uint32_t len) { lds_inc(&lht[len]); },
-                [&](uint32_t first) {
-                    const uint32_t tt = opaque(t);
-                    if ((int64_t)first < hs) atomicAdd(&hrow[(size_t)tt * hs + first], 1u);
-                });
-        }
-    }
+                                           uint32_t (&run)[TG], int nt, uint32_t *lh, uint32_t *hrow, int64_t hs,
+                                           ScanMode &md) {
+    const bool dense = md.dense || (md.blk++ & 15) == 0;
+    md.dense = 3 * scan_core<TG, NONES, SCAN_ASK, blcap<TG>()>(
+                       R, keep, force, run, nt, lh, lane_ones<NONES, blcap<TG>()>(), dense,
+                       [&](uint32_t t, uint32_t first) {
+                           if ((int64_t)first < hs) atomicAdd(&hrow[(size_t)t * hs + first], 1u);
+                       }) >= nt;
 }
 
 // The runs still open at the end of a sequence.
@@ -151,8 +134,8 @@ __device__ __forceinline__ void batch_close(const uint32_t (&run)[TG], int nt, u
     for (int t = 0; t < TG; t++) {
         const uint32_t len = run[t];
         if (t < nt && len) {
-            if (len < (uint32_t)BLCAP)
-                lds_inc(&lh[t * BLROW + len]);
+            if (len < (uint32_t)blcap<TG>())
+                lds_inc(&lh[t * blrow<TG>() + len]);
             else if ((int64_t)len < hs)
                 atomicAdd(&hrow[(size_t)opaque(t) * hs + len], 1u);
         }
@@ -164,13 +147,18 @@ template <int TG>
 __device__ __forceinline__ void batch_flush(uint32_t *lh, int nt, uint32_t *hrow, int64_t hs) {
     const int lane = threadIdx.x & (WAVE - 1);
     wave_sync();
-    for (int e = lane; e < TG * BLCAP; e += WAVE) {
-        const int t = e / BLCAP, len = e - t * BLCAP;
-        const uint32_t v = lh[t * BLROW + len];
-        if (v) {
-            if (len && t < nt && len < hs) atomicAdd(&hrow[(size_t)t * hs + len], v);
-            lh[t * BLROW + len] = 0u;
-        }
+    constexpr int CAP = blcap<TG>();
+    for (int e = lane; e < TG * CAP; e += WAVE) {
+        const int t = e / CAP, len = e - t * CAP;
+        uint32_t *row = lh + t * blrow<TG>();
+        uint32_t v = row[len];
+        row[len] = 0u;
+        if (len == 1)
+            for (int k = 0; k < NONES; k++) {
+                v += row[CAP + k];
+                row[CAP + k] = 0u;
+            }
+        if (v && len && t < nt && len < hs) atomicAdd(&hrow[(size_t)t * hs + len], v);
     }
     wave_sync();
 }
@@ -189,16 +177,16 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
     BatchWave<F, TG> &Wv = wv[wave];
-    for (int e = lane; e < TG * BLROW; e += WAVE) Wv.lh[e] = 0u;
+    for (int e = lane; e < TG * blrow<TG>(); e += WAVE) Wv.lh[e] = 0u;
     const int64_t nitems = ipre[np];
-    constexpr int MJ = 8;   // column samples kept in registers (LAM); dimensions past them load per block
+    constexpr int MJ = 4;   // column samples kept in registers (LAM); dimensions past them load per block
 
     int cur = -1, cur_kind = -1;   // (problem, kind) whose runs the LDS histogram holds
     uint32_t *cur_row = nullptr;
     int64_t cur_hs = 0;
     int cur_nt = 0;
     int p = 0;
-    LutParams P{0u, 0, 1};
+    LutParams P{0, 0u, 1};
     while (true) {
         unsigned long long it = 0;
         if (lane == 0) it = atomicAdd(queue, 1ull);
@@ -244,6 +232,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         uint32_t run[TG];
 #pragma unroll
         for (int t = 0; t < TG; t++) run[t] = 0u;
+        ScanMode md;
 
         if (kind == 0) {
             // LAM: band `local`, full columns
@@ -275,8 +264,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                 pack_ranks<F, TG>(s, R, Wv.lut, P, Wv.bnd, nt);
                 // rows past the column's end count as recurrent padding, taken back below
                 const uint32_t fill = nb == BLK ? 0u : (0xFFFFFFFFu << nb);
-                batch_scan<TG>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, Wv.lh, BLCAP - 1 + lane,
-                               cur_row, hs);
+                batch_scan<TG>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, Wv.lh, cur_row, hs, md);
                 if (fill && jv) {
 #pragma unroll
                     for (int t = 0; t < TG; t++) run[t] -= (uint32_t)(BLK - nb);
@@ -321,7 +309,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                 const int64_t nv64 = dlen - s0;
                 const int nvalid = nv64 <= 0 ? 0 : (nv64 >= BLK ? BLK : (int)nv64);
                 const uint32_t vmask = nvalid >= BLK ? 0xFFFFFFFFu : ((1u << nvalid) - 1u);
-                batch_scan<TG>(R, 0xFFFFFFFFu, ~vmask, run, nt, Wv.lh, BLCAP - 1 + lane, cur_row, hs);
+                batch_scan<TG>(R, 0xFFFFFFFFu, ~vmask, run, nt, Wv.lh, cur_row, hs, md);
             }
             if (rv) batch_close<TG>(run, nt, Wv.lh, cur_row, hs);
         }

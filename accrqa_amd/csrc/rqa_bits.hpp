@@ -31,7 +31,6 @@ constexpr uint32_t PRE = 0x40000000u;
 // goes to the slow path), so that the wave's adds that count nothing spread
 // over NSPARE addresses instead of meeting on one.
 constexpr int NSPARE = 16;
-constexpr int LROW = LCAP + NSPARE;    // LDS words per threshold row
 
 // Position of the lowest / highest set bit (as the hardware's find-first-bit
 // instructions): 0xFFFFFFFF for a zero word.  On the device they are the
@@ -112,30 +111,56 @@ RQA_HD void rank_planes(const uint32_t (&R)[8], uint32_t (&P)[B], uint32_t keep 
 }
 
 // Comparator tree over the planes: ge(c) = mask of steps with rank >= c, so
-// nw(t) = ge(t + 1).  lo[c] (c < 2^(B-1)) compares the low B-1 bits; the top
-// bit is applied per threshold.  All indices are compile-time constants
-// after unrolling, so the tree costs one logic operation per node.
+// nw(t) = ge(t + 1).  lo[c] (c < 2^(B-2)) compares the low B-2 bits; the two
+// top bits are applied per threshold, in one three-input operation.  Keeping a
+// quarter of the comparisons instead of half saves a register per four
+// thresholds and 2^(B-2) operations a word, and the registers are what holds
+// the scans' waves per SIMD.  All indices are compile-time constants after
+// unrolling.
 template <int B>
 struct GeTree {
-    static constexpr int H = 1 << (B - 1);
+    static_assert(B >= 2, "at least two planes");
+    static constexpr int H = 1 << (B - 2);
     uint32_t lo[H];
-    uint32_t top;
+    uint32_t mid, top;
 
     RQA_HD GeTree(const uint32_t (&P)[B]) {
         lo[0] = 0xFFFFFFFFu;
 #pragma unroll
-        for (int j = 0; j < B - 1; j++) {
+        for (int j = 0; j < B - 2; j++) {
             const int n = 1 << j;
 #pragma unroll
             for (int c = n; c < 2 * n; c++) lo[c] = P[j] & lo[c - n];
 #pragma unroll
             for (int c = 0; c < n; c++) lo[c] = P[j] | lo[c];
         }
+        mid = P[B - 2];
         top = P[B - 1];
     }
     // rank >= c, for 1 <= c < 2^B
-    RQA_HD uint32_t ge(int c) const { return (c & H) ? (top & lo[c & (H - 1)]) : (top | lo[c & (H - 1)]); }
+    RQA_HD uint32_t ge(int c) const {
+        const uint32_t l = lo[c & (H - 1)];
+        const uint32_t m = (c & H) ? (mid & l) : (mid | l);
+        return (c & (2 * H)) ? (top & m) : (top | m);
+    }
 };
+
+// The steps of a word's inner runs: recurrent ones above the lowest
+// non-recurrent one (~nw & -nw) and at or below the highest (0 for nw == 0);
+// tail = ffbh(nw).
+RQA_HD uint32_t inner_steps(uint32_t nw, uint32_t tail) { return ~nw & (0u - nw) & ones_shr(tail); }
+
+// inner(len) for each run of the steps mid.
+template <class Inner>
+RQA_HD void inner_runs(uint32_t mid, uint32_t nw, Inner &&inner) {
+    while (mid) {
+        // both operands are non-zero: mid by the loop test, nw >> lo because
+        // an inner run ends before the word's last non-recurrent step
+        const uint32_t lo = (uint32_t)__builtin_ctz(mid);
+        inner((uint32_t)__builtin_ctz(nw >> lo));   // ends at the next non-recurrent step
+        mid &= mid + (1u << lo);                     // clear that run
+    }
+}
 
 // One 32-step word of one threshold.  nw: bit u set = step u not recurrent
 // (bit 0 = oldest).  run: recurrent steps carried in from earlier words, with
@@ -162,19 +187,34 @@ RQA_HD void consume(uint32_t nw, uint32_t &run, uint32_t spare, First &&first_bi
     const uint32_t first = add_sat(run, lead);      // the carried run, closed by that first step
     first_bin(umin(first - 1u, spare));             // first = 0 wraps to a spare bin too
     if ((int32_t)first >= (int32_t)CAP) slow(first);
-    // runs strictly inside the word: recurrent steps above the lowest
-    // non-recurrent one (~nw & -nw) and at or below the highest (for nw == 0
-    // mid is 0)
-    uint32_t mid = ~nw & (0u - nw) & ones_shr(tail);
-    while (mid) {
-        // both operands are non-zero: mid by the loop test, nw >> lo because
-        // an inner run ends before the word's last non-recurrent step
-        const uint32_t lo = (uint32_t)__builtin_ctz(mid);
-        inner((uint32_t)__builtin_ctz(nw >> lo));   // ends at the next non-recurrent step
-        mid &= mid + (1u << lo);                     // clear that run
-    }
+    uint32_t mid = inner_steps(nw, tail);
+    inner_runs(mid, nw, inner);
     run = umin(run + 32u, tail);
 }
+
+// The same with the carried run counted only where one closes (first(len), 1
+// <= len < CAP): a compare in the place of the minimum, and no add at all from
+// the lanes that have nothing to count.  In the large-N scans' LDS histograms
+// those adds met four to eight on a spare bin, one after the other: without
+// them, 20 thresholds, N = 131,072, k_lam_hscan takes 3.7 instead of 4.2 ms and
+// k_det_scan 5.1 instead of 5.8.  take(mid) may count and clear some of the
+// word's inner runs (mid: their steps) before the loop reads the rest.
+template <uint32_t CAP, class First, class Take, class Inner, class Slow>
+RQA_HD void consume_word(uint32_t nw, uint32_t &run, First &&first_run, Take &&take, Inner &&inner, Slow &&slow) {
+    static_assert(CAP >= 32, "inner runs (up to 30 steps) always take the histogram");
+    const uint32_t lead = ffbl(nw);
+    const uint32_t tail = ffbh(nw);
+    const uint32_t first = add_sat(run, lead);
+    if (first - 1u < CAP - 1u) first_run(first);
+    if ((int32_t)first >= (int32_t)CAP) slow(first);
+    uint32_t mid = inner_steps(nw, tail);
+    take(mid);
+    inner_runs(mid, nw, inner);
+    run = umin(run + 32u, tail);
+}
+
+// The inner runs of one step among the steps mid.
+RQA_HD uint32_t single_steps(uint32_t mid) { return mid & ~(mid << 1) & ~(mid >> 1); }
 
 // Segment end: (prefix run, suffix run) for the stitch.  A segment whose
 // first run never closed is recurrent throughout: prefix = suffix = length.

@@ -34,6 +34,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "rqa_bits.hpp"
 
 // A translation unit that only needs the device helpers defines
@@ -48,12 +50,12 @@ constexpr int WAVE = 64;
 constexpr int BLK = 32;            // steps per decision word
 constexpr int WG = 256;            // threads per workgroup (4 waves)
 constexpr int WAVES = WG / WAVE;
-// k_lam, fp32 Euclidean up to 16 thresholds: 4 waves per SIMD (128 VGPRs, a
+// k_lam, fp32 up to 16 thresholds: 4 waves per SIMD (128 VGPRs, a
 // few bytes spilled) instead of the compiler's 3 (measured: 61.8 -> 56.0 ms
 // on the default workload); the other instantiations keep what their
 // registers give (1 = no minimum).
 #define RQA_WPE_LAM(F, NORM, TG) \
-    __attribute__((amdgpu_waves_per_eu((sizeof(F) == 4 && (NORM) == 1 && (TG) <= 16) ? 4 : 1)))
+    __attribute__((amdgpu_waves_per_eu((sizeof(F) == 4 && (TG) <= 16) ? 4 : 1)))
 // k_lam_mx, k_det_mx: three waves per SIMD with the line scan (168 VGPRs for
 // 16 thresholds, no spills; left to itself the compiler takes a few registers
 // more and halves that), four without it (the LDS allows four workgroups).
@@ -133,13 +135,15 @@ __device__ __forceinline__ int wave_id() {
 // scratch histogram, counted with workgroup-scope atomics (no other
 // workgroup touches the slice, so the adds stay in the XCD's L2 without
 // contention); longer runs with device-scope atomics straight into the
-// result.  The slice is zeroed on entry and added to the result on exit.
+// result.  The slices are zero between launches (cleared once when they are
+// allocated): on exit a workgroup adds what its slice counted to the result
+// and clears it again.
 constexpr int PCAP = 2048;
 constexpr int PBINS = PCAP - LCAP;   // private bins per threshold
 
 struct Sink {
-    uint32_t *lh;                  // LDS: row t at t * lrow<NSP>(), bins 1 .. LCAP-1, then NSP spare bins
-    uint32_t spare;                // this lane's spare bin (lane_spare), in consume's numbering
+    uint32_t *lh;                  // LDS: row t at t * lrow<NSP>(), bins 1 .. LCAP-1, then NSP ones bins
+    uint32_t ones;                 // this lane's ones bin (lane_ones)
     uint32_t *priv;                // workgroup slice: row t at t * PBINS, bin len - LCAP
     unsigned long long *hist;      // result: row t at t * (nc + 1)
     int64_t nc;
@@ -154,38 +158,53 @@ __device__ __forceinline__ uint32_t *priv_slice(uint32_t *priv_base) {
     return priv_base + (size_t)blockIdx.x * TG * PBINS;
 }
 
-template <int TG>
-__device__ __forceinline__ void priv_zero(uint32_t *priv, int nt, int nthreads) {
-    for (int e = threadIdx.x; e < nt * PBINS; e += nthreads) priv[e] = 0u;
-}
-
-// A kernel's LDS histogram rows hold LCAP bins and NSP spare bins (WAVE / NSP
-// lanes share one): NSP = NSPARE where LDS is tight, WAVE where it is not.
-template <int NSP>
+// A kernel's LDS histogram rows hold CAP bins (LCAP, or more where the LDS of
+// the waves per SIMD that its registers allow leaves room: fewer runs then
+// take the slow path) and NSP ones bins, which collect the runs of one step in
+// the dense form (WAVE / NSP lanes share one).
+constexpr int NONES = 16;
+template <int NSP = NONES, int CAP = LCAP>
 constexpr int lrow() {
-    static_assert(NSP >= 1 && NSP <= WAVE && WAVE % NSP == 0, "spare bins per row");
-    return LCAP + NSP;
+    static_assert(NSP >= 1 && NSP <= WAVE && WAVE % NSP == 0, "ones bins per row");
+    static_assert(CAP >= 32 && CAP <= PCAP, "longer runs have a private bin");
+    return CAP + NSP;
 }
-template <int NSP = NSPARE>
-__device__ __forceinline__ uint32_t lane_spare() {
-    return LCAP - 1 + ((threadIdx.x & (WAVE - 1)) / (WAVE / NSP));
+template <int NSP = NONES, int CAP = LCAP>
+__device__ __forceinline__ uint32_t lane_ones() {
+    return CAP + ((threadIdx.x & (WAVE - 1)) / (WAVE / NSP));
 }
 
 // Adds the workgroup's LDS and private bins to the result (after a barrier):
-// bins 1 .. LCAP-1 of each LDS row (bin 0 and the spare bins count nothing).
-template <int TG, int NSP = NSPARE>
-__device__ __forceinline__ void flush_hist(const uint32_t *lh, uint32_t *priv, int nt, unsigned long long *hist,
-                                           int64_t nc, int nthreads) {
-    for (int e = threadIdx.x; e < TG * LCAP; e += nthreads) {
-        const int t = e / LCAP, b = e - t * LCAP;
-        const uint32_t v = lh[t * lrow<NSP>() + b];
-        if (v && b && t < nt) glob_add(&hist[(size_t)t * (nc + 1) + b], v);
+// bins 1 .. CAP-1 of each LDS row (bin 0 counts nothing), the
+// ones bins with bin 1, and the slice, which is cleared.
+template <int TG, int NSP = NONES, int CAP = LCAP>
+__device__ __forceinline__ void flush_hist(const uint32_t *lh, const Sink &K, int nt, int nthreads) {
+    const int64_t hs = K.nc + 1;
+    for (int e = threadIdx.x; e < TG * CAP; e += nthreads) {
+        const int t = e / CAP, b = e - t * CAP;
+        const uint32_t *row = lh + t * lrow<NSP, CAP>();
+        uint32_t v = row[b];
+        if (b == 1)
+            for (int k = 0; k < NSP; k++) v += row[CAP + k];
+        if (v && b && t < nt && b < hs) glob_add(&K.hist[(size_t)t * hs + b], v);
     }
-    for (int e = threadIdx.x; e < nt * PBINS; e += nthreads) {
-        const uint32_t v = __hip_atomic_load(&priv[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int t = e / PBINS;
-        const int64_t len = LCAP + (e - t * PBINS);
-        if (v && len <= nc) glob_add(&hist[(size_t)t * (nc + 1) + len], v);
+    // four bins a load, four loads in flight, past the L1 (the adds went to L2)
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    static_assert(PBINS % 4 == 0, "rows of whole 16-byte words");
+    uint4 *pv = (uint4 *)K.priv;
+#pragma unroll 4
+    for (int e = threadIdx.x; e < nt * (PBINS / 4); e += nthreads) {
+        const uint4 v = pv[e];
+        if (v.x | v.y | v.z | v.w) {
+            const int t = e / (PBINS / 4);
+            const int64_t len = LCAP + 4 * (e - t * (PBINS / 4));
+            unsigned long long *h = K.hist + (size_t)t * hs + len;
+            pv[e] = make_uint4(0u, 0u, 0u, 0u);
+            if (v.x && len < hs) glob_add(h, v.x);
+            if (v.y && len + 1 < hs) glob_add(h + 1, v.y);
+            if (v.z && len + 2 < hs) glob_add(h + 2, v.z);
+            if (v.w && len + 3 < hs) glob_add(h + 3, v.w);
+        }
     }
 }
 
@@ -219,33 +238,103 @@ __device__ __forceinline__ void close_run(uint2 *slot, uint32_t run) {
 // Thresholds are sorted, so a step that does not recur at t does not recur at
 // any lower threshold, and a run open at t is open at every higher one: the
 // thresholds at which every lane's word is all non-recurrent and no lane has
-// a run open form a prefix.  consume() would change nothing there (no run
-// closes or opens), so the wave skips them, testing up to the first threshold
-// that fails.
-template <int TG, int NSP = NSPARE>
-__device__ __forceinline__ void scan_words(const uint32_t (&R)[8], uint32_t keep, uint32_t force, uint32_t (&run)[TG],
-                                           int nt, const Sink &K, uint2 *cslot, size_t cstride) {
+// a run open form a prefix.  consume_word() would change nothing there (no run
+// closes or opens), so the wave skips them two at a time, by one test of the
+// higher one.  (Testing each threshold until the first that fails took a
+// dozen scalar operations and three branches a threshold; two at a time
+// measured best of 1, 2 and 4.)
+//
+// Form (SCAN_PLAIN, SCAN_DENSE, or SCAN_ASK: dense where the flag says so).
+// Dense: the words' inner runs of one step are taken by bit counts first (six
+// operations and one LDS add spread over the ones bins) and the loop reads
+// the longer ones.  Returns how many thresholds had eight or more lanes with
+// such runs (dense form only).
+enum { SCAN_PLAIN, SCAN_DENSE, SCAN_ASK };
+template <int TG, int NSP, int FORM, int CAP, class Slow>
+__device__ __forceinline__ int scan_core(const uint32_t (&R)[8], uint32_t keep, uint32_t force, uint32_t (&run)[TG],
+                                         int nt, uint32_t *lh, uint32_t ones, bool dense, Slow &&slow) {
     constexpr int B = rank_bits<TG>();
     uint32_t Pl[B];
     rank_planes<B>(R, Pl, keep, force);
     const GeTree<B> G(Pl);
-    bool lead_in = true;
+    int many = 0;
 #pragma unroll
-    for (int t = 0; t < TG; t++) {
-        if (t < nt) {
-            const uint32_t nw = G.ge(t + 1);
-            if (lead_in) {
-                if (__builtin_amdgcn_ballot_w64((~nw | run[t]) != 0u) == 0ull) continue;
-                lead_in = false;
+    for (int g = 0; g < TG; g += 2) {
+        if (g >= nt || __builtin_amdgcn_ballot_w64((~G.ge(g + 2) | run[g + 1]) != 0u) == 0ull) continue;
+#pragma unroll
+        for (int t = g; t < g + 2; t++) {
+            if (t < nt) {
+                uint32_t *lht = lh + t * lrow<NSP, CAP>();
+                consume_word<CAP>(
+                    G.ge(t + 1), run[t], [&](uint32_t len) { lds_inc(&lht[len]); },
+                    [&](uint32_t &mid) {
+                        if (FORM == SCAN_DENSE || (FORM == SCAN_ASK && dense)) {
+                            const uint32_t e1 = single_steps(mid);
+                            many += __popcll(__builtin_amdgcn_ballot_w64(e1 != 0u)) >= 8 ? 1 : 0;
+                            __hip_atomic_fetch_add(&lht[ones], (uint32_t)__popc(e1), __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                            mid ^= e1;
+                        }
+                    },
+                    [&](uint32_t len) { lds_inc(&lht[len]); }, [&](uint32_t first) { slow(opaque(t), first); });
             }
-            uint32_t *lht = K.lh + t * lrow<NSP>();
-            consume(
-                nw, run[t], K.spare, [&](uint32_t b) { lds_inc(&lht[b + 1]); },
-                [&](uint32_t len) { lds_inc(&lht[len]); },
-                [&](uint32_t first) {
-                    const uint32_t tt = opaque(t);
-                    slow_run(first, cslot + (size_t)tt * cstride, K, tt);
-                });
+        }
+    }
+    return many;
+}
+
+template <int TG, int NSP, int FORM, int CAP = LCAP>
+__device__ __forceinline__ int scan_block(const uint32_t (&R)[8], uint32_t keep, uint32_t force, uint32_t (&run)[TG],
+                                          int nt, const Sink &K, uint2 *cslot, size_t cstride, bool dense = false) {
+    return scan_core<TG, NSP, FORM, CAP>(
+        R, keep, force, run, nt, K.lh, K.ones, dense,
+        [&](uint32_t t, uint32_t first) { slow_run(first, cslot + (size_t)t * cstride, K, t); });
+}
+
+// Maps and noise leave mostly runs of one step: the plain loop then runs once
+// per run of the busiest lane (3-8 times a word) and its adds meet on bin 1,
+// which the LDS serves lane by lane.  Smooth series have few such runs and
+// would pay for the bit counts.  So the form follows the data: a wave takes
+// the dense form on every 16th block (scan_loop: every 65th) and keeps it while
+// a third of the thresholds had eight or more lanes with single steps.  N_c = 9,998 logistic,
+// 5 thresholds: k_lam 98 -> 66 us, k_lam_hscan 75 -> 43.
+struct ScanMode {
+    int blk = 0;
+    bool dense = false;
+};
+
+// One block of a kernel whose other work hides the form's test per threshold.
+template <int TG, int NSP = NONES>
+__device__ __forceinline__ void scan_words(const uint32_t (&R)[8], uint32_t keep, uint32_t force, uint32_t (&run)[TG],
+                                           int nt, const Sink &K, uint2 *cslot, size_t cstride, ScanMode &md) {
+    if constexpr (TG > 16) {
+        scan_block<TG, NSP, SCAN_PLAIN>(R, keep, force, run, nt, K, cslot, cstride);   // no registers to spare
+    } else {
+        const bool dense = md.dense || (md.blk++ & 15) == 0;
+        md.dense = 3 * scan_block<TG, NSP, SCAN_ASK>(R, keep, force, run, nt, K, cslot, cstride, dense) >= nt;
+    }
+}
+
+// The blocks b0, b0 + BLK, .. below b1 of a pure scan: block(i0, form) scans
+// one and returns scan_block's count.  Each form has its own loop, because a
+// test per threshold costs a smooth series 3-4 % (N = 262,144, m = 16: 2 ms of
+// 57), and both forms in one loop body more registers than there are.
+template <int TG, typename Block>
+__device__ __forceinline__ void scan_loop(int64_t b0, int64_t b1, int nt, Block &&block) {
+    using Plain = std::integral_constant<int, SCAN_PLAIN>;
+    using Dense = std::integral_constant<int, SCAN_DENSE>;
+    int64_t i0 = b0;
+    if constexpr (TG > 16) {
+        for (; i0 < b1; i0 += BLK) block(i0, Plain{});
+    } else {
+        while (i0 < b1) {
+            int many;
+            do {
+                many = block(i0, Dense{});
+                i0 += BLK;
+            } while (i0 < b1 && 3 * many >= nt);
+            const int64_t end = min(b1, i0 + 64 * BLK);
+            for (; i0 < end; i0 += BLK) block(i0, Plain{});
         }
     }
 }
@@ -265,12 +354,12 @@ __device__ __forceinline__ void close_segment(const uint32_t (&run)[TG], int nt,
 // the high bits of s (exact: a bucket holds at most one bound, whose key is
 // stored with the bucket; a bucket with several bounds sends the wave to a
 // direct count).  Keys are the IEEE bit patterns, which order non-negative
-// values exactly; NaN maps to +inf, i.e. rank T, never recurrent.
+// values exactly, with NaN above them all, i.e. rank T, never recurrent.
 constexpr int NB_MAX = 2048;   // bucket table entries (LDS)
 
 struct LutParams {
-    uint32_t base;   // high key bits of the first bucket
-    int sh;          // bucket width = 1 << sh (in high key bits)
+    int sh;          // bucket width = 1 << sh (in high key bits); bucket edges are multiples of it
+    uint32_t qlo;    // bucket 0's number on the high key >> sh scale
     int nb;          // number of buckets
 };
 
@@ -288,19 +377,30 @@ struct LutEntry<double> {
     uint32_t pad;
 };
 
-__device__ __forceinline__ uint32_t skey(float s) { return min(__float_as_uint(s), 0x7F800000u); }
-__device__ __forceinline__ unsigned long long skey(double s) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(s);
-    return b > 0x7FF0000000000000ull ? 0x7FF0000000000000ull : b;
-}
+__device__ __forceinline__ uint32_t skey(float s) { return __float_as_uint(s); }
+__device__ __forceinline__ unsigned long long skey(double s) { return (unsigned long long)__double_as_longlong(s); }
 __device__ __forceinline__ uint32_t khi(uint32_t k) { return k; }
 __device__ __forceinline__ uint32_t khi(unsigned long long k) { return (uint32_t)(k >> 32); }
 
+// The median of three unsigned values: one instruction clamps a bucket number.
+__device__ __forceinline__ uint32_t umed3(uint32_t v, uint32_t lo, uint32_t hi) {
+    uint32_t r;
+    asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(lo), "v"(hi));
+    return r;
+}
+
+// One shift and one clamp give the bucket, the subtraction of qlo is part of
+// the table's address.  Keys order unsigned: a NaN of either sign lies above
+// every finite key and +inf, in the last bucket.
 template <typename F>
 __device__ __forceinline__ uint32_t rank_of(F s, const LutEntry<F> *lut, const LutParams &P, uint32_t &flags) {
     const auto key = skey(s);
-    const int b = max(min((int)(khi(key) - P.base) >> P.sh, P.nb - 1), 0);
-    const LutEntry<F> e = lut[b];
+    constexpr uint32_t LS = sizeof(F) == 4 ? 3 : 4;   // log2 of the entry's size
+    static_assert(sizeof(LutEntry<F>) == (1u << LS), "entry size");
+    const uint32_t q = umed3(khi(key) >> P.sh, P.qlo, P.qlo + (uint32_t)P.nb - 1u);
+    uint32_t o;   // (q - qlo) entries, in bytes: one instruction where the compiler makes two
+    asm("v_lshl_add_u32 %0, %1, %2, %3" : "=v"(o) : "v"(q), "n"(LS), "s"(0u - (P.qlo << LS)));
+    const LutEntry<F> e = *(const LutEntry<F> *)((const char *)lut + o);
     flags |= e.info;
     return (e.info & 0xFFu) + (key > e.next ? 1u : 0u);
 }
@@ -385,23 +485,22 @@ __global__ __launch_bounds__(WG) RQA_WPE_LAM(F, NORM, TG) void k_lam(const F *__
                                             LamWork W, unsigned long long *__restrict__ hist,
                                             uint2 *__restrict__ carry, uint32_t *__restrict__ priv_base,
                                             uint8_t *__restrict__ tiles) {
-    __shared__ uint32_t lh[TG * LROW];
+    __shared__ uint32_t lh[TG * lrow()];
     __shared__ LutEntry<F> lut_s[NB_MAX];
     __shared__ F bnd_s[TG];
-    for (int e = threadIdx.x; e < TG * LROW; e += WG) lh[e] = 0;
+    for (int e = threadIdx.x; e < TG * lrow(); e += WG) lh[e] = 0;
     load_lut(lut_s, lut, P.nb);
     if (threadIdx.x < TG) bnd_s[threadIdx.x] = S.s[threadIdx.x];
-    priv_zero<TG>(priv_slice<TG>(priv_base), nt, WG);
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
-    const Sink K{lh, lane_spare(), priv, hist, nc};
+    const Sink K{lh, lane_ones(), priv, hist, nc};
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
     const int64_t nbands = (nc + WAVE - 1) / WAVE;
     const int64_t nitems = W.items ? W.nitems : nbands * W.nseg;
     const size_t cstride = (size_t)W.cseg * nc;   // carry stride between thresholds
-    constexpr int MJ = sizeof(F) == 4 ? 16 : 8;  // column samples kept in registers
+    constexpr int MJ = 4;  // column samples kept in registers (16 cost a wave per SIMD and served few calls)
 
     for (int64_t item = (int64_t)blockIdx.x * WAVES + wave; item < nitems; item += (int64_t)gridDim.x * WAVES) {
         int64_t band;
@@ -424,6 +523,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_LAM(F, NORM, TG) void k_lam(const F *__
         uint32_t run[TG];
 #pragma unroll
         for (int t = 0; t < TG; t++) run[t] = jv ? PRE : 0u;
+        ScanMode md;
         // the column's samples x[j + k tau] are the same for every block of the item
         F xjc[MJ];
 #pragma unroll
@@ -453,7 +553,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_LAM(F, NORM, TG) void k_lam(const F *__
             if (tiles) store_tile(tiles, i0 / BLK, band, nbands, R);
             // rows past the segment count as recurrent padding, taken back below
             const uint32_t fill = nb == BLK ? 0u : (0xFFFFFFFFu << nb);
-            scan_words<TG>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, K, cslot, cstride);
+            scan_words<TG>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, K, cslot, cstride, md);
             if (fill && jv) {
 #pragma unroll
                 for (int t = 0; t < TG; t++) run[t] -= (uint32_t)(BLK - nb);
@@ -463,7 +563,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_LAM(F, NORM, TG) void k_lam(const F *__
     }
 
     __syncthreads();
-    flush_hist<TG>(lh, priv, nt, hist, nc, WG);
+    flush_hist<TG>(lh, K, nt, WG);
 }
 
 // ---------------------------------------------------------------- k_det
@@ -478,17 +578,16 @@ __global__ __launch_bounds__(WG) void k_det(const F *__restrict__ x, int64_t nc,
                                             int nseg, const int2 *__restrict__ items, int64_t nitems,
                                             unsigned long long *__restrict__ hist, uint2 *__restrict__ carry,
                                             uint32_t *__restrict__ priv_base) {
-    __shared__ uint32_t lh[TG * LROW];
+    __shared__ uint32_t lh[TG * lrow()];
     __shared__ LutEntry<F> lut_s[NB_MAX];
     __shared__ F win[WAVES][DET_WIN];
     __shared__ F bnd_s[TG];
-    for (int e = threadIdx.x; e < TG * LROW; e += WG) lh[e] = 0;
+    for (int e = threadIdx.x; e < TG * lrow(); e += WG) lh[e] = 0;
     load_lut(lut_s, lut, P.nb);
     if (threadIdx.x < TG) bnd_s[threadIdx.x] = S.s[threadIdx.x];
-    priv_zero<TG>(priv_slice<TG>(priv_base), nt, WG);
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
-    const Sink K{lh, lane_spare(), priv, hist, nc};
+    const Sink K{lh, lane_ones(), priv, hist, nc};
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
@@ -514,6 +613,7 @@ __global__ __launch_bounds__(WG) void k_det(const F *__restrict__ x, int64_t nc,
         uint32_t run[TG];
 #pragma unroll
         for (int t = 0; t < TG; t++) run[t] = rv ? PRE : 0u;
+        ScanMode md;
 
         for (int64_t s0 = sb; s0 < se; s0 += BLK) {
             F s[BLK];
@@ -539,7 +639,7 @@ __global__ __launch_bounds__(WG) void k_det(const F *__restrict__ x, int64_t nc,
             const int64_t nv64 = dlen - s0;
             const int nvalid = nv64 <= 0 ? 0 : (nv64 >= BLK ? BLK : (int)nv64);
             const uint32_t vmask = nvalid >= BLK ? 0xFFFFFFFFu : ((1u << nvalid) - 1u);
-            scan_words<TG>(R, 0xFFFFFFFFu, ~vmask, run, nt, K, cslot, cstride);
+            scan_words<TG>(R, 0xFFFFFFFFu, ~vmask, run, nt, K, cslot, cstride, md);
         }
         // Steps past the strip's end decide 0 for every lane, so a segment cut
         // short by the end of the diagonals reports the same (prefix, suffix)
@@ -548,7 +648,7 @@ __global__ __launch_bounds__(WG) void k_det(const F *__restrict__ x, int64_t nc,
     }
 
     __syncthreads();
-    flush_hist<TG>(lh, priv, nt, hist, nc, WG);
+    flush_hist<TG>(lh, K, nt, WG);
 }
 
 // ---------------------------------------------------------------- k_det_scan
@@ -573,16 +673,15 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 3) void k_det_scan(const ui
                                                  int64_t nitems, unsigned long long *__restrict__ hist,
                                                  uint2 *__restrict__ carry, uint32_t *__restrict__ priv_base) {
     static_assert(DRECS <= 2 * WG, "each thread moves at most two records per block");
-    // 32 thresholds: 8 spare bins per row keep the workgroup's LDS under a
-    // fifth of the CU's, so five fit (16 spare bins: four)
-    constexpr int NSP = TG >= 32 ? 8 : NSPARE;
-    __shared__ uint32_t lh[TG * lrow<NSP>()];
+    // the test for the dense form only where registers allow it
+    constexpr int NSP = TG <= 8 ? NONES : 1;
+    constexpr int CAP = TG == 16 ? 140 : LCAP;
+    __shared__ uint32_t lh[TG * lrow<NSP, CAP>()];
     __shared__ uint32_t tl[DRECS * TREC];
-    for (int e = threadIdx.x; e < TG * lrow<NSP>(); e += WG) lh[e] = 0;
-    priv_zero<TG>(priv_slice<TG>(priv_base), nt, WG);
+    for (int e = threadIdx.x; e < TG * lrow<NSP, CAP>(); e += WG) lh[e] = 0;
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
-    const Sink K{lh, lane_spare<NSP>(), priv, hist, nc};
+    const Sink K{lh, lane_ones<NSP, CAP>(), priv, hist, nc};
 
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
@@ -609,6 +708,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 3) void k_det_scan(const ui
         uint32_t run[TG];
 #pragma unroll
         for (int t = 0; t < TG; t++) run[t] = rv ? PRE : 0u;
+        ScanMode md;
 
         uint4 pf[4];
         auto fetch = [&](int64_t s) {
@@ -658,14 +758,17 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 3) void k_det_scan(const ui
                 const int64_t nv64 = dlen - s0;
                 const int nvalid = nv64 <= 0 ? 0 : (nv64 >= BLK ? BLK : (int)nv64);
                 const uint32_t vmask = nvalid >= BLK ? 0xFFFFFFFFu : ((1u << nvalid) - 1u);
-                scan_words<TG, NSP>(R, 0xFFFFFFFFu, ~vmask, run, nt, K, cslot, cstride);
+                if constexpr (TG <= 8)
+                    scan_words<TG, NSP>(R, 0xFFFFFFFFu, ~vmask, run, nt, K, cslot, cstride, md);
+                else
+                    scan_block<TG, NSP, SCAN_PLAIN, CAP>(R, 0xFFFFFFFFu, ~vmask, run, nt, K, cslot, cstride);
             }
         }
         if (rv && wact) close_segment<TG>(run, nt, cslot, cstride);
     }
 
     __syncthreads();
-    flush_hist<TG, NSP>(lh, priv, nt, hist, nc, WG);
+    flush_hist<TG, NSP, CAP>(lh, K, nt, WG);
 }
 
 // ---------------------------------------------------------------- k_lam_hscan
@@ -690,16 +793,14 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 6) void k_lam_hscan(const u
                                                   int seg_len, int nseg, const int2 *__restrict__ items,
                                                   int64_t nitems, unsigned long long *__restrict__ hist,
                                                   uint2 *__restrict__ carry, uint32_t *__restrict__ priv_base) {
-    // one spare bin per lane up to 16 thresholds; at 32, 8 spare bins per row
-    // keep six workgroups' LDS within the CU's
-    constexpr int NSP = TG >= 32 ? 8 : WAVE;
-    __shared__ uint32_t lh[TG * lrow<NSP>()];
+    constexpr int NSP = TG > 16 ? 1 : NONES;
+    constexpr int CAP = TG == 16 ? 192 : LCAP;
+    __shared__ uint32_t lh[TG * lrow<NSP, CAP>()];
     __shared__ __align__(16) uint32_t tl[WAVES][8 * HW];
-    for (int e = threadIdx.x; e < TG * lrow<NSP>(); e += WG) lh[e] = 0;
-    priv_zero<TG>(priv_slice<TG>(priv_base), nt, WG);
+    for (int e = threadIdx.x; e < TG * lrow<NSP, CAP>(); e += WG) lh[e] = 0;
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
-    const Sink K{lh, lane_spare<NSP>(), priv, hist, nc};
+    const Sink K{lh, lane_ones<NSP, CAP>(), priv, hist, nc};
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
@@ -740,7 +841,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 6) void k_lam_hscan(const u
             v1 = src[1];
         };
         if (has_rows && cb < ce) fetch(cb);
-        for (int64_t c0 = cb; c0 < ce; c0 += BLK) {
+        scan_loop<TG>(cb, ce, nt, [&](int64_t c0, auto form) {
             const int nb = ce - c0 < BLK ? (int)(ce - c0) : BLK;
             wave_sync();   // the previous block's gathers are done
             if (has_rows) {
@@ -761,17 +862,19 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 6) void k_lam_hscan(const u
             }
             // columns past the part count as recurrent padding, taken back below
             const uint32_t fill = nb == BLK ? 0u : (0xFFFFFFFFu << nb);
-            scan_words<TG, NSP>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, K, cslot, cstride);
+            const int many = scan_block<TG, NSP, decltype(form)::value, CAP>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run,
+                                                                        nt, K, cslot, cstride);
             if (fill && jv) {
 #pragma unroll
                 for (int t = 0; t < TG; t++) run[t] -= (uint32_t)(BLK - nb);
             }
-        }
+            return many;
+        });
         if (jv) close_segment<TG>(run, nt, cslot, cstride);
     }
 
     __syncthreads();
-    flush_hist<TG, NSP>(lh, priv, nt, hist, nc, WG);
+    flush_hist<TG, NSP, CAP>(lh, K, nt, WG);
 }
 
 // ---------------------------------------------------------------- k_rp
@@ -1927,7 +2030,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
                                                unsigned long long *__restrict__ hist, uint2 *__restrict__ carry,
                                                uint32_t *__restrict__ priv_base, uint8_t *__restrict__ tiles,
                                                unsigned long long *__restrict__ stats) {
-    __shared__ uint32_t lh[SCAN ? TG * LROW : 1];
+    __shared__ uint32_t lh[SCAN ? TG * lrow() : 1];
     uint32_t st_rank = 0, st_flag = 0, st_exact = 0;
     __shared__ uint8_t lut_s[NBX_LAM];
     __shared__ float bnd_s[NBND];
@@ -1939,7 +2042,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
     // both rounded to fp32, scaled and split into window words
     __shared__ MxWin<2> win[WAVES];
     if constexpr (SCAN)
-        for (int e = threadIdx.x; e < TG * LROW; e += WG) lh[e] = 0;
+        for (int e = threadIdx.x; e < TG * lrow(); e += WG) lh[e] = 0;
     for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
     if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, nt, S.s);
     if constexpr (sizeof(F) == 8)
@@ -1949,10 +2052,9 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
         bndx = bndx_s;
     else
         bndx = bnd_s;
-    if constexpr (SCAN) priv_zero<TG>(priv_slice<TG>(priv_base), nt, WG);
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
-    const Sink K{lh, lane_spare(), priv, hist, nc};
+    const Sink K{lh, lane_ones(), priv, hist, nc};
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
@@ -1992,6 +2094,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
         uint32_t run[TG];
 #pragma unroll
         for (int t = 0; t < TG; t++) run[t] = jv ? PRE : 0u;
+        ScanMode md;
 
         // column window once per item; row window of the first block
         for (int e = lane; e < cspan; e += WAVE) cw[e] = win_word<G>((float)x[j0 + e] * Z.s);
@@ -2028,7 +2131,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
             if (tiles) store_tile(tiles, i0 / BLK, band, nbands, R);
             if constexpr (SCAN) {
                 const uint32_t fill = nb == BLK ? 0u : (0xFFFFFFFFu << nb);
-                scan_words<TG>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, K, cslot, cstride);
+                scan_words<TG>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, K, cslot, cstride, md);
                 if (fill && jv) {
 #pragma unroll
                     for (int t = 0; t < TG; t++) run[t] -= (uint32_t)(BLK - nb);
@@ -2041,7 +2144,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
 
     if constexpr (SCAN) {
         __syncthreads();
-        flush_hist<TG>(lh, priv, nt, hist, nc, WG);
+        flush_hist<TG>(lh, K, nt, WG);
     }
     if constexpr (STATS) {
         if (st_rank) atomicAdd(&stats[0], (unsigned long long)st_rank);
@@ -2528,12 +2631,13 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 6) void k_lam_vscan(const u
                                                   int nt, int seg_len, LamWork W,
                                                   unsigned long long *__restrict__ hist, uint2 *__restrict__ carry,
                                                   uint32_t *__restrict__ priv_base) {
-    __shared__ uint32_t lh[TG * lrow<WAVE>()];
-    for (int e = threadIdx.x; e < TG * lrow<WAVE>(); e += WG) lh[e] = 0;
-    priv_zero<TG>(priv_slice<TG>(priv_base), nt, WG);
+    constexpr int NSP = TG > 16 ? 1 : NONES;
+    constexpr int CAP = TG > 16 ? 192 : 256;
+    __shared__ uint32_t lh[TG * lrow<NSP, CAP>()];
+    for (int e = threadIdx.x; e < TG * lrow<NSP, CAP>(); e += WG) lh[e] = 0;
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
-    const Sink K{lh, lane_spare<WAVE>(), priv, hist, nc};
+    const Sink K{lh, lane_ones<NSP, CAP>(), priv, hist, nc};
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
@@ -2561,23 +2665,25 @@ __global__ __launch_bounds__(WG) RQA_WPE_SCAN(TG, 7, 6) void k_lam_vscan(const u
             v1 = src[1];
         };
         if (ib < ie) fetch(ib);
-        for (int64_t i0 = ib; i0 < ie; i0 += BLK) {
+        scan_loop<TG>(ib, ie, nt, [&](int64_t i0, auto form) {
             const int nb = ie - i0 < BLK ? (int)(ie - i0) : BLK;
             const uint32_t R[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
             if (i0 + BLK < ie) fetch(i0 + BLK);
             // rows past the part count as recurrent padding, taken back below
             const uint32_t fill = nb == BLK ? 0u : (0xFFFFFFFFu << nb);
-            scan_words<TG, WAVE>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run, nt, K, cslot, cstride);
+            const int many = scan_block<TG, NSP, decltype(form)::value, CAP>(R, jv ? ~fill : 0u, jv ? 0u : 0xFFFFFFFFu, run,
+                                                                        nt, K, cslot, cstride);
             if (fill && jv) {
 #pragma unroll
                 for (int t = 0; t < TG; t++) run[t] -= (uint32_t)(BLK - nb);
             }
-        }
+            return many;
+        });
         if (jv) close_segment<TG>(run, nt, cslot, cstride);
     }
 
     __syncthreads();
-    flush_hist<TG, WAVE>(lh, priv, nt, hist, nc, WG);
+    flush_hist<TG, NSP, CAP>(lh, K, nt, WG);
 }
 
 // ---------------------------------------------------------------- k_det_mx
@@ -2597,19 +2703,18 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(true) void k_det_mx(const float *__r
                                                const int2 *__restrict__ items, int64_t nitems,
                                                unsigned long long *__restrict__ hist, uint2 *__restrict__ carry,
                                                uint32_t *__restrict__ priv_base) {
-    __shared__ uint32_t lh[TG * LROW];
+    __shared__ uint32_t lh[TG * lrow()];
     __shared__ uint8_t lut_s[NBX];
     __shared__ uint32_t skew[WAVES][WAVE * SKB / 4];
     __shared__ float bnd_s[NBND];
     // rw: x[s0 .. s0 + 31 + (m-1)tau]; cw: x[c0 .. c0 + 95 + (m-1)tau]
     __shared__ MxWin<3> win[WAVES];
-    for (int e = threadIdx.x; e < TG * LROW; e += WG) lh[e] = 0;
+    for (int e = threadIdx.x; e < TG * lrow(); e += WG) lh[e] = 0;
     for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
     if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, nt, S.s);
-    priv_zero<TG>(priv_slice<TG>(priv_base), nt, WG);
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
-    const Sink K{lh, lane_spare(), priv, hist, nc};
+    const Sink K{lh, lane_ones(), priv, hist, nc};
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = wave_id();
@@ -2641,6 +2746,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(true) void k_det_mx(const float *__r
         uint32_t run[TG];
 #pragma unroll
         for (int t = 0; t < TG; t++) run[t] = rv ? PRE : 0u;
+        ScanMode md;
 
         // operand windows of the first block
         float pr[2], pc[3];
@@ -2715,13 +2821,13 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(true) void k_det_mx(const float *__r
             const int64_t nv64 = dlen - s0;
             const int nvalid = nv64 <= 0 ? 0 : (nv64 >= BLK ? BLK : (int)nv64);
             const uint32_t vmask = nvalid >= BLK ? 0xFFFFFFFFu : ((1u << nvalid) - 1u);
-            scan_words<TG>(R, 0xFFFFFFFFu, ~vmask, run, nt, K, cslot, cstride);
+            scan_words<TG>(R, 0xFFFFFFFFu, ~vmask, run, nt, K, cslot, cstride, md);
         }
         if (rv) close_segment<TG>(run, nt, cslot, cstride);
     }
 
     __syncthreads();
-    flush_hist<TG>(lh, priv, nt, hist, nc, WG);
+    flush_hist<TG>(lh, K, nt, WG);
 }
 
 // ---------------------------------------------------------------- k_stitch
@@ -2759,16 +2865,27 @@ __global__ __launch_bounds__(STT) void k_stitch(const uint2 *__restrict__ carry,
         uint64_t cur = 0;
         auto part = [&](int64_t plen, const uint2 *pc0) {
             const int64_t np = (plen + seg_len - 1) / seg_len;
-            for (int64_t q = 0; q < np; q++) {
-                const uint2 pc = pc0[(size_t)q * nseq];
-                const int64_t L = (q + 1) * seg_len <= plen ? seg_len : plen - q * seg_len;
-                if ((int64_t)pc.x == L) {   // whole segment recurrent
-                    cur += (uint64_t)L;
-                    continue;
+            // eight slots in flight at a time: the loop is a chain of loads otherwise
+            constexpr int NPF = 8;
+            for (int64_t q0 = 0; q0 < np; q0 += NPF) {
+                uint2 pf[NPF];
+#pragma unroll
+                for (int k = 0; k < NPF; k++) pf[k] = pc0[(size_t)min(q0 + k, np - 1) * nseq];
+#pragma unroll
+                for (int k = 0; k < NPF; k++) {
+                    const int64_t q = q0 + k;
+                    if (q < np) {
+                        const uint2 pc = pf[k];
+                        const int64_t L = (q + 1) * seg_len <= plen ? seg_len : plen - q * seg_len;
+                        if ((int64_t)pc.x == L) {   // whole segment recurrent
+                            cur += (uint64_t)L;
+                        } else {
+                            const uint64_t tot = cur + pc.x;
+                            if (tot) count(tot);
+                            cur = pc.y;
+                        }
+                    }
                 }
-                const uint64_t tot = cur + pc.x;
-                if (tot) count(tot);
-                cur = pc.y;
             }
         };
         if (is_det) {

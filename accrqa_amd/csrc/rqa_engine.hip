@@ -2,7 +2,7 @@
 // (include/accrqa_amd.h).
 //
 // One call handles one (tau, emb) block for all thresholds: thresholds are
-// turned into exact comparison bounds, sorted, split into groups of 4/8/16/32
+// turned into exact comparison bounds, sorted, split into groups of 4/8/16/24/32
 // (one pass over the pairs per group), and each group runs on one HIP stream
 //   RR alone:   k_rr -> k_rr_out
 //   LAM:        k_lam | k_lam_mx (column pass; keeps the rank tiles when they
@@ -278,7 +278,9 @@ int init_ctx() {
     return E_OK;
 }
 
-int tg_for(int nt) { return nt <= 4 ? 4 : (nt <= 8 ? 8 : (nt <= 16 ? 16 : 32)); }
+// Threshold group: 24 beside 16 and 32 because the scans' registers and planes
+// go with it (20 thresholds, N = 131,072, maximal norm: 17.9 -> 16.4 ms a call).
+int tg_for(int nt) { return nt <= 4 ? 4 : (nt <= 8 ? 8 : (nt <= 16 ? 16 : (nt <= 24 ? 24 : 32))); }
 
 inline uint32_t hkey(float v) {
     uint32_t b;
@@ -299,19 +301,19 @@ inline unsigned long long key_at(double, unsigned long long hi) {
 
 // Bucket table for the rank of a pair (see rank_of in rqa_device.hpp).  b:
 // the group's bounds, ascending, non-negative and finite.  Bucket bk covers
-// high key bits [base + bk<<sh, base + (bk+1)<<sh); the last bucket lies past
+// high key bits [(qlo + bk)<<sh, (qlo + bk + 1)<<sh); the last bucket lies past
 // the largest bound, so keys clamped into it get rank nt.
 template <typename F>
 void build_lut(const F *b, int nt, rqa::LutEntry<F> *out, rqa::LutParams &P) {
     std::vector<unsigned long long> key(nt);
     for (int t = 0; t < nt; t++) key[t] = hkey(b[t]);
-    const uint32_t base = hhi(decltype(hkey(F(0)))(key[0]));
-    const uint32_t range = hhi(decltype(hkey(F(0)))(key[nt - 1])) - base;
+    const uint32_t lo = hhi(decltype(hkey(F(0)))(key[0])), hi = hhi(decltype(hkey(F(0)))(key[nt - 1]));
     int sh = 0;
-    while ((range >> sh) > (uint32_t)(rqa::NB_MAX - 2)) sh++;
-    const int nb = (int)(range >> sh) + 2;
+    while ((hi >> sh) - (lo >> sh) > (uint32_t)(rqa::NB_MAX - 2)) sh++;
+    const uint32_t qlo = lo >> sh;
+    const int nb = (int)((hi >> sh) - qlo) + 2;
     for (int bk = 0; bk < nb; bk++) {
-        const unsigned long long s_hi = (unsigned long long)base + ((unsigned long long)bk << sh);
+        const unsigned long long s_hi = (unsigned long long)(qlo + (uint32_t)bk) << sh;
         const unsigned long long start = key_at(F(0), s_hi);
         const unsigned long long end = key_at(F(0), s_hi + (1ull << sh));
         int r_lo = 0, inside = 0;
@@ -322,8 +324,8 @@ void build_lut(const F *b, int nt, rqa::LutEntry<F> *out, rqa::LutParams &P) {
         out[bk].next = r_lo < nt ? (decltype(out[bk].next))key[r_lo] : (decltype(out[bk].next))~0ull;
         out[bk].info = (uint32_t)r_lo | (inside >= 2 ? 0x100u : 0u);
     }
-    P.base = base;
     P.sh = sh;
+    P.qlo = qlo;
     P.nb = nb;
 }
 
@@ -474,10 +476,24 @@ int seg_len_for(int64_t nc) {
     return (int)std::min<int64_t>(L, 1 << 29);
 }
 
-// Workgroup-private long-run bins for a launch of `grid` workgroups.
+// Workgroup-private long-run bins for a launch of `grid` workgroups: zero
+// between launches (the kernels clear what they count), so cleared here only
+// when newly allocated, in the order of `st`.
+int ensure_priv_bytes(DevBuf &b, uint64_t &cleared, size_t bytes, hipStream_t st) {
+    int e;
+    if ((e = ensure(b, bytes))) return e;
+    if (cleared != b.gen) {
+        fill_zero((unsigned long long *)b.p, b.cap / 8, st);
+        HIP_TRY(hipGetLastError());
+        cleared = b.gen;
+    }
+    return E_OK;
+}
+uint64_t g_priv_cleared = 0, g_priv2_cleared = 0;   // allocations known zero
+
 template <int TG>
-int ensure_priv(unsigned grid) {
-    return ensure(g_ctx.priv, (size_t)grid * TG * rqa::PBINS * sizeof(uint32_t));
+int ensure_priv(unsigned grid, hipStream_t st) {
+    return ensure_priv_bytes(g_ctx.priv, g_priv_cleared, (size_t)grid * TG * rqa::PBINS * sizeof(uint32_t), st);
 }
 
 // Bytes of the rank tiles the LAM pass keeps for k_det_scan: row blocks
@@ -745,7 +761,7 @@ int det_scan_beside(const uint8_t *tiles, int64_t nbands, int64_t nc, int nt, in
     int e;
     const size_t pd = lds_cap_pad(rqa::k_det_scan<TG>, g_scan_waves);
     const unsigned g = grid_for_wg(rqa::k_det_scan<TG>, d1 - d0, c.ncu, pd);
-    if ((e = ensure(c.priv2, (size_t)g * TG * rqa::PBINS * sizeof(uint32_t)))) return e;
+    if ((e = ensure_priv_bytes(c.priv2, g_priv2_cleared, (size_t)g * TG * rqa::PBINS * sizeof(uint32_t), st))) return e;
     HIP_TRY(hipEventRecord(c.ev_tiles, st));
     HIP_TRY(hipStreamWaitEvent(c.side, c.ev_tiles, 0));
     hipLaunchKernelGGL((rqa::k_det_scan<TG>), dim3(g), dim3(rqa::WG), pd, c.side, tiles, nbands, nc, nt, L, nseg,
@@ -830,7 +846,7 @@ int launch_group_slabs(const F *dx, int64_t nc, int tau, int m, const rqa::Bound
                     if ((e = fork_det())) return e;
                     const size_t pv = lds_cap_pad(rqa::k_lam_vscan<TG>, g_scan_waves);
                     const unsigned gv = grid_for(rqa::k_lam_vscan<TG>, LW.nitems, c.ncu, pv);
-                    if ((e = ensure_priv<TG>(gv))) return e;
+                    if ((e = ensure_priv<TG>(gv, st))) return e;
                     prof_begin("k_lam_vscan", st);
                     hipLaunchKernelGGL((rqa::k_lam_vscan<TG>), dim3(gv), dim3(rqa::WG), pv, st, (const uint8_t *)tiles,
                                        nbands, nc, nt, L, LW, hist, carry, (uint32_t *)c.priv.p);
@@ -841,7 +857,7 @@ int launch_group_slabs(const F *dx, int64_t nc, int tau, int m, const rqa::Bound
             }
             if (!done) {
                 const unsigned g = grid_for(rqa::k_lam<F, NORM, TG>, LW.nitems, c.ncu);
-                if ((e = ensure_priv<TG>(g))) return e;
+                if ((e = ensure_priv<TG>(g, st))) return e;
                 prof_begin("k_lam", st);
                 hipLaunchKernelGGL((rqa::k_lam<F, NORM, TG>), dim3(g), dim3(rqa::WG), 0, st, dx, nc, tau, m, B, nt,
                                    d_lut, P, L, LW, hist, carry, (uint32_t *)c.priv.p, tiles);
@@ -854,7 +870,7 @@ int launch_group_slabs(const F *dx, int64_t nc, int tau, int m, const rqa::Bound
         if (h1 > h0) {
             const size_t ph = lds_cap_pad(rqa::k_lam_hscan<TG>, g_scan_waves);
             const unsigned g = grid_for(rqa::k_lam_hscan<TG>, h1 - h0, c.ncu, ph);
-            if ((e = ensure_priv<TG>(g))) return e;
+            if ((e = ensure_priv<TG>(g, st))) return e;
             prof_begin("k_lam_hscan", st);
             hipLaunchKernelGGL((rqa::k_lam_hscan<TG>), dim3(g), dim3(rqa::WG), ph, st, (const uint8_t *)tiles, nbands,
                                nc, nt, L, nseg, (const int2 *)c.items_lamh.p + h0, h1 - h0, hist, carry,
@@ -865,7 +881,7 @@ int launch_group_slabs(const F *dx, int64_t nc, int tau, int m, const rqa::Bound
         if (want_det && d1 > d0 && !det_pending) {
             const size_t pd = lds_cap_pad(rqa::k_det_scan<TG>, g_scan_waves);
             const unsigned g = grid_for_wg(rqa::k_det_scan<TG>, d1 - d0, c.ncu, pd);
-            if ((e = ensure_priv<TG>(g))) return e;
+            if ((e = ensure_priv<TG>(g, st))) return e;
             prof_begin("k_det_scan", st);
             hipLaunchKernelGGL((rqa::k_det_scan<TG>), dim3(g), dim3(rqa::WG), pd, st, (const uint8_t *)tiles, nbands,
                                nc, nt, L, nseg, (const int2 *)c.items_dets.p + d0, d1 - d0, hist2, carry2,
@@ -1033,7 +1049,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                     if ((e = fork_det())) return e;
                     const size_t pv = lds_cap_pad(rqa::k_lam_vscan<TG>, g_scan_waves);
                     const unsigned gv = grid_for(rqa::k_lam_vscan<TG>, LW.nitems, c.ncu, pv);
-                    if ((e = ensure_priv<TG>(gv))) return e;
+                    if ((e = ensure_priv<TG>(gv, st))) return e;
                     prof_begin("k_lam_vscan", st);
                     hipLaunchKernelGGL((rqa::k_lam_vscan<TG>), dim3(gv), dim3(rqa::WG), pv, st,
                                        (const uint8_t *)tiles, nbands, nc, nt, L, LW, hist, carry,
@@ -1042,7 +1058,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                     HIP_TRY(hipGetLastError());
                 } else {
                     const unsigned g = grid_for(rqa::k_lam_mx<F, TG, true>, LW.nitems, c.ncu);
-                    if ((e = ensure_priv<TG>(g))) return e;
+                    if ((e = ensure_priv<TG>(g, st))) return e;
                     prof_begin("k_lam_mx", st);
                     hipLaunchKernelGGL((rqa::k_lam_mx<F, TG, true>), dim3(g), dim3(rqa::WG), 0, st, dx,
                                        (const float *)c.nrm.p, (const unsigned int *)c.nmax.p, nc, tau, m, Bf, B, nt, (const uint8_t *)c.lut8.p, MP, L,
@@ -1052,7 +1068,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                 }
             } else {
                 const unsigned g = grid_for(rqa::k_lam<F, NORM, TG>, LW.nitems, c.ncu);
-                if ((e = ensure_priv<TG>(g))) return e;
+                if ((e = ensure_priv<TG>(g, st))) return e;
                 prof_begin("k_lam", st);
                 hipLaunchKernelGGL((rqa::k_lam<F, NORM, TG>), dim3(g), dim3(rqa::WG), 0, st, dx, nc, tau, m, B, nt,
                                    d_lut, P, L, LW, hist, carry, (uint32_t *)c.priv.p, tiles);
@@ -1061,7 +1077,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
             }
         } else {
             const unsigned g = grid_for(rqa::k_lam<F, NORM, TG>, LW.nitems, c.ncu);
-            if ((e = ensure_priv<TG>(g))) return e;
+            if ((e = ensure_priv<TG>(g, st))) return e;
             prof_begin("k_lam", st);
             hipLaunchKernelGGL((rqa::k_lam<F, NORM, TG>), dim3(g), dim3(rqa::WG), 0, st, dx, nc, tau, m, B, nt, d_lut,
                                P, L, LW, hist, carry, (uint32_t *)c.priv.p, tiles);
@@ -1072,7 +1088,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
         if (tiles && c.n_items_lamh > 0) {
             const size_t ph = lds_cap_pad(rqa::k_lam_hscan<TG>, g_scan_waves);
             const unsigned g = grid_for(rqa::k_lam_hscan<TG>, c.n_items_lamh, c.ncu, ph);
-            if ((e = ensure_priv<TG>(g))) return e;
+            if ((e = ensure_priv<TG>(g, st))) return e;
             prof_begin("k_lam_hscan", st);
             hipLaunchKernelGGL((rqa::k_lam_hscan<TG>), dim3(g), dim3(rqa::WG), ph, st, (const uint8_t *)tiles, nbands,
                                nc, nt, L, nseg, (const int2 *)c.items_lamh.p, c.n_items_lamh, hist, carry,
@@ -1148,7 +1164,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                 const int64_t nig = c.n_items_dets;
                 const size_t pd = lds_cap_pad(rqa::k_det_scan<TG>, g_scan_waves);
                 const unsigned g = grid_for_wg(rqa::k_det_scan<TG>, nig, c.ncu, pd);
-                if ((e = ensure_priv<TG>(g))) return e;
+                if ((e = ensure_priv<TG>(g, st))) return e;
                 prof_begin("k_det_scan", st);
                 hipLaunchKernelGGL((rqa::k_det_scan<TG>), dim3(g), dim3(rqa::WG), pd, st, (const uint8_t *)tiles,
                                    nbands, nc, nt, L, nseg,
@@ -1168,7 +1184,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                                        (const unsigned int *)c.nmax.p, lut8d);
                     HIP_TRY(hipGetLastError());
                     const unsigned g = grid_for(rqa::k_det_mx<TG>, ni, c.ncu);
-                    if ((e = ensure_priv<TG>(g))) return e;
+                    if ((e = ensure_priv<TG>(g, st))) return e;
                     prof_begin("k_det_mx", st);
                     hipLaunchKernelGGL((rqa::k_det_mx<TG>), dim3(g), dim3(rqa::WG), 0, st, (const float *)dx,
                                        (const float *)c.nrm.p, (const unsigned int *)c.nmax.p, nc, tau, m, Bf, nt,
@@ -1181,7 +1197,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
             }
             if (!done) {
                 const unsigned g = grid_for(rqa::k_det<F, NORM, TG>, ni, c.ncu);
-                if ((e = ensure_priv<TG>(g))) return e;
+                if ((e = ensure_priv<TG>(g, st))) return e;
                 prof_begin("k_det", st);
                 hipLaunchKernelGGL((rqa::k_det<F, NORM, TG>), dim3(g), dim3(rqa::WG), 0, st, dx, nc, tau, m, B, nt,
                                    d_lut, P, L, nseg, (const int2 *)c.items_det.p, ni, hist, carry,
@@ -1248,6 +1264,9 @@ int launch_tg(int TG, const F *dx, int64_t nc, int tau, int m, const F *bounds, 
                                             d_rr, d_det, d_lam, st);
         case 16:
             return launch_group<F, NORM, 16>(dx, nc, tau, m, bounds, nt, lut, P, rr, det, lam, d_lmins, nl, d_perm,
+                                             T, d_rr, d_det, d_lam, st);
+        case 24:
+            return launch_group<F, NORM, 24>(dx, nc, tau, m, bounds, nt, lut, P, rr, det, lam, d_lmins, nl, d_perm,
                                              T, d_rr, d_det, d_lam, st);
         default:
             return launch_group<F, NORM, 32>(dx, nc, tau, m, bounds, nt, lut, P, rr, det, lam, d_lmins, nl, d_perm,
