@@ -2841,13 +2841,25 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(true) void k_det_mx(const float *__r
 // columns, either one part (slots 0 ..) or, split (split != 0), rows [0, V)
 // in slots 0 .. and rows [V, nc) in slots nseg .., V = min(64 (sq/64 + 1),
 // nc).  Part segment q covers [q*seg_len, min((q+1)*seg_len, part length)).
+// Grid (blocks, threshold, part): LAM's and DET's sequences in one launch.
 constexpr int STT = 256;
 constexpr int SCAP = 4096;
 
+struct StitchPart {
+    const uint2 *carry;
+    unsigned long long *hist;
+    int64_t nseq;
+    int is_det, split, cseg;
+};
+
 #ifndef RQA_HELPERS_ONLY
-__global__ __launch_bounds__(STT) void k_stitch(const uint2 *__restrict__ carry, int nt, int64_t nseq, int64_t nc,
-                                                int is_det, int split, int seg_len, int nseg, int cseg,
-                                                unsigned long long *__restrict__ hist) {
+__global__ __launch_bounds__(STT) void k_stitch(StitchPart p0, StitchPart p1, int nt, int64_t nc, int seg_len,
+                                                int nseg) {
+    const StitchPart P = blockIdx.z ? p1 : p0;
+    const uint2 *carry = P.carry;
+    unsigned long long *hist = P.hist;
+    const int64_t nseq = P.nseq;
+    const int is_det = P.is_det, split = P.split, cseg = P.cseg;
     __shared__ uint32_t sh[SCAP];
     const int t = blockIdx.y;   // threshold: the grid has nt rows
     if (t >= nt) return;
@@ -2906,32 +2918,31 @@ __global__ __launch_bounds__(STT) void k_stitch(const uint2 *__restrict__ carry,
 #endif
 
 // ---------------------------------------------------------------- k_finalize
-// One workgroup per threshold.  Turns a line histogram into the reference's
-// five measures for every l_min (AccRQA_functions.cpp:48-133 and
-// rqa_process_length_histogram, AccRQA_CPU_function.cpp:181-204).
-// For DET it first applies correctDETHistogram (AccRQA_CPU_function.cpp:156-162).
-// metric/scan are workspaces of nt*(nc+1) u64 each (suffix sums, written up
-// to the highest non-zero bin below the last).
-// Output per (t, l): 5 values in F, laid out by out_index(t, l).
-constexpr int FIN = 1024;
-
-// Before k_finalize, grid (blocks, threshold): for DET, correctDETHistogram
+// Before k_finalize where histograms are long (FIN_SMALL) or asked for raw,
+// grid (blocks, threshold, part): for DET, correctDETHistogram
 // (AccRQA_CPU_function.cpp:156-162: every bin doubled, then the
 // line-of-identity bin nc incremented); for both, the highest non-zero bin
-// below nc of each threshold, as tops[t] = bin + 1 (0 if none; tops zeroed
-// before the launch).
+// below nc of each threshold, as tops[part * nt + t] = bin + 1 (0 if none;
+// tops zeroed before the launch).
+struct FinPart {
+    unsigned long long *hist;
+    void *out;         // the caller's measures (F), null to write none
+    int is_det;
+};
+
 constexpr int HPT = 256;
 #ifndef RQA_HELPERS_ONLY
-__global__ __launch_bounds__(HPT) void k_hist_prep(unsigned long long *__restrict__ hist, int64_t nc, int is_det,
+__global__ __launch_bounds__(HPT) void k_hist_prep(FinPart p0, FinPart p1, int nt, int64_t nc,
                                                    unsigned long long *__restrict__ tops) {
+    const FinPart P = blockIdx.z ? p1 : p0;
     const int t = blockIdx.y;
     const int64_t hs = nc + 1;
-    unsigned long long *h = hist + (size_t)t * hs;
+    unsigned long long *h = P.hist + (size_t)t * hs;
     unsigned long long best = 0;
     for (int64_t f = (int64_t)blockIdx.x * HPT + threadIdx.x; f < hs; f += (int64_t)gridDim.x * HPT) {
         unsigned long long v = h[f];
-        if (is_det) {
-            v = (unsigned long long)(2.0 * (double)v) + (f == hs - 1 ? 1ull : 0ull);
+        if (P.is_det) {
+            v = 2ull * v + (f == hs - 1 ? 1ull : 0ull);
             h[f] = v;
         }
         if (v && f < hs - 1) best = (unsigned long long)f + 1;   // f grows, so this is the thread's highest
@@ -2943,162 +2954,168 @@ __global__ __launch_bounds__(HPT) void k_hist_prep(unsigned long long *__restric
         if ((int)threadIdx.x < off) red[threadIdx.x] = max(red[threadIdx.x], red[threadIdx.x + off]);
         __syncthreads();
     }
-    if (threadIdx.x == 0 && red[0]) atomicMax(&tops[t], red[0]);
+    if (threadIdx.x == 0 && red[0]) atomicMax(&tops[(size_t)blockIdx.z * nt + t], red[0]);
 }
 #endif
 
+// One workgroup per (threshold, part): turns a line histogram into the
+// reference's five measures for every l_min (AccRQA_functions.cpp:48-133 and
+// rqa_process_length_histogram, AccRQA_CPU_function.cpp:181-204), and LAM's
+// into RR as well.  tops null: the histograms are as counted, and the DET
+// correction and the highest bin are this kernel's part (one launch and no
+// second pass, which short histograms would wait for: N_c = 9,998, both parts,
+// 45 us in seven launches before, 13 in one); else k_hist_prep has run.
+//
+// Lmax and TTmax are the values the reference's bisection over the suffix
+// counts (tertiary_metric) returns for a non-increasing scan: the largest l
+// whose suffix count exceeds the last bin's (DET: the longest line below N_c,
+// 0 if none) or exceeds 0 (LAM: the longest line).  Sums of bins above the
+// highest non-zero one below N_c are skipped, bin N_c is taken by itself.
+constexpr int FIN = 512;
+constexpr int FIN_CACHE = 4096;      // bins kept in LDS
+constexpr int FIN_SMALL = 32768;     // bins up to which one workgroup a threshold reads them all
+constexpr int FIN_L = 4;             // l_min values per pass
+
+// Sums of N values over the workgroup's threads, to every thread.
+template <int N, typename V>
+__device__ __forceinline__ void fin_sum(V (&v)[N], V *sh) {
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        for (int off = WAVE / 2; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off);
+        if (lane == 0) sh[wave * N + k] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        V a = V(0);
+        for (int w = 0; w < FIN / WAVE; w++) a += sh[w * N + k];
+        v[k] = a;
+    }
+}
+
 template <typename F>
-__global__ __launch_bounds__(FIN) void k_finalize(unsigned long long *__restrict__ hist, int64_t nc, int nt,
+__global__ __launch_bounds__(FIN) void k_finalize(FinPart p0, FinPart p1, int64_t nc, int nt,
                                                   const unsigned long long *__restrict__ tops,
-                                                  const int *__restrict__ lmins, int nl,
-                                                  unsigned long long *__restrict__ metric,
-                                                  unsigned long long *__restrict__ scan, F *__restrict__ out,
-                                                  int det_layout, const int *__restrict__ perm, int T,
-                                                  unsigned long long *__restrict__ m0_out) {
+                                                  const int *__restrict__ lmins, int nl, const int *__restrict__ perm,
+                                                  int T, unsigned long long *__restrict__ m0_out,
+                                                  F *__restrict__ rr_out) {
+    __shared__ unsigned long long cache[FIN_CACHE];
+    __shared__ unsigned long long ru[FIN / WAVE * 2 * FIN_L];
+    __shared__ double rd[FIN / WAVE * FIN_L];
+    __shared__ unsigned long long top_s;
+    const FinPart P = blockIdx.y ? p1 : p0;
     const int t = blockIdx.x;
-    if (t >= nt) return;
     const int64_t hs = nc + 1;
-    unsigned long long *h = hist + (size_t)t * hs;
-    unsigned long long *M = metric + (size_t)t * hs;
-    unsigned long long *Sc = scan + (size_t)t * hs;
+    const unsigned long long *h = P.hist + (size_t)t * hs;
     const int tid = threadIdx.x;
-    const bool is_det = det_layout != 0;
+    const bool raw = tops == nullptr;
+    const bool dbl = raw && P.is_det;
+    auto bin = [&](int64_t f) -> unsigned long long { return dbl ? 2ull * h[f] : h[f]; };
 
-    // k_hist_prep has applied the DET correction and found top = the highest
-    // non-zero bin below hs - 1 (-1 if none): the histogram is zero above its
-    // longest line except the line-of-identity bin hs - 1.  Suffix sums are
-    // formed over [0, top] only, and read above it through SC / MM, where only
-    // bin hs - 1 contributes.
-    const int64_t top = (int64_t)tops[t] - 1;
-    const unsigned long long hl = h[hs - 1];
-    const unsigned long long ml_top = (unsigned long long)(hs - 1) * hl;   // M above top
-
-    // suffix sums M[f] = sum_{g >= f} g h[g], Sc[f] = sum_{g >= f} h[g] for
-    // f <= top: tiles of FIN*FPT bins from the top down, FPT consecutive bins
-    // per thread, an inclusive suffix scan of the threads' totals inside each
-    // tile, the tiles above carried in (cm, cs)
-    constexpr int FPT = 8;
-    constexpr int64_t TILE = (int64_t)FIN * FPT;
-    __shared__ unsigned long long bm[FIN], bs[FIN];
-    unsigned long long cm = ml_top, cs = hl;
-    for (int64_t b0 = top >= 0 ? (top / TILE) * TILE : -1; b0 >= 0; b0 -= TILE) {
-        const int64_t f0 = b0 + (int64_t)tid * FPT;
-        unsigned long long v[FPT], lm = 0, ls = 0;
-#pragma unroll
-        for (int k = 0; k < FPT; k++) {
-            v[k] = f0 + k <= top ? h[f0 + k] : 0ull;
-            lm += (unsigned long long)(f0 + k) * v[k];
-            ls += v[k];
-        }
-        bm[tid] = lm;
-        bs[tid] = ls;
+    // the highest non-zero bin below nc (top = bin + 1), M0 = sum f h
+    int64_t top;
+    unsigned long long m[1] = {0ull};
+    if (raw) {
+        unsigned long long best = 0;
+        if (tid == 0) top_s = 0ull;
         __syncthreads();
-        for (int off = 1; off < FIN; off <<= 1) {
-            unsigned long long am = 0, as = 0;
-            if (tid + off < FIN) {
-                am = bm[tid + off];
-                as = bs[tid + off];
-            }
-            __syncthreads();
-            bm[tid] += am;
-            bs[tid] += as;
-            __syncthreads();
+#pragma unroll 8
+        for (int64_t f = tid; f < nc; f += FIN) {
+            const unsigned long long v = bin(f);
+            if (f < FIN_CACHE) cache[f] = v;
+            m[0] += (unsigned long long)f * v;
+            if (v) best = (unsigned long long)f + 1;
         }
-        unsigned long long rm = (tid + 1 < FIN ? bm[tid + 1] : 0ull) + cm;   // bins above my chunk
-        unsigned long long rs = (tid + 1 < FIN ? bs[tid + 1] : 0ull) + cs;
-#pragma unroll
-        for (int k = FPT - 1; k >= 0; k--) {
-            rm += (unsigned long long)(f0 + k) * v[k];
-            rs += v[k];
-            if (f0 + k <= top) {
-                M[f0 + k] = rm;
-                Sc[f0 + k] = rs;
-            }
+        for (int off = WAVE / 2; off > 0; off >>= 1) best = max(best, (unsigned long long)__shfl_xor(best, off));
+        if ((tid & (WAVE - 1)) == 0 && best) atomicMax(&top_s, best);
+    } else {
+        top = (int64_t)tops[(size_t)blockIdx.y * nt + t];
+#pragma unroll 4
+        for (int64_t f = tid; f < top; f += FIN) {
+            const unsigned long long v = h[f];
+            if (f < FIN_CACHE) cache[f] = v;
+            m[0] += (unsigned long long)f * v;
         }
-        const unsigned long long tm = bm[0], ts = bs[0];
-        __syncthreads();
-        cm += tm;
-        cs += ts;
     }
-    __syncthreads();
-    __threadfence_block();
-    auto SC = [&](int64_t f) -> unsigned long long { return f <= top ? Sc[f] : (f <= hs - 1 ? hl : 0ull); };
-    auto MM = [&](int64_t f) -> unsigned long long { return f <= top ? M[f] : (f <= hs - 1 ? ml_top : 0ull); };
-
-    // Lmax / TTmax: the reference's bisection (tertiary_metric), one thread.
-    __shared__ unsigned long long lmax_s;
-    if (tid == 0) {
-        unsigned long long last, start, mid, end, length, mv, mv1;
-        bool found = false;
-        end = hs - 1;
-        mid = hs / 2;
-        last = is_det ? SC((int64_t)end) : 0ull;
-        start = 0;
-        length = hs;
-        while (!found) {
-            mv = SC((int64_t)mid);
-            mv1 = mid > 0 ? SC((int64_t)mid - 1) : 0ull;
-            if (mv == last && mv1 > mv) {
-                mid = mid - 1;
-                found = true;
-            } else if (length == 0) {
-                break;
-            } else if (mid == 0) {
-                break;
-            } else if (mv > last) {
-                start = mid;
-                length = end - start;
-                mid = mid + (length + 1) / 2;
-            } else if (mv == last && mv1 == last) {
-                end = mid;
-                length = end - start;
-                mid = start + (length >> 1);
-            } else {
-                break;   // unreachable for a non-increasing scan
-            }
-        }
-        lmax_s = mid;
-        if (m0_out) m0_out[t] = MM(0);   // recurrence count (sum of l * h[l])
-    }
-    __syncthreads();
-
-    __shared__ double red[FIN];
+    fin_sum(m, ru);
+    if (raw) top = (int64_t)top_s;
+    const unsigned long long hl = bin(nc) + (dbl ? 1ull : 0ull);
+    const unsigned long long m0 = m[0] + (unsigned long long)nc * hl;
     const int ot = perm ? perm[t] : t;   // position of this threshold in the caller's order
-    for (int l = 0; l < nl; l++) {
-        const int64_t lm = lmins[l];
-        const unsigned long long sl = SC(lm);
-        double e = 0.0;
-        for (int64_t f = lm + tid; f <= top; f += FIN) {
-            const double p = (double)h[f] / (double)sl;
-            if (p > 0) e += p * log(p);
+    if (tid == 0 && !P.is_det) {
+        if (m0_out) m0_out[t] = m0;
+        if (rr_out) rr_out[ot] = ((F)(int64_t)m0) / ((F)(int64_t)(nc * nc));
+    }
+    F *out = (F *)P.out;
+    if (!out) return;
+    const double lmax = !P.is_det && hl ? (double)nc : (double)(top ? top - 1 : 0);
+    auto hv = [&](int64_t f) -> unsigned long long { return f < FIN_CACHE ? cache[f] : bin(f); };
+
+    for (int l0 = 0; l0 < nl; l0 += FIN_L) {
+        int64_t lm[FIN_L];
+        unsigned long long sm[2 * FIN_L];   // S = sum h, M = sum f h over f >= l_min
+#pragma unroll
+        for (int q = 0; q < FIN_L; q++) {
+            lm[q] = l0 + q < nl ? lmins[l0 + q] : hs;
+            sm[q] = sm[FIN_L + q] = 0ull;
         }
-        if (tid == 0 && hs - 1 > top && hs - 1 >= lm) {   // bin hs - 1
-            const double p = (double)hl / (double)sl;
-            if (p > 0) e += p * log(p);
+        for (int64_t f = tid; f < top; f += FIN) {
+            const unsigned long long v = hv(f);
+#pragma unroll
+            for (int q = 0; q < FIN_L; q++)
+                if (f >= lm[q]) {
+                    sm[q] += v;
+                    sm[FIN_L + q] += (unsigned long long)f * v;
+                }
         }
-        red[tid] = e;
-        __syncthreads();
-        for (int off = FIN / 2; off > 0; off >>= 1) {
-            if (tid < off) red[tid] += red[tid + off];
-            __syncthreads();
+        fin_sum(sm, ru);
+#pragma unroll
+        for (int q = 0; q < FIN_L; q++)
+            if (nc >= lm[q]) {
+                sm[q] += hl;
+                sm[FIN_L + q] += (unsigned long long)nc * hl;
+            }
+        double E[FIN_L];
+#pragma unroll
+        for (int q = 0; q < FIN_L; q++) {
+            E[q] = 0.0;
+            if (tid == 0 && hl && nc >= lm[q]) {
+                const double p = (double)hl / (double)sm[q];
+                E[q] += p * log(p);
+            }
         }
-        if (tid == 0) {
-            const unsigned long long m0 = MM(0), ml = MM(lm);
-            const double v0 = m0 > 0 ? (double)ml / (double)m0 : __builtin_nan("");
-            const double v1 = sl > 0 ? (double)ml / (double)sl : __builtin_nan("");
-            const double v2 = (double)lmax_s;
-            const double v3 = (-1.0) * red[0];
-            const double v4 = (double)m0 / (double)(nc * nc);
+        for (int64_t f = tid; f < top; f += FIN) {
+            const unsigned long long v = hv(f);
+            if (!v) continue;
+#pragma unroll
+            for (int q = 0; q < FIN_L; q++)
+                if (f >= lm[q]) {
+                    const double p = (double)v / (double)sm[q];
+                    E[q] += p * log(p);
+                }
+        }
+        fin_sum(E, rd);
+        if (tid < FIN_L && l0 + tid < nl) {
+            double e = 0.0;
+            unsigned long long sl = 0, ml = 0;
+#pragma unroll
+            for (int q = 0; q < FIN_L; q++)
+                if (q == tid) {
+                    e = E[q];
+                    sl = sm[q];
+                    ml = sm[FIN_L + q];
+                }
+            const int l = l0 + tid;
             // DET: [T][nL][5] (l fastest); LAM: [nL][T][5] (threshold fastest)
-            const size_t pos = det_layout ? ((size_t)ot * nl + l) : ((size_t)l * T + ot);
-            F *o = out + 5 * pos;
-            o[0] = (F)v0;
-            o[1] = (F)v1;
-            o[2] = (F)v2;
-            o[3] = (F)v3;
-            o[4] = (F)v4;
+            F *o = out + 5 * (P.is_det ? ((size_t)ot * nl + l) : ((size_t)l * T + ot));
+            o[0] = (F)(m0 > 0 ? (double)ml / (double)m0 : __builtin_nan(""));
+            o[1] = (F)(sl > 0 ? (double)ml / (double)sl : __builtin_nan(""));
+            o[2] = (F)lmax;
+            o[3] = (F)((-1.0) * e);
+            o[4] = (F)((double)m0 / (double)(nc * nc));
         }
-        __syncthreads();
     }
 }
 

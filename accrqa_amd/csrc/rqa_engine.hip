@@ -238,8 +238,8 @@ int init_ctx() {
         if (g_ctx.device >= 0) {
             int cur = dev;
             (void)hipSetDevice(g_ctx.device);
-            DevBuf *all[] = {&g_ctx.x,       &g_ctx.hist,       &g_ctx.carry,      &g_ctx.metric,
-                             &g_ctx.scan,    &g_ctx.counts,     &g_ctx.perm,       &g_ctx.lmins,
+            DevBuf *all[] = {&g_ctx.x,       &g_ctx.hist,       &g_ctx.carry,      &g_ctx.counts,
+                                 &g_ctx.perm,       &g_ctx.lmins,
                              &g_ctx.lut,     &g_ctx.nrm,        &g_ctx.nmax,       &g_ctx.lut8,
                              &g_ctx.out_rr,  &g_ctx.out_det,    &g_ctx.out_lam,    &g_ctx.priv,
                              &g_ctx.tiles,   &g_ctx.dump,       &g_ctx.tops,
@@ -330,10 +330,13 @@ void build_lut(const F *b, int nt, rqa::LutEntry<F> *out, rqa::LutParams &P) {
 }
 
 // ---------------------------------------------------------------- launches
-__global__ void k_fill_u64(unsigned long long *p, size_t n) {
+__global__ void k_fill_u64(unsigned long long *p, size_t n, unsigned long long *q, size_t nq) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) p[i] = 0ull;
+    for (; i < n + nq; i += stride) {
+        if (i < n) p[i] = 0ull;
+        else q[i - n] = 0ull;
+    }
 }
 
 template <typename F>
@@ -343,11 +346,12 @@ __global__ void k_pad_copy(const F *__restrict__ src, F *__restrict__ dst, size_
     for (; i < ntot; i += stride) dst[i] = i < n ? src[i] : F(0);
 }
 
-void fill_zero(unsigned long long *p, size_t n, hipStream_t st) {
-    if (!n) return;
-    unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_fill_u64, dim3(blocks), dim3(256), 0, st, p, n);
+void fill_zero2(unsigned long long *p, size_t n, unsigned long long *q, size_t nq, hipStream_t st) {
+    if (!(n + nq)) return;
+    unsigned blocks = (unsigned)std::min<size_t>((n + nq + 255) / 256, 4096);
+    hipLaunchKernelGGL(k_fill_u64, dim3(blocks), dim3(256), 0, st, p, n, q, nq);
 }
+void fill_zero(unsigned long long *p, size_t n, hipStream_t st) { fill_zero2(p, n, nullptr, 0, st); }
 
 // Row t of a group's raw results (hs words) -> out + perm[t] * hs.
 __global__ void k_dump_rows(const unsigned long long *__restrict__ src, size_t hs, const int *__restrict__ perm,
@@ -359,23 +363,31 @@ __global__ void k_dump_rows(const unsigned long long *__restrict__ src, size_t h
         o[i] = s[i];
 }
 
-// k_hist_prep (DET correction, highest occupied bin) then k_finalize (suffix
-// sums, Lmax, ENTR, the five measures) for the nt histograms of a group.
+// The measures of the nt histograms of a group, LAM's and DET's parts in one
+// launch (either may be absent): k_finalize alone for short histograms,
+// k_hist_prep (DET correction, highest occupied bin, over many workgroups)
+// before it for long ones and where the raw rows are asked for.  counts: LAM's
+// recurrence counts; d_rr: RR from them.
 template <typename F>
-int finalize(unsigned long long *hist, int64_t nc, int nt, int is_det, const int *d_lmins, int nl, F *out,
-             const int *d_perm, int T, unsigned long long *m0_out, hipStream_t st) {
+int finalize(unsigned long long *lam_hist, unsigned long long *det_hist, int64_t nc, int nt, const int *d_lmins, int nl,
+             F *d_lam, F *d_det, const int *d_perm, int T, unsigned long long *counts, F *d_rr, hipStream_t st) {
     Ctx &c = g_ctx;
-    int e;
-    if ((e = ensure(c.tops, std::max<size_t>(64, (size_t)nt) * sizeof(unsigned long long)))) return e;
-    unsigned long long *tops = (unsigned long long *)c.tops.p;
-    fill_zero(tops, (size_t)nt, st);
+    int e, np = 0;
+    rqa::FinPart part[2] = {};
+    if (lam_hist) part[np++] = rqa::FinPart{lam_hist, d_lam, 0};
+    if (det_hist) part[np++] = rqa::FinPart{det_hist, d_det, 1};
     const int64_t hs = nc + 1;
-    const unsigned bx = (unsigned)std::min<int64_t>((hs + rqa::HPT - 1) / rqa::HPT, 64);
-    hipLaunchKernelGGL(rqa::k_hist_prep, dim3(bx, nt), dim3(rqa::HPT), 0, st, hist, nc, is_det, tops);
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL((rqa::k_finalize<F>), dim3(nt), dim3(rqa::FIN), 0, st, hist, nc, nt,
-                       (const unsigned long long *)tops, d_lmins, nl, (unsigned long long *)c.metric.p,
-                       (unsigned long long *)c.scan.p, out, is_det, d_perm, T, m0_out);
+    unsigned long long *tops = nullptr;
+    if (hs > rqa::FIN_SMALL || c.dump_det) {
+        if ((e = ensure(c.tops, std::max<size_t>(64, (size_t)np * nt) * sizeof(unsigned long long)))) return e;
+        tops = (unsigned long long *)c.tops.p;
+        fill_zero(tops, (size_t)np * nt, st);
+        const unsigned bx = (unsigned)std::min<int64_t>((hs + rqa::HPT - 1) / rqa::HPT, 64);
+        hipLaunchKernelGGL(rqa::k_hist_prep, dim3(bx, nt, np), dim3(rqa::HPT), 0, st, part[0], part[1], nt, nc, tops);
+        HIP_TRY(hipGetLastError());
+    }
+    hipLaunchKernelGGL((rqa::k_finalize<F>), dim3(nt, np), dim3(rqa::FIN), 0, st, part[0], part[1], nc, nt,
+                       (const unsigned long long *)tops, d_lmins, nl, d_perm, T, counts, d_rr);
     HIP_TRY(hipGetLastError());
     return E_OK;
 }
@@ -542,6 +554,39 @@ int slab_len_for(int64_t nc) {
 
 unsigned stitch_blocks(int64_t nseq) {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>((nseq + rqa::STT - 1) / rqa::STT, 64));
+}
+
+// The end of a group: joined runs, raw rows and measures of LAM (carry / hist)
+// and DET (carry2 / hist2), whichever is asked for, in one launch each.
+template <typename F>
+int finish_group(bool lam, bool det, bool split, int64_t nc, int nt, int L, int nseg, unsigned long long *hist,
+                 const uint2 *carry, unsigned long long *hist2, const uint2 *carry2, const int *d_lmins, int nl,
+                 const int *d_perm, int T, F *d_rr, F *d_det, F *d_lam, hipStream_t st) {
+    Ctx &c = g_ctx;
+    const size_t hs = (size_t)nc + 1;
+    unsigned long long *counts = (unsigned long long *)c.counts.p;
+    rqa::StitchPart part[2] = {};
+    int np = 0, e;
+    if (lam) part[np++] = rqa::StitchPart{carry, hist, nc, 0, split ? 1 : 0, split ? 2 * nseg : nseg};
+    if (det && nc > 1) part[np++] = rqa::StitchPart{carry2, hist2, nc - 1, 1, 0, nseg};
+    if (np) {
+        prof_begin("k_stitch", st);
+        hipLaunchKernelGGL(rqa::k_stitch, dim3(stitch_blocks(nc), nt, np), dim3(rqa::STT), 0, st, part[0], part[1], nt,
+                           nc, L, nseg);
+        prof_end(st);
+        HIP_TRY(hipGetLastError());
+    }
+    if (lam && (e = dump_rows(hist, nt, hs, d_perm, c.dump_lam, st))) return e;
+    prof_begin("k_finalize", st);
+    if ((e = finalize<F>(lam ? hist : nullptr, det ? hist2 : nullptr, nc, nt, d_lmins, nl, d_lam, d_det, d_perm, T,
+                         lam ? counts : nullptr, lam ? d_rr : nullptr, st)))
+        return e;
+    prof_end(st);
+    // the recurrence count of a LAM pass is its histogram's sum of l h[l]
+    if (lam && d_rr && (e = dump_rows(counts, nt, 1, d_perm, c.dump_rr, st))) return e;
+    // finalize leaves h_D doubled with the line-of-identity bin where it is dumped
+    if (det && (e = dump_rows(hist2, nt, hs, d_perm, c.dump_det, st))) return e;
+    return E_OK;
 }
 
 // Work-item tables (uploaded once per (N_c, segment length)):
@@ -786,11 +831,8 @@ int launch_group_slabs(const F *dx, int64_t nc, int tau, int m, const rqa::Bound
     const size_t hs = (size_t)nc + 1;
     const int64_t nbands = (nc + rqa::WAVE - 1) / rqa::WAVE;
     int e;
-    unsigned long long *counts = (unsigned long long *)c.counts.p;
     if ((e = ensure(c.tiles, slab_bytes(nc, L)))) return e;
     if ((e = ensure(c.hist, (size_t)nt * hs * 8))) return e;
-    if ((e = ensure(c.metric, (size_t)nt * hs * 8))) return e;
-    if ((e = ensure(c.scan, (size_t)nt * hs * 8))) return e;
     if ((e = ensure(c.carry, (size_t)nt * (size_t)nc * 2 * nseg * sizeof(uint2)))) return e;
     if (want_det) {
         if ((e = ensure(c.hist2, (size_t)nt * hs * 8))) return e;
@@ -798,8 +840,7 @@ int launch_group_slabs(const F *dx, int64_t nc, int tau, int m, const rqa::Bound
     }
     unsigned long long *hist = (unsigned long long *)c.hist.p, *hist2 = (unsigned long long *)c.hist2.p;
     uint2 *carry = (uint2 *)c.carry.p, *carry2 = (uint2 *)c.carry2.p;
-    fill_zero(hist, (size_t)nt * hs, st);
-    if (want_det) fill_zero(hist2, (size_t)nt * hs, st);
+    fill_zero2(hist, (size_t)nt * hs, hist2, want_det ? (size_t)nt * hs : 0, st);
     const bool mx = NORM == 1 && use_mfma<F>(1, m, tau);
     rqa::Bounds<float, TG> Bf;
     for (int t = 0; t < TG; t++) Bf.s[t] = (float)B.s[t];
@@ -891,33 +932,8 @@ int launch_group_slabs(const F *dx, int64_t nc, int tau, int m, const rqa::Bound
         }
     }
     if (det_pending) HIP_TRY(hipStreamWaitEvent(st, c.ev_det, 0));
-    prof_begin("k_stitch", st);
-    hipLaunchKernelGGL(rqa::k_stitch, dim3(stitch_blocks(nc), nt), dim3(rqa::STT), 0, st, (const uint2 *)carry, nt,
-                       nc, nc, 0, 1, L, nseg, 2 * nseg, hist);
-    prof_end(st);
-    HIP_TRY(hipGetLastError());
-    if ((e = dump_rows(hist, nt, hs, d_perm, c.dump_lam, st))) return e;
-    prof_begin("k_finalize", st);
-    if ((e = finalize<F>(hist, nc, nt, 0, d_lmins, nl, d_lam, d_perm, T, counts, st))) return e;
-    prof_end(st);
-    if (want_rr) {
-        if ((e = dump_rows(counts, nt, 1, d_perm, c.dump_rr, st))) return e;
-        hipLaunchKernelGGL((rqa::k_rr_out<F>), dim3(1), dim3(64), 0, st, (const unsigned long long *)counts, nt, nc,
-                           d_perm, d_rr);
-        HIP_TRY(hipGetLastError());
-    }
-    if (want_det) {
-        prof_begin("k_stitch", st);
-        hipLaunchKernelGGL(rqa::k_stitch, dim3(stitch_blocks(nc - 1), nt), dim3(rqa::STT), 0, st,
-                           (const uint2 *)carry2, nt, nc - 1, nc, 1, 0, L, nseg, nseg, hist2);
-        prof_end(st);
-        HIP_TRY(hipGetLastError());
-        prof_begin("k_finalize", st);
-        if ((e = finalize<F>(hist2, nc, nt, 1, d_lmins, nl, d_det, d_perm, T, nullptr, st))) return e;
-        prof_end(st);
-        if ((e = dump_rows(hist2, nt, hs, d_perm, c.dump_det, st))) return e;
-    }
-    return E_OK;
+    return finish_group<F>(true, want_det, true, nc, nt, L, nseg, hist, carry, hist2, carry2, d_lmins, nl, d_perm, T,
+                           want_rr ? d_rr : nullptr, d_det, d_lam, st);
 }
 
 // One group of up to 32 possibly-recurrent thresholds (sorted bounds).
@@ -982,31 +998,28 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
         }
     }
 
-    if (want_lam || want_det) {
+    // LAM's histogram and carries, and DET's: both are zeroed in one launch, and
+    // with the tile store the DET scan runs beside the LAM scans, once the rank
+    // pass has written the tiles
+    if (want_lam) {
         if ((e = ensure(c.hist, (size_t)nt * hs * 8))) return e;
-        if ((e = ensure(c.metric, (size_t)nt * hs * 8))) return e;
-        if ((e = ensure(c.scan, (size_t)nt * hs * 8))) return e;
         if ((e = ensure(c.carry, (size_t)nt * (size_t)nc * cseg_lam * sizeof(uint2)))) return e;
     }
-    unsigned long long *hist = (unsigned long long *)c.hist.p;
-    uint2 *carry = (uint2 *)c.carry.p;
-    // with the tile store, the DET scan runs beside the LAM scans, into hist2
-    // and carry2, once the rank pass has written the tiles
+    if (want_det) {
+        if ((e = ensure(c.hist2, (size_t)nt * hs * 8))) return e;
+        if ((e = ensure(c.carry2, (size_t)nt * (size_t)std::max<int64_t>(nc - 1, 1) * nseg * sizeof(uint2)))) return e;
+    }
+    unsigned long long *hist = (unsigned long long *)c.hist.p, *hist2 = (unsigned long long *)c.hist2.p;
+    uint2 *carry = (uint2 *)c.carry.p, *carry2 = (uint2 *)c.carry2.p;
+    fill_zero2(hist, want_lam ? (size_t)nt * hs : 0, hist2, want_det ? (size_t)nt * hs : 0, st);
     bool det_forked = false;
     auto fork_det = [&]() -> int {
         if (!tiles || !want_det || nc <= 1 || det_forked || !overlap_on()) return E_OK;
-        int e2;
-        const size_t hs2 = (size_t)nc + 1;
-        if ((e2 = ensure(c.hist2, (size_t)nt * hs2 * 8))) return e2;
-        if ((e2 = ensure(c.carry2, (size_t)nt * (size_t)(nc - 1) * nseg * sizeof(uint2)))) return e2;
-        fill_zero((unsigned long long *)c.hist2.p, (size_t)nt * hs2, st);
         det_forked = true;
-        return det_scan_beside<TG>(tiles, nbands, nc, nt, L, nseg, 0, c.n_items_dets,
-                                   (unsigned long long *)c.hist2.p, (uint2 *)c.carry2.p, st);
+        return det_scan_beside<TG>(tiles, nbands, nc, nt, L, nseg, 0, c.n_items_dets, hist2, carry2, st);
     };
 
     if (want_lam) {
-        fill_zero(hist, (size_t)nt * hs, st);
         if constexpr (NORM == 1) {
             if (use_mfma<F>(1, m, tau)) {
                 rqa::Bounds<float, TG> Bf;
@@ -1096,40 +1109,17 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
             prof_end(st);
             HIP_TRY(hipGetLastError());
         }
-        prof_begin("k_stitch", st);
-        hipLaunchKernelGGL(rqa::k_stitch, dim3(stitch_blocks(nc), nt), dim3(rqa::STT), 0, st, (const uint2 *)carry,
-                           nt, nc, nc, 0, tiles ? 1 : 0, L, nseg, cseg_lam, hist);
-        prof_end(st);
-        HIP_TRY(hipGetLastError());
-        if ((e = dump_rows(hist, nt, hs, d_perm, c.dump_lam, st))) return e;
-        // The LAM histogram covers every recurrent pair of the full matrix once,
-        // so its sum of l*h[l] is the RR count as well.
-        prof_begin("k_finalize", st);
-        if ((e = finalize<F>(hist, nc, nt, 0, d_lmins, nl, d_lam, d_perm, T, counts, st))) return e;
-        prof_end(st);
     }
-    if (want_rr) {
+    if (want_rr && !want_lam) {
         if ((e = dump_rows(counts, nt, 1, d_perm, c.dump_rr, st))) return e;
         hipLaunchKernelGGL((rqa::k_rr_out<F>), dim3(1), dim3(64), 0, st, (const unsigned long long *)counts, nt, nc,
                            d_perm, d_rr);
         HIP_TRY(hipGetLastError());
     }
-    if (want_det && det_forked) {
-        unsigned long long *hist2 = (unsigned long long *)c.hist2.p;
-        HIP_TRY(hipStreamWaitEvent(st, c.ev_det, 0));
-        prof_begin("k_stitch", st);
-        hipLaunchKernelGGL(rqa::k_stitch, dim3(stitch_blocks(nc - 1), nt), dim3(rqa::STT), 0, st,
-                           (const uint2 *)c.carry2.p, nt, nc - 1, nc, 1, 0, L, nseg, nseg, hist2);
-        prof_end(st);
-        HIP_TRY(hipGetLastError());
-        prof_begin("k_finalize", st);
-        if ((e = finalize<F>(hist2, nc, nt, 1, d_lmins, nl, d_det, d_perm, T, nullptr, st))) return e;
-        prof_end(st);
-        if ((e = dump_rows(hist2, nt, hs, d_perm, c.dump_det, st))) return e;
-        return E_OK;
-    }
-    if (want_det) {
-        fill_zero(hist, (size_t)nt * hs, st);
+    if (!want_lam && !want_det) return E_OK;
+    if (det_forked) HIP_TRY(hipStreamWaitEvent(st, c.ev_det, 0));
+    const bool lam_split = want_lam && tiles;
+    if (want_det && !det_forked) {
         if (nc > 1) {
             const int64_t ni = c.n_items_det;
             bool done = false;
@@ -1154,7 +1144,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                     prof_begin("k_lam_mx", st);
                     hipLaunchKernelGGL((rqa::k_lam_mx<F, TG, false>), dim3(g), dim3(rqa::WG), 0, st, dx,
                                        (const float *)c.nrm.p, (const unsigned int *)c.nmax.p, nc, tau, m, Bf, B, nt,
-                                       (const uint8_t *)c.lut8.p, MP, L, RW, hist, carry, (uint32_t *)c.priv.p, tiles,
+                                       (const uint8_t *)c.lut8.p, MP, L, RW, hist2, carry2, (uint32_t *)c.priv.p, tiles,
                                        (unsigned long long *)nullptr);
                     prof_end(st);
                     HIP_TRY(hipGetLastError());
@@ -1168,7 +1158,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                 prof_begin("k_det_scan", st);
                 hipLaunchKernelGGL((rqa::k_det_scan<TG>), dim3(g), dim3(rqa::WG), pd, st, (const uint8_t *)tiles,
                                    nbands, nc, nt, L, nseg,
-                                   (const int2 *)c.items_dets.p, nig, hist, carry, (uint32_t *)c.priv.p);
+                                   (const int2 *)c.items_dets.p, nig, hist2, carry2, (uint32_t *)c.priv.p);
                 prof_end(st);
                 HIP_TRY(hipGetLastError());
                 done = true;
@@ -1189,7 +1179,7 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                     hipLaunchKernelGGL((rqa::k_det_mx<TG>), dim3(g), dim3(rqa::WG), 0, st, (const float *)dx,
                                        (const float *)c.nrm.p, (const unsigned int *)c.nmax.p, nc, tau, m, Bf, nt,
                                        (const uint8_t *)lut8d, MP, L, nseg,
-                                       (const int2 *)c.items_det.p, ni, hist, carry, (uint32_t *)c.priv.p);
+                                       (const int2 *)c.items_det.p, ni, hist2, carry2, (uint32_t *)c.priv.p);
                     prof_end(st);
                     HIP_TRY(hipGetLastError());
                     done = true;
@@ -1200,24 +1190,15 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                 if ((e = ensure_priv<TG>(g, st))) return e;
                 prof_begin("k_det", st);
                 hipLaunchKernelGGL((rqa::k_det<F, NORM, TG>), dim3(g), dim3(rqa::WG), 0, st, dx, nc, tau, m, B, nt,
-                                   d_lut, P, L, nseg, (const int2 *)c.items_det.p, ni, hist, carry,
+                                   d_lut, P, L, nseg, (const int2 *)c.items_det.p, ni, hist2, carry2,
                                    (uint32_t *)c.priv.p);
                 prof_end(st);
                 HIP_TRY(hipGetLastError());
             }
-            prof_begin("k_stitch", st);
-            hipLaunchKernelGGL(rqa::k_stitch, dim3(stitch_blocks(nc - 1), nt), dim3(rqa::STT), 0, st,
-                               (const uint2 *)carry, nt, nc - 1, nc, 1, 0, L, nseg, nseg, hist);
-            prof_end(st);
-            HIP_TRY(hipGetLastError());
         }
-        prof_begin("k_finalize", st);
-        if ((e = finalize<F>(hist, nc, nt, 1, d_lmins, nl, d_det, d_perm, T, nullptr, st))) return e;
-        prof_end(st);
-        // finalize leaves h_D doubled with the line-of-identity bin
-        if ((e = dump_rows(hist, nt, hs, d_perm, c.dump_det, st))) return e;
     }
-    return E_OK;
+    return finish_group<F>(want_lam, want_det, lam_split, nc, nt, L, nseg, hist, carry, hist2, carry2, d_lmins, nl,
+                           d_perm, T, want_rr && want_lam ? d_rr : nullptr, d_det, d_lam, st);
 }
 
 // Thresholds that never recur: empty histograms, measures straight from finalize.
@@ -1228,10 +1209,9 @@ int launch_never(int64_t nc, int nt, bool want_rr, bool want_det, bool want_lam,
     const size_t hs = (size_t)nc + 1;
     int e;
     if ((e = ensure(c.hist, (size_t)nt * hs * 8))) return e;
-    if ((e = ensure(c.metric, (size_t)nt * hs * 8))) return e;
-    if ((e = ensure(c.scan, (size_t)nt * hs * 8))) return e;
+    if ((e = ensure(c.hist2, (size_t)nt * hs * 8))) return e;
     if ((e = ensure(c.counts, std::max<size_t>(64, (size_t)nt) * sizeof(unsigned long long)))) return e;
-    unsigned long long *hist = (unsigned long long *)c.hist.p;
+    unsigned long long *hist = (unsigned long long *)c.hist.p, *hist2 = (unsigned long long *)c.hist2.p;
     unsigned long long *counts = (unsigned long long *)c.counts.p;
     if (want_rr) {
         fill_zero(counts, (size_t)nt, st);
@@ -1240,14 +1220,13 @@ int launch_never(int64_t nc, int nt, bool want_rr, bool want_det, bool want_lam,
         HIP_TRY(hipGetLastError());
         if ((e = dump_rows(counts, nt, 1, d_perm, c.dump_rr, st))) return e;
     }
-    for (int kind = 0; kind < 2; kind++) {
-        const bool det = kind == 1;
-        if (det ? !want_det : !want_lam) continue;
-        fill_zero(hist, (size_t)nt * hs, st);
-        if ((e = finalize<F>(hist, nc, nt, det ? 1 : 0, d_lmins, nl, det ? d_det : d_lam, d_perm, T, nullptr, st)))
-            return e;
-        if ((e = dump_rows(hist, nt, hs, d_perm, det ? c.dump_det : c.dump_lam, st))) return e;
-    }
+    if (!want_lam && !want_det) return E_OK;
+    fill_zero2(hist, want_lam ? (size_t)nt * hs : 0, hist2, want_det ? (size_t)nt * hs : 0, st);
+    if ((e = finalize<F>(want_lam ? hist : nullptr, want_det ? hist2 : nullptr, nc, nt, d_lmins, nl, d_lam, d_det, d_perm,
+                         T, nullptr, nullptr, st)))
+        return e;
+    if (want_lam && (e = dump_rows(hist, nt, hs, d_perm, c.dump_lam, st))) return e;
+    if (want_det && (e = dump_rows(hist2, nt, hs, d_perm, c.dump_det, st))) return e;
     return E_OK;
 }
 
