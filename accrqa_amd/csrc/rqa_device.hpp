@@ -1594,16 +1594,31 @@ __global__ void k_mx_lut(Bounds<float, TG> S, int nt, MxParams P, const unsigned
     lut[b] = (uint8_t)e;
 }
 
-// Bucket of s~ (bucket edges are multiples of 2^sh in key bits): key >> sh,
-// clamped to the table by one median-of-three.  A slightly negative s~
-// (rounding near 0) has a negative bit pattern as an integer and lands in
-// bucket 0, like +0; keys below the table saturate to bucket 0 and keys above
-// it to the last bucket.
-__device__ __forceinline__ uint32_t mx_key_bucket(float st, const MxParams &P) {
-    const int q = __float_as_int(st) >> P.sh;
-    int qc;
-    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(qc) : "v"(q), "v"(P.qlo), "v"(P.qlo + P.nb - 1));
-    return (uint32_t)(qc - P.qlo);
+// Place of s~'s bucket in a table of NBX bytes: bucket edges are multiples of
+// 2^sh in key bits, and bucket number key >> sh lies at its low bits, so after
+// one median-of-three on the bits one bit-field extract is the address (a table
+// that starts at bucket 0 takes a subtraction per element more: k_lam_mx,
+// N = 262,144, m = 16, 16 thresholds, 15.75 ms, 16.04 so; k_rr_mx, N_c = 65,536,
+// four passes of 31 thresholds, 6.01 and 6.21).  A slightly negative
+// s~ (rounding near 0) has a negative bit pattern as an integer and lands in
+// the first bucket, like +0; keys below the table go to the first bucket, keys
+// above it to the last.
+template <int NBX>
+__device__ __forceinline__ uint32_t mx_bucket(float st, const MxParams &P) {
+    static_assert((NBX & (NBX - 1)) == 0, "places are the low bits of bucket numbers");
+    int k;
+    asm("v_med3_i32 %0, %1, %2, %3"
+        : "=v"(k)
+        : "v"(__float_as_int(st)), "v"(P.qlo << P.sh), "v"((P.qlo + P.nb - 1) << P.sh));
+    return __builtin_amdgcn_ubfe((uint32_t)k, (uint32_t)P.sh, (uint32_t)__builtin_ctz(NBX));
+}
+
+// The workgroup's copy of the table, rotated so (P.nb <= NBX; P.nb and P.qlo
+// are multiples of four).
+template <int NBX>
+__device__ __forceinline__ void mx_load_lut(uint8_t *lut_s, const uint8_t *__restrict__ lut, const MxParams &P) {
+    for (int e = threadIdx.x; e < P.nb / 4; e += WG)
+        ((uint32_t *)lut_s)[(P.qlo / 4 + e) & (NBX / 4 - 1)] = ((const uint32_t *)lut)[e];
 }
 
 // Second stage of one flagged element (table byte with bit 7 set): the one
@@ -1884,7 +1899,8 @@ __device__ __forceinline__ floatx16 gram_tile(const MxWin<NT> &W, const float *c
 // bound within reach decides with the pair's own E_ij; fm gets the elements
 // still ambiguous after that (a few in 10^5 pairs), which the caller
 // re-decides in exact order.  ni[e]: norm of element e's row, nj: norm of the
-// lane's column.
+// lane's column; N: the table's size (mx_bucket).
+template <int N>
 __device__ __forceinline__ void tile_ranks(const floatx16 &acc, const float (&ni)[16], float nj, const uint8_t *lut_s,
                                            const MxParams &P, const MxScale &Z, const float *bnd_s, uint32_t (&Rq)[4],
                                            uint32_t &fm, uint32_t &flw) {
@@ -1893,7 +1909,7 @@ __device__ __forceinline__ void tile_ranks(const floatx16 &acc, const float (&ni
 #pragma unroll
     for (int e = 0; e < 16; e++) {
         const float st = fmaf(Z.c2, acc[e], ni[e] + nj);
-        Rq[e & 3] |= (uint32_t)lut_s[mx_key_bucket(st, P)] << (8 * (e >> 2));
+        Rq[e & 3] |= (uint32_t)lut_s[mx_bucket<N>(st, P)] << (8 * (e >> 2));
     }
     fm = 0u;
     // this lane's flagged elements: bit 8g + c <=> element 4g + c (table byte bit 7)
@@ -1963,7 +1979,7 @@ __device__ __forceinline__ void mx_block(const MxWin<2> &Wn, const float *const 
     {
         const floatx16 acc = gram_tile<2, 0, G>(Wn, pa, col, h, m, tau);
         uint32_t Rq[4], f;
-        tile_ranks(acc, ni, nrm[j0 + col], lut_s, P, Z, bnd_s, Rq, f, flw0);
+        tile_ranks<NBX_LAM>(acc, ni, nrm[j0 + col], lut_s, P, Z, bnd_s, Rq, f, flw0);
 #pragma unroll
         for (int c = 0; c < 4; c++) Rr[c] = Rq[c];
         if (j0 + col < nc) fm |= f & rowm;
@@ -1971,7 +1987,7 @@ __device__ __forceinline__ void mx_block(const MxWin<2> &Wn, const float *const 
     {
         const floatx16 acc = gram_tile<2, 1, G>(Wn, pa, col, h, m, tau);
         uint32_t Rq[4], f;
-        tile_ranks(acc, ni, nrm[j0 + 32 + col], lut_s, P, Z, bnd_s, Rq, f, flw1);
+        tile_ranks<NBX_LAM>(acc, ni, nrm[j0 + 32 + col], lut_s, P, Z, bnd_s, Rq, f, flw1);
 #pragma unroll
         for (int c = 0; c < 4; c++) Rr[4 + c] = Rq[c];
         if (j0 + 32 + col < nc) fm |= (f & rowm) << 16;
@@ -2043,7 +2059,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(SCAN) void k_lam_mx(const F *__restr
     __shared__ MxWin<2> win[WAVES];
     if constexpr (SCAN)
         for (int e = threadIdx.x; e < TG * lrow(); e += WG) lh[e] = 0;
-    for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
+    mx_load_lut<NBX_LAM>(lut_s, lut, P);
     if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, nt, S.s);
     if constexpr (sizeof(F) == 8)
         if (threadIdx.x < NBND) bndx_s[threadIdx.x] = (int)threadIdx.x < nt ? SX.s[threadIdx.x] : (F)__builtin_inf();
@@ -2171,7 +2187,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(false) void k_rr_mx(
     __shared__ F bndx_s[sizeof(F) == 8 ? NBND : 1];
     __shared__ MxWin<2> win[WAVES];
     for (int e = threadIdx.x; e < TG; e += WG) acc[e] = 0;
-    for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
+    mx_load_lut<NBX_LAM>(lut_s, lut, P);
     if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, nt, S.s);
     if constexpr (sizeof(F) == 8)
         if (threadIdx.x < NBND) bndx_s[threadIdx.x] = (int)threadIdx.x < nt ? SX.s[threadIdx.x] : (F)__builtin_inf();
@@ -2250,7 +2266,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(false) void k_rp_mx(const float *__r
     __shared__ uint8_t lut_s[NBX_LAM];
     __shared__ float bnd_s[NBND];
     __shared__ MxWin<2> win[WAVES];
-    for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
+    mx_load_lut<NBX_LAM>(lut_s, lut, P);
     if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, 1, &bound);
     __syncthreads();
     const int lane = threadIdx.x & (WAVE - 1);
@@ -2280,7 +2296,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(false) void k_rp_mx(const float *__r
         for (int p = 0; p < 2; p++) {
             const floatx16 acc = p == 0 ? gram_tile<2, 0>(Wn, pa, col, h, m, tau) : gram_tile<2, 1>(Wn, pa, col, h, m, tau);
             uint32_t Rq[4], fm, flw;
-            tile_ranks(acc, ni, nrm[j0 + 32 * p + col], lut_s, P, Z, bnd_s, Rq, fm, flw);
+            tile_ranks<NBX_LAM>(acc, ni, nrm[j0 + 32 * p + col], lut_s, P, Z, bnd_s, Rq, fm, flw);
             const int64_t j = j0 + 32 * p + col;
             const bool jv = j < nc;
             // exact re-decision of the ambiguous elements by their own lane
@@ -2710,7 +2726,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(true) void k_det_mx(const float *__r
     // rw: x[s0 .. s0 + 31 + (m-1)tau]; cw: x[c0 .. c0 + 95 + (m-1)tau]
     __shared__ MxWin<3> win[WAVES];
     for (int e = threadIdx.x; e < TG * lrow(); e += WG) lh[e] = 0;
-    for (int e = threadIdx.x; e < P.nb / 4; e += WG) ((uint32_t *)lut_s)[e] = ((const uint32_t *)lut)[e];
+    mx_load_lut<NBX>(lut_s, lut, P);
     if (threadIdx.x < NBND) bnd_s[threadIdx.x] = mx_bound_slot((int)threadIdx.x, nt, S.s);
     __syncthreads();
     uint32_t *priv = priv_slice<TG>(priv_base);
@@ -2790,7 +2806,7 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(true) void k_det_mx(const float *__r
                                      : p == 1 ? gram_tile<3, 1>(Wn, pa, col, h, m, tau)
                                               : gram_tile<3, 2>(Wn, pa, col, h, m, tau);
                 uint32_t Rq[4], fm, flw;
-                tile_ranks(acc, ni, nrm[c0 + 32 * p + col], lut_s, P, Z, bnd_s, Rq, fm, flw);
+                tile_ranks<NBX>(acc, ni, nrm[c0 + 32 * p + col], lut_s, P, Z, bnd_s, Rq, fm, flw);
                 uint32_t need = 0;
 #pragma unroll
                 for (int e = 0; e < 16; e++) {

@@ -722,8 +722,10 @@ rqa::MxParams mx_params(const float *b, int nt, int m, int nbmax, int extra_u = 
     const uint32_t base = hkey(lo), top = hkey(hi);
     int sh = 0;
     while (((top - base) >> sh) > (uint32_t)(nbmax - 8)) sh++;
-    // bucket edges at multiples of 2^sh: the device finds a bucket as key >> sh
-    const uint32_t base_al = base & ~((1u << sh) - 1u);
+    // bucket edges at multiples of 2^sh: the device finds a bucket as key >> sh;
+    // the first one's number is a multiple of four, so that the table rotates into
+    // its place in LDS (mx_load_lut) by whole words
+    const uint32_t base_al = base & ~((4u << sh) - 1u);
     int nb = (int)((top - base_al) >> sh) + 2;
     nb = (nb + 3) & ~3;
     P.base = base_al;
