@@ -488,6 +488,15 @@ int seg_len_for(int64_t nc) {
     return (int)std::min<int64_t>(L, 1 << 29);
 }
 
+// Segment length of k_rr and k_rr_mx, asked alone: no segment carries anything
+// to a stitch, so a short series is cut finer, down to single blocks, into about
+// 2,048 items (N_c^2 / 128 L of them).  RR of 1,000 samples, m = 2, 3 thresholds:
+// 76 us a call at 256 steps, 63 so (N = 4,001, m = 12, 12 thresholds: 104 and 98).
+int seg_len_rr(int64_t nc) {
+    const int64_t L = (nc * nc / (128 * 2048) + rqa::BLK - 1) / rqa::BLK * rqa::BLK;
+    return (int)std::min<int64_t>(seg_len_for(nc), std::max<int64_t>(L, rqa::BLK));
+}
+
 // Workgroup-private long-run bins for a launch of `grid` workgroups: zero
 // between launches (the kernels clear what they count), so cleared here only
 // when newly allocated, in the order of `st`.
@@ -1298,7 +1307,7 @@ int run_block(const F *dx, size_t n, int tau, int emb, const F *thr, int T, cons
         return e;
     // the split form's shape: the whole tile store, slab by slab, or none
     // (launch_group decides per group whether to take it)
-    c.blk_L = seg_len_for(nc);
+    c.blk_L = d_lam || d_det ? seg_len_for(nc) : seg_len_rr(nc);
     c.blk_slab = false;
     if (d_lam && nc > 1 && g_split == 0 && (g_slab_rows > 0 || !tile_store_fits(nc))) {
         const int Ls = slab_len_for(nc);
