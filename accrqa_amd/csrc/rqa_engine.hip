@@ -1565,7 +1565,9 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
 
 // Shape of a plot's work.  Measured (MI355X, bytes, m = 3 exact unless said):
 //   SMALL  blocks of 32 x 256, every element: enough workgroups for a small
-//          plot (N_c = 1,500: 4.8 us, 64-squares 8.0; 4,000: 9.6 and 9.2)
+//          plot (N_c = 1,500: 4.8 us, 64-squares 8.0), with few dimensions also a
+//          larger one (a call at 4,000, m = 3: 17.5 us, 64-squares 20.9; m = 8:
+//          21.3 and 23.2; m = 32: 44.9 and 42.5; 6,000, m = 1: 17.7 and 19.1)
 //   SQ64   64-squares, mirrored: while the plot fits the 256 MB last-level
 //          cache its short mirrored runs merge there (12,000: 30 us, 256-squares
 //          36, rows 41; 20,000: 140, 128, 102)
@@ -1578,8 +1580,8 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
 //          (m = 16: 265 and 379 us, m = 32: 617 and 490), or at most 15 VALU
 //          operations an element (m = 5: 318 and 346 us, m = 6: 372 and 351)
 enum { RP_SMALL, RP_SQ64, RP_SQ256, RP_ROWS };
-int rp_shape(int64_t nc, const void *out, bool cheap) {
-    if (nc <= 3072) return RP_SMALL;
+int rp_shape(int64_t nc, const void *out, int m, bool cheap) {
+    if (nc <= 3072 || (nc <= 4608 && m <= 8) || (nc <= 8192 && m == 1)) return RP_SMALL;
     if (nc <= 16384) return RP_SQ64;
     if (nc % 128 == 0 && (uintptr_t)out % 128 == 0) return RP_SQ256;
     return cheap ? RP_ROWS : RP_SQ256;
@@ -1663,7 +1665,7 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
             for (int t = 0; t < 4; t++) Bf.s[t] = (float)b;
             if (sym) {
                 prof_begin("k_rp_mx_sq", st);
-                rp_launch_mx(rp_shape(nc, d_out, emb <= 16), (const float *)dx, nc, tau, emb, (float)b,
+                rp_launch_mx(rp_shape(nc, d_out, emb, emb <= 16), (const float *)dx, nc, tau, emb, (float)b,
                              mx_params(Bf.s, 1, emb, rqa::NBX_LAM, rqa::RP_EXTRA_U), (char *)d_out, st);
             } else {
                 const rqa::MxParams MP = mx_params(Bf.s, 1, emb, rqa::NBX_LAM);
@@ -1684,9 +1686,12 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
         }
     }
     if constexpr (sizeof(O) == 1) {
-        if (sym) {
+        // between 2,048 and 3,072 with many dimensions a launch is one wave's sums
+        // long, and the way through LDS only adds to them (2,500, m = 32: 28.6 us a
+        // call, k_rp 26.1; m = 8: 16.4 and 15.1)
+        if (sym && !(nc > 2048 && nc <= 3072 && emb >= 8)) {
             const int ops = (dist == 1 ? 3 : 2) * emb * (sizeof(F) == 8 ? 2 : 1);
-            const int shape = rp_shape(nc, d_out, ops <= 15);
+            const int shape = rp_shape(nc, d_out, emb, ops <= 15);
             prof_begin("k_rp_sq", st);
             if (dist == 1) rp_launch_exact<F, 1>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
             else rp_launch_exact<F, 2>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
