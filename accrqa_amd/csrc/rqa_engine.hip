@@ -470,31 +470,42 @@ void prof_collect(hipStream_t) {
     if (g_prof.pending.size() > 16384) prof_fold();
 }
 
-// Segment length: enough full-column (band, segment) items for about sixteen
-// per resident wave of a full GPU (65536 items; the split LAM and DET passes
-// have items of very different sizes, so they get many), in multiples of 32
-// steps, at least 256.
-// Every segment boundary costs a carry slot per (threshold, sequence) and a
-// join in k_stitch, so segments stay as long as the parallelism allows.  At
-// most 2^29 steps: a run counter (the open-prefix flag, bit 30, plus at most
-// a segment and a word) then stays below 2^31, as the line scan's signed test
-// needs.
-int seg_len_for(int64_t nc) {
-    const int64_t nbands = (nc + rqa::WAVE - 1) / rqa::WAVE;
-    const int64_t nseg = std::max<int64_t>(1, (65536 + nbands - 1) / nbands);
-    int64_t L = (nc + nseg - 1) / nseg;
-    L = std::max<int64_t>(L, 256);
+// Segment lengths, in multiples of 32 steps.  A long series is cut so that
+// every kernel gets about 65,536 items (the triangular ones have items of very
+// different sizes, so they get many).  At most 2^29 steps: a run counter (the
+// open-prefix flag, bit 30, plus at most a segment and a word) then stays below
+// 2^31, as the line scan's signed test needs.
+int seg_of(int64_t L) {
     L = (L + rqa::BLK - 1) / rqa::BLK * rqa::BLK;
     return (int)std::min<int64_t>(L, 1 << 29);
 }
+int64_t seg_by_items(int64_t nc) {
+    const int64_t nbands = (nc + rqa::WAVE - 1) / rqa::WAVE;
+    const int64_t nseg = std::max<int64_t>(1, (65536 + nbands - 1) / nbands);
+    return (nc + nseg - 1) / nseg;
+}
 
-// Segment length of k_rr and k_rr_mx, asked alone: no segment carries anything
-// to a stitch, so a short series is cut finer, down to single blocks, into about
-// 2,048 items (N_c^2 / 128 L of them).  RR of 1,000 samples, m = 2, 3 thresholds:
-// 76 us a call at 256 steps, 63 so (N = 4,001, m = 12, 12 thresholds: 104 and 98).
+// LAM and DET: every segment boundary costs a carry slot per (threshold,
+// sequence) and a join in k_stitch, every segment a serial chain of blocks, so a
+// sequence has 32 segments (40 of them between 16,384 and 49,152, where the items
+// then fill the waves that are resident) unless the items ask for fewer.
+// LAM, 12 thresholds, microseconds a call at m = 3 / m = 16, with at least 256
+// steps and the items' 65,536 alone, and so: N = 700: 165 / 168, 117 / 146;
+// 3,000: 173 / 178, 151 / 179; 16,000: 416 / 414, 388 / 343; 32,000: 1100 / 971,
+// 1009 / 769; 65,000: 3731 / 2376, 3720 / 2199.  Half and twice these lengths were
+// slower at most of the sizes (16,000, m = 16, half: 498).
+int seg_len_for(int64_t nc) {
+    const int64_t nseg = nc > 16384 && nc <= 49152 ? 40 : 32;
+    return seg_of(std::max(seg_by_items(nc), std::max<int64_t>((nc + nseg - 1) / nseg, 64)));
+}
+
+// RR asked alone (k_rr, k_rr_mx): no segment carries anything to a stitch, so a
+// short series is cut finer, down to single blocks, into about 2,048 items
+// (N_c^2 / 128 L of them).  RR of 1,000 samples, m = 2, 3 thresholds: 76 us a call
+// at 256 steps, 61 so (N = 4,001, m = 12, 12 thresholds: 104 and 98).
 int seg_len_rr(int64_t nc) {
-    const int64_t L = (nc * nc / (128 * 2048) + rqa::BLK - 1) / rqa::BLK * rqa::BLK;
-    return (int)std::min<int64_t>(seg_len_for(nc), std::max<int64_t>(L, rqa::BLK));
+    const int64_t L = std::min<int64_t>(nc * nc / (128 * 2048), 256);
+    return seg_of(std::max(seg_by_items(nc), std::max<int64_t>(L, rqa::BLK)));
 }
 
 // Workgroup-private long-run bins for a launch of `grid` workgroups: zero

@@ -26,3 +26,16 @@ def _hists(amd, oracle, n, m, nt, dist, dt, which):
 def test_rr_alone(oracle, nc, m, dist, dt):
     import accrqa_amd as amd
     _hists(amd, oracle, nc + m - 1, m, 3, dist, dt, 1)
+
+
+@pytest.mark.parametrize("nc", [63, 64, 65, 127, 129, 2047, 2049, 2080, 3105])
+@pytest.mark.parametrize("m,dist,dt", [(2, 1, np.float32), (12, 1, np.float32), (3, 2, np.float64), (9, 1, np.float64)])
+@pytest.mark.parametrize("split", [True, False])
+def test_segments(oracle, nc, m, dist, dt, split):
+    import accrqa_amd as amd
+    amd.set_split(amd.SPLIT_AUTO if split else amd.SPLIT_NEVER)
+    try:
+        _hists(amd, oracle, nc + m - 1, m, 5, dist, dt, 7)
+        _hists(amd, oracle, nc + m - 1, m, 3, dist, dt, 2)
+    finally:
+        amd.set_split(amd.SPLIT_AUTO)
