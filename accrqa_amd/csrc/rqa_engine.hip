@@ -212,7 +212,7 @@ int stage_upload(void *dst, const void *src, size_t bytes, hipStream_t st) {
 // Copies up to this size between host arrays and the device pass through the
 // arena (a copy of pageable memory costs the call the runtime's own staging and
 // a wait): RR of 1,000 samples 61 us a call with two pageable copies up and one
-// down, 39 so; the threshold search of 65,551 samples, five calls, 7.1 and 6.0 ms.
+// down, 39 so.
 constexpr size_t STAGE_MAX = (size_t)1 << 20;
 
 int upload_once(const DevBuf &b, Uploaded &u, const void *src, size_t bytes, hipStream_t st) {
