@@ -2980,7 +2980,7 @@ __global__ __launch_bounds__(HPT) void k_hist_prep(FinPart p0, FinPart p1, int n
 // into RR as well.  tops null: the histograms are as counted, and the DET
 // correction and the highest bin are this kernel's part (one launch and no
 // second pass, which short histograms would wait for: N_c = 9,998, both parts,
-// 45 us in seven launches before, 13 in one); else k_hist_prep has run.
+// 45 us in seven launches before, 13-18 in one); else k_hist_prep has run.
 //
 // Lmax and TTmax are the values the reference's bisection over the suffix
 // counts (tertiary_metric) returns for a non-increasing scan: the largest l
@@ -2992,19 +2992,24 @@ constexpr int FIN_CACHE = 4096;      // bins kept in LDS
 constexpr int FIN_SMALL = 32768;     // bins up to which one workgroup a threshold reads them all
 constexpr int FIN_L = 4;             // l_min values per pass
 
-// Sums of N values over the workgroup's threads, to every thread.
+// Sums of the first n of N values (n uniform) over the workgroup's threads, to
+// every thread.  A value's sum is a chain of shuffles, so those of l_min values that
+// are not there are left out: 18 launches of a grid call (two l_min) 1.33 -> 1.28 ms,
+// logistic N = 10,000 (one) 184 -> 180 us.
 template <int N, typename V>
-__device__ __forceinline__ void fin_sum(V (&v)[N], V *sh) {
+__device__ __forceinline__ void fin_sum(V (&v)[N], V *sh, int n = N) {
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < N; k++) {
+        if (k >= n) break;
         for (int off = WAVE / 2; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off);
         if (lane == 0) sh[wave * N + k] = v[k];
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < N; k++) {
+        if (k >= n) break;
         V a = V(0);
         for (int w = 0; w < FIN / WAVE; w++) a += sh[w * N + k];
         v[k] = a;
@@ -3017,7 +3022,7 @@ __device__ __forceinline__ void fin_sum(V (&v)[N], V *sh) {
 // relative terms: 5.0e-18 with a tree over all threads, up to 1.4 times that with
 // plain sums in wave order, 4.8e-18 so (1 us a launch more than those).
 template <int N>
-__device__ __forceinline__ void fin_sum_exact(double (&v)[N], double *sh) {
+__device__ __forceinline__ void fin_sum_exact(double (&v)[N], double *sh, int n) {
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     auto add = [](double &s, double &c, double o, double oc) {
         const double t = s + o, z = t - s;
@@ -3027,6 +3032,7 @@ __device__ __forceinline__ void fin_sum_exact(double (&v)[N], double *sh) {
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < N; k++) {
+        if (k >= n) break;
         double c = 0.0;
         for (int off = WAVE / 2; off > 0; off >>= 1) add(v[k], c, __shfl_xor(v[k], off), __shfl_xor(c, off));
         if (lane == 0) {
@@ -3037,6 +3043,7 @@ __device__ __forceinline__ void fin_sum_exact(double (&v)[N], double *sh) {
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < N; k++) {
+        if (k >= n) break;
         double a = 0.0, c = 0.0;
         for (int w = 0; w < FIN / WAVE; w++) add(a, c, sh[2 * (w * N + k)], sh[2 * (w * N + k) + 1]);
         v[k] = a + c;
@@ -3102,35 +3109,36 @@ __global__ __launch_bounds__(FIN) void k_finalize(FinPart p0, FinPart p1, int64_
     auto hv = [&](int64_t f) -> unsigned long long { return f < FIN_CACHE ? cache[f] : bin(f); };
 
     for (int l0 = 0; l0 < nl; l0 += FIN_L) {
+        const int nq = min(FIN_L, nl - l0);
         int64_t lm[FIN_L];
-        unsigned long long sm[2 * FIN_L];   // S = sum h, M = sum f h over f >= l_min
+        unsigned long long sm[2 * FIN_L];   // (S, M) = (sum h, sum f h) over f >= l_min, per l_min
 #pragma unroll
         for (int q = 0; q < FIN_L; q++) {
             lm[q] = l0 + q < nl ? lmins[l0 + q] : hs;
-            sm[q] = sm[FIN_L + q] = 0ull;
+            sm[2 * q] = sm[2 * q + 1] = 0ull;
         }
         for (int64_t f = tid; f < top; f += FIN) {
             const unsigned long long v = hv(f);
 #pragma unroll
             for (int q = 0; q < FIN_L; q++)
                 if (f >= lm[q]) {
-                    sm[q] += v;
-                    sm[FIN_L + q] += (unsigned long long)f * v;
+                    sm[2 * q] += v;
+                    sm[2 * q + 1] += (unsigned long long)f * v;
                 }
         }
-        fin_sum(sm, ru);
+        fin_sum(sm, ru, 2 * nq);
 #pragma unroll
         for (int q = 0; q < FIN_L; q++)
             if (nc >= lm[q]) {
-                sm[q] += hl;
-                sm[FIN_L + q] += (unsigned long long)nc * hl;
+                sm[2 * q] += hl;
+                sm[2 * q + 1] += (unsigned long long)nc * hl;
             }
         double E[FIN_L];
 #pragma unroll
         for (int q = 0; q < FIN_L; q++) {
             E[q] = 0.0;
             if (tid == 0 && hl && nc >= lm[q]) {
-                const double p = (double)hl / (double)sm[q];
+                const double p = (double)hl / (double)sm[2 * q];
                 E[q] = fma(p, log(p), E[q]);
             }
         }
@@ -3140,11 +3148,11 @@ __global__ __launch_bounds__(FIN) void k_finalize(FinPart p0, FinPart p1, int64_
 #pragma unroll
             for (int q = 0; q < FIN_L; q++)
                 if (f >= lm[q]) {
-                    const double p = (double)v / (double)sm[q];
+                    const double p = (double)v / (double)sm[2 * q];
                     E[q] = fma(p, log(p), E[q]);
                 }
         }
-        fin_sum_exact(E, rd);
+        fin_sum_exact(E, rd, nq);
         if (tid < FIN_L && l0 + tid < nl) {
             double e = 0.0;
             unsigned long long sl = 0, ml = 0;
@@ -3152,8 +3160,8 @@ __global__ __launch_bounds__(FIN) void k_finalize(FinPart p0, FinPart p1, int64_
             for (int q = 0; q < FIN_L; q++)
                 if (q == tid) {
                     e = E[q];
-                    sl = sm[q];
-                    ml = sm[FIN_L + q];
+                    sl = sm[2 * q];
+                    ml = sm[2 * q + 1];
                 }
             const int l = l0 + tid;
             // DET: [T][nL][5] (l fastest); LAM: [nL][T][5] (threshold fastest)
