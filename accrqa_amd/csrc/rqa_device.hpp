@@ -1067,8 +1067,34 @@ __device__ __forceinline__ uint32_t bit_transpose(uint32_t x) {
     return x;
 }
 
-// 16 bytes at any address: one global store, whatever the row's alignment.
+// 16 (2, 4, 8) bytes at any address: one global store, whatever the row's alignment.
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
+
+// The last `left` < 16 columns of a row, from the low bits of v: 8, 4, 2 and 1
+// bytes as the bits of `left` say, for the lanes whose chunk the row's end cuts.
+// (A store per byte there is a chain of up to 15 stores a row, 1 us of a call.)
+__device__ __forceinline__ void rp_store_tail(char *p, uint32_t v, int left, const uint2 *tab) {
+    uint2 a = tab[v & 0xFFu];
+    if (left & 8) {
+        *(u32x2_any *)p = (u32x2_any){a.x, a.y};
+        p += 8;
+        a = tab[(v >> 8) & 0xFFu];
+    }
+    if (left & 4) {
+        *(u32_any *)p = a.x;
+        p += 4;
+        a.x = a.y;
+    }
+    if (left & 2) {
+        *(u16_any *)p = (uint16_t)a.x;
+        p += 2;
+        a.x >>= 16;
+    }
+    if (left & 1) *p = (char)a.x;
+}
 
 // Rows r0 .. r0+S-1, columns c0 .. c0+S-1 of the plot from the row words w.
 template <int S>
@@ -1092,12 +1118,9 @@ __device__ __forceinline__ void rp_store(const uint32_t *w, const uint2 *tab, in
             *(u32x4_any *)(dst + (int64_t)(16 * k) * nc) = (u32x4_any){a.x, a.y, b.x, b.y};
         }
     } else {
-#pragma clang loop vectorize(disable) unroll(disable)
-        for (int k = 0; k < S / 16 && 16 * k < rows; k++) {
-            const uint32_t v = src[16 * k] >> sh;
-#pragma clang loop vectorize(disable) unroll(disable)
-            for (int e = 0; e < (int)left; e++) dst[(int64_t)(16 * k) * nc + e] = (char)((v >> e) & 1u);
-        }
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < S / 16 && 16 * k < rows; k++)
+            rp_store_tail(dst + (int64_t)(16 * k) * nc, src[16 * k] >> sh, (int)left, tab);
     }
 }
 
@@ -1146,11 +1169,13 @@ __global__ __launch_bounds__(S) void k_rp_sq(const F *__restrict__ x, int64_t nc
                     for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xk[k]);
                 }
             }
-            for (int k = RPK; k < m; k++) {
-                const F xv = xj[(int64_t)k * tau];
+            F xv = m > RPK ? xj[(int64_t)RPK * tau] : F(0);
+            for (int k = RPK; k < m; k++) {   // the next dimension's sample is under way
+                const F xn = xj[(int64_t)(k + 1 < m ? k + 1 : k) * tau];
                 const F *xr = x + i0 + (int64_t)k * tau;
 #pragma unroll
                 for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xv);
+                xv = xn;
             }
 #pragma unroll
             for (int u = BLK - 1; u >= 0; u--) push_le(w, s[u], bound);
@@ -1211,12 +1236,9 @@ __device__ __forceinline__ void rp_store_rows(const RpRows<R, C> &M, int64_t r0,
             *(u32x4_any *)(dst + (int64_t)(RP * k) * nc) = (u32x4_any){a.x, a.y, b.x, b.y};
         }
     } else {
-#pragma clang loop vectorize(disable) unroll(disable)
-        for (int k = 0; k < R / RP && RP * k < rows; k++) {
-            const uint32_t v = src[RP * k] >> sh;
-#pragma clang loop vectorize(disable) unroll(disable)
-            for (int e = 0; e < (int)left; e++) dst[(int64_t)(RP * k) * nc + e] = (char)((v >> e) & 1u);
-        }
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < R / RP && RP * k < rows; k++)
+            rp_store_tail(dst + (int64_t)(RP * k) * nc, src[RP * k] >> sh, (int)left, M.tab);
     }
 }
 
@@ -1251,11 +1273,13 @@ __global__ __launch_bounds__(WG) void k_rp_row(const F *__restrict__ x, int64_t 
                     for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xk[k]);
                 }
             }
-            for (int k = RPK; k < m; k++) {
-                const F xv = xj[(int64_t)k * tau];
+            F xv = m > RPK ? xj[(int64_t)RPK * tau] : F(0);
+            for (int k = RPK; k < m; k++) {   // the next dimension's sample is under way
+                const F xn = xj[(int64_t)(k + 1 < m ? k + 1 : k) * tau];
                 const F *xr = x + i0 + (int64_t)k * tau;
 #pragma unroll
                 for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xv);
+                xv = xn;
             }
             uint32_t w = 0u;
 #pragma unroll

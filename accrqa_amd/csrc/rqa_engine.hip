@@ -1602,28 +1602,47 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
     return E_OK;
 }
 
-// Shape of a plot's work.  Measured (MI355X, bytes, m = 3 exact unless said):
+// Shape of a plot's work.  Measured (MI355X, bytes; microseconds a call, exact
+// form, fp32 and Euclidean unless said):
 //   SMALL  blocks of 32 x 256, every element: enough workgroups for a small
-//          plot (N_c = 1,500: 4.8 us, 64-squares 8.0), with few dimensions also a
-//          larger one (a call at 4,000, m = 3: 17.5 us, 64-squares 20.9; m = 8:
-//          21.3 and 23.2; m = 32: 44.9 and 42.5; 6,000, m = 1: 17.7 and 19.1)
+//          plot (1,500, m = 3: 11.6, 64-squares 14.2, k_rp4 12.7), with few
+//          dimensions also a larger one (3,600, m = 3: 15.0, 64-squares 15.5;
+//          m = 5: 16.6 and 16.5; maximal, m = 8: 20.1 and 18.5; with one
+//          dimension: 11,000: 31, 64-squares 37, k_rp4 33)
 //   SQ64   64-squares, mirrored: while the plot fits the 256 MB last-level
-//          cache its short mirrored runs merge there (12,000: 30 us, 256-squares
-//          36, rows 41; 20,000: 140, 128, 102)
+//          cache its short mirrored runs merge there (12,000, m = 3: 35,
+//          256-squares 43, rows 45; 20,000: 146, 134, 105)
 //   SQ256  256-squares, mirrored: large plots whose rows start on 128-byte
-//          lines, so every run is whole lines (65,536: 0.88 ms, rows 1.03)
+//          lines, so every run is whole lines (65,536: 880, rows 1,030)
 //   ROWS   blocks of 64 (MFMA, large: 128) x 1,024, every element: other large
 //          plots, where the runs' partial lines cost more than the second
-//          half's decisions (30,011: 225 us, 256-squares 346), as long as the
-//          decisions are cheap: the MFMA form in one chunk of 16 dimensions
-//          (m = 16: 265 and 379 us, m = 32: 617 and 490), or at most 15 VALU
-//          operations an element (m = 5: 318 and 346 us, m = 6: 372 and 351)
+//          half's decisions, as long as the decisions are cheap: the MFMA form
+//          in one chunk of 16 dimensions (28,000, m = 16: 216, 256-squares 287;
+//          30,011, m = 32: 617 and 490) or at most 16 VALU operations an element
+//          (30,011, m = 3: 226 and 356; maximal, m = 4: 302 and 361, m = 5:
+//          358 and 347; fp64, m = 2: 263 and 351, m = 3 at 40,000: 556 and
+//          477); with one dimension from 13,312 on (14,000: 41.5, SMALL 43,
+//          64-squares 46; 32,768: 174, 256-squares 221)
 enum { RP_SMALL, RP_SQ64, RP_SQ256, RP_ROWS };
 int rp_shape(int64_t nc, const void *out, int m, bool cheap) {
-    if (nc <= 3072 || (nc <= 4608 && m <= 8) || (nc <= 8192 && m == 1)) return RP_SMALL;
+    if (m == 1) return nc <= 13312 ? RP_SMALL : RP_ROWS;
+    if (nc <= 3072 || (nc <= 4096 && m <= 3)) return RP_SMALL;
     if (nc <= 16384) return RP_SQ64;
     if (nc % 128 == 0 && (uintptr_t)out % 128 == 0) return RP_SQ256;
     return cheap ? RP_ROWS : RP_SQ256;
+}
+
+// Small plots in the exact form that stay with one store per decision: fp64
+// with k_rp4's waves of 8 rows, whose chains are a quarter as long as the
+// blocks' of 32 (500: 4.0 us in the kernel at m = 3, 4.4 in blocks; maximal,
+// m = 16: a call 13.3 and 15.9; 2,300, m = 32, Euclidean: 29.8 and 30.5), and
+// odd sizes in fp32 with many dimensions of the maximal norm (1,250, m = 32:
+// 18.3 and 19.4).
+template <typename F>
+bool rp_direct(int64_t nc, const void *out, int m, int dist) {
+    if (sizeof(F) == 8)
+        return nc % 4 == 0 && (uintptr_t)out % 4 == 0 && (nc <= 1024 || (nc <= 3072 && m >= (dist == 1 ? 16 : 8)));
+    return dist == 2 && m >= 16 && nc % 4 != 0 && nc <= 1536;
 }
 
 unsigned rp_grid(int64_t nc, int64_t S) { return (unsigned)rqa::rp_items((nc + S - 1) / S); }
@@ -1664,8 +1683,8 @@ void rp_launch_mx(int shape, const float *dx, int64_t nc, int tau, int m, float 
         case RP_SMALL: row(rqa::k_rp_mx_row<32, 256>, rqa::rp_blocks<32, 256>(nc)); break;
         case RP_SQ64: sq(rqa::k_rp_mx_sq<64>, 64); break;
         case RP_SQ256: sq(rqa::k_rp_mx_sq<256>, 256); break;
-        default:
-            if (nc > 24576) row(rqa::k_rp_mx_row<128, 1024>, rqa::rp_blocks<128, 1024>(nc));
+        default:   // 24,001, m = 16: 159 us, 128 rows 176; 45,001: 527 and 523; 60,000: 921 and 873
+            if (nc > 45056) row(rqa::k_rp_mx_row<128, 1024>, rqa::rp_blocks<128, 1024>(nc));
             else row(rqa::k_rp_mx_row<64, 1024>, rqa::rp_blocks<64, 1024>(nc));
             break;
     }
@@ -1703,8 +1722,9 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
             rqa::Bounds<float, 4> Bf;
             for (int t = 0; t < 4; t++) Bf.s[t] = (float)b;
             if (sym) {
-                prof_begin("k_rp_mx_sq", st);
-                rp_launch_mx(rp_shape(nc, d_out, emb, emb <= 16), (const float *)dx, nc, tau, emb, (float)b,
+                const int shape = rp_shape(nc, d_out, emb, emb <= 16);
+                prof_begin(shape == RP_SMALL || shape == RP_ROWS ? "k_rp_mx_row" : "k_rp_mx_sq", st);
+                rp_launch_mx(shape, (const float *)dx, nc, tau, emb, (float)b,
                              mx_params(Bf.s, 1, emb, rqa::NBX_LAM, rqa::RP_EXTRA_U), (char *)d_out, st);
             } else {
                 const rqa::MxParams MP = mx_params(Bf.s, 1, emb, rqa::NBX_LAM);
@@ -1725,13 +1745,10 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
         }
     }
     if constexpr (sizeof(O) == 1) {
-        // between 2,048 and 3,072 with many dimensions a launch is one wave's sums
-        // long, and the way through LDS only adds to them (2,500, m = 32: 28.6 us a
-        // call, k_rp 26.1; m = 8: 16.4 and 15.1)
-        if (sym && !(nc > 2048 && nc <= 3072 && emb >= 8)) {
-            const int ops = (dist == 1 ? 3 : 2) * emb * (sizeof(F) == 8 ? 2 : 1);
-            const int shape = rp_shape(nc, d_out, emb, ops <= 15);
-            prof_begin("k_rp_sq", st);
+        if (sym && !rp_direct<F>(nc, d_out, emb, dist)) {
+            const int64_t ops = (int64_t)(dist == 1 ? 3 : 4) * emb * (sizeof(F) == 8 ? 2 : 1);
+            const int shape = rp_shape(nc, d_out, emb, ops <= 16);
+            prof_begin(shape == RP_SMALL || shape == RP_ROWS ? "k_rp_row" : "k_rp_sq", st);
             if (dist == 1) rp_launch_exact<F, 1>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
             else rp_launch_exact<F, 2>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
             prof_end(st);
