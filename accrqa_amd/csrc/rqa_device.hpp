@@ -2358,8 +2358,16 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(false) void k_rp_mx(const float *__r
 // Against s~ - B of the table form, n_j - B and the sum round once more:
 // at most 2u (n_i + n_j + B) with u = 2^-24, and where B > 4 (n_i + n_j), so
 // B > 2 s, |d| exceeds that and E_ij by far; the host adds RP_EXTRA_U = 12 u
-// to the coefficient cE for B <= 4 (n_i + n_j).  Non-finite or huge norms
-// make E_max infinite: every pair is then decided exactly.
+// to the coefficient cE for B <= 4 (n_i + n_j).
+//
+// Non-finite or huge norms make E_max infinite, which only takes every tile to
+// its elements' own E_ij; the samples then enter unscaled (mx_scale's e = 0).
+// A pair of finite norms whose samples stay below 65,520 keeps the Gram's sign
+// where |d| > E_ij: the bound's terms need fp16(a) finite, not |a| < 2^14, and
+// what is small beside 1 is covered by the additive m 2^-25.  A sample past that
+// has h = +-inf and l = -+inf, so l.h' and h.h' meet as opposite infinities (or
+// inf.0), the sum is NaN, and so is d of a NaN sample or an infinite norm: all
+// of those fail |d| > E_ij and are summed in exact order.
 //
 // Wave w takes the rows 64w .. 64w+63 in two 32-row tiles, each against the
 // square's column tiles two at a time.  A lane's 16 signs of a tile go into
@@ -2368,7 +2376,8 @@ __global__ __launch_bounds__(WG) RQA_WPE_MX(false) void k_rp_mx(const float *__r
 // lane with all 32 rows of one column.
 //
 // About 4 lane-operations an element plus the matrix cores, against about 12
-// with the byte table: N_c = 65,536, m = 16: 1.45 -> 0.93 ms (4.6 TB/s).
+// with the byte table: N_c = 65,536, m = 16: 1.45 -> 0.86 ms (5.0 TB/s); m = 32:
+// 1.66 -> 0.89.
 constexpr int RP_EXTRA_U = 12;
 
 template <int S>
@@ -2378,10 +2387,106 @@ struct RpWin {
     float nr[S], nj[S];                      // norms of the rows and columns
 };
 
-template <int S>
-__global__ __launch_bounds__(S) __attribute__((amdgpu_waves_per_eu(4))) void k_rp_mx_sq(const float *__restrict__ x, const float *__restrict__ nrm,
-                                                const unsigned int *__restrict__ nmax_bits, int64_t nc, int tau,
-                                                int m, float bound, MxParams P, char *__restrict__ out) {
+// Gram tiles of one 32-row tile of a plot's window against 32-column tiles,
+// h.l and l.h of every chunk of 16 dimensions, then h.h of every chunk (the
+// order the bound on the adds is taken in); ROWS_A: element = row, lane =
+// column, else the other way round.  NCH = 1, 2: that many chunks, the row
+// operands and the window offsets kept in registers for all column tiles (the
+// windows read again for every tile and product, offsets and all: N_c = 28,000,
+// m = 32, 400 us a call, 258 so; 65,536: 1.75 ms and 0.89); 3: any m, both
+// windows read twice a tile (16,000, m = 48: 163 us with an offset computed per
+// read, 121 so).  The row operands of dimensions past
+// m are 0; what the column operands hold there gives a product of 0, or NaN
+// where it is not finite, which only sends the pair to the exact sum.
+template <int NCH, bool ROWS_A>
+struct RpGram {
+    static constexpr uint32_t SH = 0x05040100u, SL = 0x07060302u;
+    static constexpr int NK = NCH <= 2 ? NCH : 1;
+    int col, h, m, tau;
+    int o[NK][8];            // window offset of dimension 16c + 8h + t
+    halfx8 rh[NK], rl[NK];   // row operands (NCH <= 2)
+
+    __device__ __forceinline__ int offs(int k) const { return col + (k < m ? k * tau : 0); }
+    __device__ __forceinline__ RpGram(int col_, int h_, int m_, int tau_) : col(col_), h(h_), m(m_), tau(tau_) {
+#pragma unroll
+        for (int c = 0; c < NK; c++)
+#pragma unroll
+            for (int t = 0; t < 8; t++) o[c][t] = offs(16 * c + 8 * h + t);
+    }
+    static __device__ __forceinline__ floatx16 mul(halfx8 r, halfx8 c, floatx16 acc) {
+        return ROWS_A ? mfma16(r, c, acc) : mfma16(c, r, acc);
+    }
+    // The row tile whose window starts at rw.
+    __device__ __forceinline__ void rows(const uint32_t *rw) {
+        if constexpr (NCH <= 2) {
+#pragma unroll
+            for (int c = 0; c < NK; c++) {
+                uint32_t a[8];
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    const uint32_t v = rw[o[c][t]];
+                    a[t] = 16 * c + 8 * h + t < m ? v : 0u;
+                }
+                rh[c] = hl_halves<SH>(a);
+                rl[c] = hl_halves<SL>(a);
+            }
+        }
+    }
+    // Against the column tile whose window starts at cw.
+    __device__ __forceinline__ floatx16 tile(const uint32_t *rw, const uint32_t *cw) const {
+        floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        uint32_t a[8], b[8];
+        if constexpr (NCH <= 2) {
+            halfx8 bh[NK];
+#pragma unroll
+            for (int c = 0; c < NK; c++) {
+#pragma unroll
+                for (int t = 0; t < 8; t++) b[t] = cw[o[c][t]];
+                bh[c] = hl_halves<SH>(b);
+                acc = mul(rl[c], bh[c], acc);
+                acc = mul(rh[c], hl_halves<SL>(b), acc);
+            }
+#pragma unroll
+            for (int c = 0; c < NK; c++) acc = mul(rh[c], bh[c], acc);
+        } else {
+            auto load = [&](int k0) {
+                if (k0 + 16 <= m) {
+#pragma unroll
+                    for (int t = 0; t < 8; t++) {
+                        a[t] = rw[k0 * tau + o[0][t]];
+                        b[t] = cw[k0 * tau + o[0][t]];
+                    }
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 8; t++) {
+                        const int k = k0 + 8 * h + t, q = offs(k);
+                        a[t] = k < m ? rw[q] : 0u;
+                        b[t] = cw[q];
+                    }
+                }
+            };
+            for (int k0 = 0; k0 < m; k0 += 16) {
+                load(k0);
+                acc = mul(hl_halves<SL>(a), hl_halves<SH>(b), acc);
+                acc = mul(hl_halves<SH>(a), hl_halves<SL>(b), acc);
+            }
+            for (int k0 = 0; k0 < m; k0 += 16) {
+                load(k0);
+                acc = mul(hl_halves<SH>(a), hl_halves<SH>(b), acc);
+            }
+        }
+        return acc;
+    }
+};
+
+// Chunks of 16 dimensions as the kernels are instantiated.
+inline int rp_chunks(int m) { return m <= 16 ? 1 : (m <= 32 ? 2 : 3); }
+
+// Waves per SIMD: four, but three where the kept operands of two chunks would spill.
+template <int S, int NCH>
+__global__ __launch_bounds__(S) __attribute__((amdgpu_waves_per_eu(NCH == 2 ? 3 : 4))) void k_rp_mx_sq(
+    const float *__restrict__ x, const float *__restrict__ nrm, const unsigned int *__restrict__ nmax_bits, int64_t nc,
+    int tau, int m, float bound, MxParams P, char *__restrict__ out) {
     __shared__ RpBits<S> M;
     __shared__ __align__(16) RpWin<S> Wn;
     int64_t g, J;
@@ -2409,10 +2514,7 @@ __global__ __launch_bounds__(S) __attribute__((amdgpu_waves_per_eu(4))) void k_r
     }
     __syncthreads();
 
-    constexpr uint32_t SH = 0x05040100u, SL = 0x07060302u;
-    // window offset of dimension k0 + 8h + t; the row operands of dimensions
-    // past m are 0, so the column operands there may be anything finite
-    auto offs = [&](int k0, int t) { const int k = k0 + 8 * h + t; return col + (k < m ? k * tau : 0); };
+    RpGram<NCH, true> G(col, h, m, tau);
     for (int r = 0; r < 2; r++) {
         const int rb = wave * WAVE + BLK * r;
         if (r0 + rb >= nc) {   // no such rows: their words are 0
@@ -2425,46 +2527,7 @@ __global__ __launch_bounds__(S) __attribute__((amdgpu_waves_per_eu(4))) void k_r
         }
         float ni[16];
         tile_row_norms(Wn.nr, rb, h, ni);
-        uint32_t a[8], b[8];
-        auto load_a = [&](int k0) {
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                const uint32_t v = Wn.rw[rb + offs(k0, t)];
-                a[t] = k0 + 8 * h + t < m ? v : 0u;
-            }
-        };
-        load_a(0);
-        const halfx8 ah = hl_halves<SH>(a), al = hl_halves<SL>(a);
-        int o0[8];
-#pragma unroll
-        for (int t = 0; t < 8; t++) o0[t] = offs(0, t);
-        auto gram = [&](int cb) {
-            floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if (m <= 16) {
-#pragma unroll
-                for (int t = 0; t < 8; t++) b[t] = Wn.cw[cb + o0[t]];
-                const halfx8 bh = hl_halves<SH>(b);
-                acc = mfma16(al, bh, acc);
-                acc = mfma16(ah, hl_halves<SL>(b), acc);
-                return mfma16(ah, bh, acc);
-            }
-            // small products of every chunk, then h.h chunk by chunk
-            auto load = [&](int k0) {
-                load_a(k0);
-#pragma unroll
-                for (int t = 0; t < 8; t++) b[t] = Wn.cw[cb + offs(k0, t)];
-            };
-            for (int k0 = 0; k0 < m; k0 += 16) {
-                load(k0);
-                acc = mfma16(hl_halves<SL>(a), hl_halves<SH>(b), acc);
-                acc = mfma16(hl_halves<SH>(a), hl_halves<SL>(b), acc);
-            }
-            for (int k0 = 0; k0 < m; k0 += 16) {
-                load(k0);
-                acc = mfma16(hl_halves<SH>(a), hl_halves<SH>(b), acc);
-            }
-            return acc;
-        };
+        G.rows(Wn.rw + rb);
         // signs of a tile's 16 elements as a word: row 8q + 4h + c at bit 8q + c
         auto decide = [&](floatx16 acc, int cb) -> uint32_t {
             const float nj = Wn.nj[cb + col], njb = nj - bound;
@@ -2503,7 +2566,7 @@ __global__ __launch_bounds__(S) __attribute__((amdgpu_waves_per_eu(4))) void k_r
         };
 #pragma unroll 1
         for (int p = 0; p < S / BLK; p += 2) {
-            const floatx16 g0 = gram(BLK * p), g1 = gram(BLK * p + BLK);
+            const floatx16 g0 = G.tile(Wn.rw + rb, Wn.cw + BLK * p), g1 = G.tile(Wn.rw + rb, Wn.cw + BLK * p + BLK);
             const uint32_t w0 = decide(g0, BLK * p), w1 = decide(g1, BLK * p + BLK);
             // half 0: column tile p, half 1: column tile p + 1; words of rows 8q + c, then 8q + 4 + c
             const auto sw = __builtin_amdgcn_permlane32_swap(w0, w1, false, false);
@@ -2527,8 +2590,8 @@ struct RpRowWin {
     float nr[R], nj[C], njb[C];                    // norms of the rows, of the columns, columns less the bound
 };
 
-template <int R, int C>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_rp_mx_row(
+template <int R, int C, int NCH>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(NCH == 2 ? 3 : 4))) void k_rp_mx_row(
     const float *__restrict__ x, const float *__restrict__ nrm, const unsigned int *__restrict__ nmax_bits, int64_t nc,
     int tau, int m, float bound, MxParams P, char *__restrict__ out) {
     __shared__ RpRows<R, C> M;
@@ -2558,55 +2621,13 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_
     if (threadIdx.x < R) Wn.nr[threadIdx.x] = r0 + threadIdx.x < nc ? nrm[r0 + threadIdx.x] : 0.f;
     __syncthreads();
 
-    constexpr uint32_t SH = 0x05040100u, SL = 0x07060302u;
-    // window offset of dimension k0 + 8h + t; the row operands of dimensions
-    // past m are 0, so the column operands there may be anything finite
-    auto offs = [&](int k0, int t) { const int k = k0 + 8 * h + t; return col + (k < m ? k * tau : 0); };
-    int o0[8];
-#pragma unroll
-    for (int t = 0; t < 8; t++) o0[t] = offs(0, t);
+    RpGram<NCH, false> G(col, h, m, tau);
 #pragma unroll 1
     for (int r = 0; r < R / BLK; r++) {
         const int rb = BLK * r;
         if (r0 + rb >= nc) break;
-        uint32_t a[8], b[8];
-        auto load_b = [&](int k0) {
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                const uint32_t v = Wn.rw[rb + offs(k0, t)];
-                b[t] = k0 + 8 * h + t < m ? v : 0u;
-            }
-        };
-        load_b(0);
-        const halfx8 bh = hl_halves<SH>(b), bl = hl_halves<SL>(b);
+        G.rows(Wn.rw + rb);
         const float ni = Wn.nr[rb + col];
-        auto gram = [&](int cb) {
-            floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if (m <= 16) {
-#pragma unroll
-                for (int t = 0; t < 8; t++) a[t] = Wn.cw[cb + o0[t]];
-                const halfx8 ah = hl_halves<SH>(a);
-                acc = mfma16(hl_halves<SL>(a), bh, acc);
-                acc = mfma16(ah, bl, acc);
-                return mfma16(ah, bh, acc);
-            }
-            // small products of every chunk, then h.h chunk by chunk
-            auto load = [&](int k0) {
-                load_b(k0);
-#pragma unroll
-                for (int t = 0; t < 8; t++) a[t] = Wn.cw[cb + offs(k0, t)];
-            };
-            for (int k0 = 0; k0 < m; k0 += 16) {
-                load(k0);
-                acc = mfma16(hl_halves<SL>(a), hl_halves<SH>(b), acc);
-                acc = mfma16(hl_halves<SH>(a), hl_halves<SL>(b), acc);
-            }
-            for (int k0 = 0; k0 < m; k0 += 16) {
-                load(k0);
-                acc = mfma16(hl_halves<SH>(a), hl_halves<SH>(b), acc);
-            }
-            return acc;
-        };
         // signs of a tile's 16 elements as a word: column 8q + 4h + c at bit 8q + c
         auto decide = [&](floatx16 acc, int cb) -> uint32_t {
             float nb[16];
@@ -2647,7 +2668,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll 1
         for (int p = 2 * wave; p < C / BLK; p += 2 * WAVES) {
             if (c0 + BLK * p >= nc) break;
-            const floatx16 g0 = gram(BLK * p), g1 = gram(BLK * p + BLK);
+            const floatx16 g0 = G.tile(Wn.rw + rb, Wn.cw + BLK * p), g1 = G.tile(Wn.rw + rb, Wn.cw + BLK * p + BLK);
             const uint32_t w0 = decide(g0, BLK * p), w1 = decide(g1, BLK * p + BLK);
             // half 0: column tile p, half 1: column tile p + 1; columns 8q + c, then 8q + 4 + c
             const auto sw = __builtin_amdgcn_permlane32_swap(w0, w1, false, false);

@@ -1611,23 +1611,30 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
 //          dimension: 11,000: 31, 64-squares 37, k_rp4 33)
 //   SQ64   64-squares, mirrored: while the plot fits the 256 MB last-level
 //          cache its short mirrored runs merge there (12,000, m = 3: 35,
-//          256-squares 43, rows 45; 20,000: 146, 134, 105)
+//          256-squares 43, rows 45; 20,000: 146, 134, 105).  More than 32
+//          dimensions are bound by the windows' reads, which its small squares
+//          overlap best at any size (16,000, m = 48: 121, 256-squares 135;
+//          65,536: 1,720 and 1,660; 40,001: 716 and 790)
 //   SQ256  256-squares, mirrored: large plots whose rows start on 128-byte
 //          lines, so every run is whole lines (65,536: 880, rows 1,030)
 //   ROWS   blocks of 64 (MFMA, large: 128) x 1,024, every element: other large
 //          plots, where the runs' partial lines cost more than the second
 //          half's decisions, as long as the decisions are cheap: the MFMA form
-//          in one chunk of 16 dimensions (28,000, m = 16: 216, 256-squares 287;
-//          30,011, m = 32: 617 and 490) or at most 16 VALU operations an element
+//          with up to 32 dimensions (28,000, m = 16: 216, 256-squares 287;
+//          m = 32: 258 and 285) or at most 16 VALU operations an element
 //          (30,011, m = 3: 226 and 356; maximal, m = 4: 302 and 361, m = 5:
 //          358 and 347; fp64, m = 2: 263 and 351, m = 3 at 40,000: 556 and
 //          477); with one dimension from 13,312 on (14,000: 41.5, SMALL 43,
 //          64-squares 46; 32,768: 174, 256-squares 221)
+// The MFMA form's second chunk makes the decisions of 17 to 32 dimensions dear
+// enough for the larger squares from 12,288 on (12,000: 55 and 53; 16,000: 83
+// and 71).
 enum { RP_SMALL, RP_SQ64, RP_SQ256, RP_ROWS };
-int rp_shape(int64_t nc, const void *out, int m, bool cheap) {
+int rp_shape(int64_t nc, const void *out, int m, bool mx, bool cheap) {
     if (m == 1) return nc <= 13312 ? RP_SMALL : RP_ROWS;
     if (nc <= 3072 || (nc <= 4096 && m <= 3)) return RP_SMALL;
-    if (nc <= 16384) return RP_SQ64;
+    if (mx && m > 32) return RP_SQ64;
+    if (nc <= (mx && m > 16 ? 12288 : 16384)) return RP_SQ64;
     if (nc % 128 == 0 && (uintptr_t)out % 128 == 0) return RP_SQ256;
     return cheap ? RP_ROWS : RP_SQ256;
 }
@@ -1679,14 +1686,23 @@ void rp_launch_mx(int shape, const float *dx, int64_t nc, int tau, int m, float 
     auto row = [&](auto kern, int64_t blocks) {
         hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(rqa::WG), 0, st, dx, nrm, nmax, nc, tau, m, b, P, out);
     };
-    switch (shape) {
-        case RP_SMALL: row(rqa::k_rp_mx_row<32, 256>, rqa::rp_blocks<32, 256>(nc)); break;
-        case RP_SQ64: sq(rqa::k_rp_mx_sq<64>, 64); break;
-        case RP_SQ256: sq(rqa::k_rp_mx_sq<256>, 256); break;
-        default:   // 24,001, m = 16: 159 us, 128 rows 176; 45,001: 527 and 523; 60,000: 921 and 873
-            if (nc > 45056) row(rqa::k_rp_mx_row<128, 1024>, rqa::rp_blocks<128, 1024>(nc));
-            else row(rqa::k_rp_mx_row<64, 1024>, rqa::rp_blocks<64, 1024>(nc));
-            break;
+    auto sized = [&](auto nch) {
+        constexpr int N = decltype(nch)::value;
+        constexpr int NR = N <= 2 ? N : 2;   // rows: up to two chunks (rp_shape)
+        switch (shape) {
+            case RP_SMALL: row(rqa::k_rp_mx_row<32, 256, N>, rqa::rp_blocks<32, 256>(nc)); break;
+            case RP_SQ64: sq(rqa::k_rp_mx_sq<64, N>, 64); break;
+            case RP_ROWS:   // 24,001, m = 16: 159 us, 128 rows 176; 45,001: 527 and 523; 60,000: 921 and 873
+                if (nc > 45056) row(rqa::k_rp_mx_row<128, 1024, NR>, rqa::rp_blocks<128, 1024>(nc));
+                else row(rqa::k_rp_mx_row<64, 1024, NR>, rqa::rp_blocks<64, 1024>(nc));
+                break;
+            default: sq(rqa::k_rp_mx_sq<256, NR>, 256); break;   // the same
+        }
+    };
+    switch (rqa::rp_chunks(m)) {
+        case 1: sized(std::integral_constant<int, 1>()); break;
+        case 2: sized(std::integral_constant<int, 2>()); break;
+        default: sized(std::integral_constant<int, 3>()); break;
     }
 }
 
@@ -1722,7 +1738,7 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
             rqa::Bounds<float, 4> Bf;
             for (int t = 0; t < 4; t++) Bf.s[t] = (float)b;
             if (sym) {
-                const int shape = rp_shape(nc, d_out, emb, emb <= 16);
+                const int shape = rp_shape(nc, d_out, emb, true, emb <= 32);
                 prof_begin(shape == RP_SMALL || shape == RP_ROWS ? "k_rp_mx_row" : "k_rp_mx_sq", st);
                 rp_launch_mx(shape, (const float *)dx, nc, tau, emb, (float)b,
                              mx_params(Bf.s, 1, emb, rqa::NBX_LAM, rqa::RP_EXTRA_U), (char *)d_out, st);
@@ -1747,7 +1763,7 @@ int rp_run(const F *dx, size_t n, int tau, int emb, F thr, int dist, O *d_out, h
     if constexpr (sizeof(O) == 1) {
         if (sym && !rp_direct<F>(nc, d_out, emb, dist)) {
             const int64_t ops = (int64_t)(dist == 1 ? 3 : 4) * emb * (sizeof(F) == 8 ? 2 : 1);
-            const int shape = rp_shape(nc, d_out, emb, ops <= 16);
+            const int shape = rp_shape(nc, d_out, emb, false, ops <= 16);
             prof_begin(shape == RP_SMALL || shape == RP_ROWS ? "k_rp_row" : "k_rp_sq", st);
             if (dist == 1) rp_launch_exact<F, 1>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
             else rp_launch_exact<F, 2>(shape, dx, nc, tau, emb, b, (char *)d_out, st);
