@@ -161,7 +161,9 @@ SPLIT_AUTO, SPLIT_NEVER = 0, 1
 def set_split(mode):
     """LAM/DET work split: SPLIT_AUTO (rank the upper triangle once, keep the
     tiles and read the rest of LAM and all of DET from them, when they fit in
-    device memory) or SPLIT_NEVER (LAM ranks full columns, DET its own pairs).
+    device memory; DET alone in the MFMA form as well) or SPLIT_NEVER (LAM ranks
+    full columns, DET its own pairs).  The tiles' memory (N_c^2/2 bytes) is kept
+    for later calls.
     Results are identical; only speed and memory differ."""
     e = load().accrqa_amd_set_split(int(mode))
     if e:

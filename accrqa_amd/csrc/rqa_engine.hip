@@ -164,6 +164,18 @@ int ensure(DevBuf &b, size_t bytes) {
     return E_OK;
 }
 
+// The same for a buffer the call can do without: got is false, and no error is
+// left behind, where the memory is not there.
+int try_ensure(DevBuf &b, size_t bytes, bool &got) {
+    const std::string before = g_last_error;
+    const int e = ensure(b, bytes);
+    got = e == E_OK;
+    if (e != E_NO_MEMORY) return e;
+    (void)hipGetLastError();   // or the next launch's check would report it
+    g_last_error = before;
+    return E_OK;
+}
+
 // A small read-only device table uploaded only when its bytes change: the
 // (tau, emb) blocks of one call, and the calls of a loop over series, reuse
 // the same threshold permutation, l_min list and bucket tables.  Kept per
@@ -1164,12 +1176,13 @@ int launch_group(const F *dx, int64_t nc, int tau, int m, const F *bounds, int n
                 // the tile store (when it fits) and scan the tiles, instead of
                 // three Gram tiles per two of pairs and a scan at three waves
                 // per SIMD (k_det_mx): N = 100,003, m = 32, 16 thresholds,
-                // 9.0 -> 6.4 ms.
-                if (!tiles && !want_lam && g_split == 0 && use_mfma<F>(1, m, tau) && tile_store_fits(nc)) {
+                // 9.0 -> 6.4 ms.  Without the memory for it, as before.
+                bool store = !tiles && !want_lam && g_split == 0 && use_mfma<F>(1, m, tau) && tile_store_fits(nc);
+                if (store && (e = try_ensure(c.tiles, tile_store_bytes(nc), store))) return e;
+                if (store) {
                     rqa::Bounds<float, TG> Bf;
                     for (int t = 0; t < TG; t++) Bf.s[t] = (float)B.s[t];
                     const rqa::MxParams MP = mx_params(Bf.s, nt, m, rqa::NBX_LAM, sizeof(F) == 8 ? 4 : 0);
-                    if ((e = ensure(c.tiles, tile_store_bytes(nc)))) return e;
                     if ((e = ensure(c.lut8, rqa::NBX_LAM))) return e;
                     tiles = (uint8_t *)c.tiles.p;
                     hipLaunchKernelGGL((rqa::k_mx_lut<TG>), dim3((MP.nb + 255) / 256), dim3(256), 0, st, Bf, nt, MP,

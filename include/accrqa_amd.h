@@ -205,12 +205,14 @@ int accrqa_amd_rp_device_f64(const double *d_input, size_t data_size, int tau, i
 int accrqa_amd_set_form(int form);
 
 /* LAM/DET work split (no counterpart in the reference).  0 = automatic: when
- * LAM is computed and N_c^2/2 bytes of rank tiles fit in under half of the
- * free device memory, the column pass ranks only the upper triangle and the
- * diagonal tiles and keeps them; the rest of each LAM column (row runs, R
- * being symmetric) and all of DET are then read from the tiles.  1 = never:
- * LAM ranks full columns and DET recomputes its pairs.  Results are identical
- * either way.  Process-wide; returns 0, or 2 for an unknown mode. */
+ * LAM is computed, or DET alone in the MFMA form, and N_c^2/2 bytes of rank
+ * tiles fit in under half of the free device memory, one pass ranks only the
+ * upper triangle and the diagonal tiles and keeps them; the rest of each LAM
+ * column (row runs, R being symmetric) and all of DET are then read from the
+ * tiles.  The tiles' memory stays the library's for later calls (34 GB after
+ * N_c = 262,144); DET alone does without it where it cannot be allocated.
+ * 1 = never: LAM ranks full columns and DET recomputes its pairs.  Results
+ * are identical either way.  Process-wide; returns 0, or 2 for an unknown mode. */
 int accrqa_amd_set_split(int mode);
 
 /* Slab form of the split (no counterpart in the reference).  When the tile
