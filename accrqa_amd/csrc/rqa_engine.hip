@@ -65,19 +65,32 @@ struct CallOrder {
 
 // Work-item tables kept for the last few (nc, seg_len): a call with several
 // (tau, m) blocks, or a loop over many series of a few lengths, alternates
-// between them, and rebuilding costs a host pass and five uploads.  Least
-// recently used entry replaced, its new tables uploaded in stream order.
+// between them, and rebuilding costs a host pass and its uploads.  Least
+// recently used entry replaced, its new tables uploaded in stream order.  RR
+// asked alone has segments of its own (seg_len_rr), so its table has a cache of
+// its own: RR, DET and LAM asked in turn over a grid keep theirs (nine blocks of
+// N = 4,001, five lengths N_c: 1.98 ms a round with one cache for all, 1.54 so).
+constexpr int NITEMSETS = 8;
+struct ItemTable {
+    DevBuf buf;
+    int64_t n = 0;
+};
 struct ItemSet {
     int64_t nc = -1;
     int L = -1;
     bool slab = false;   // lamv, lamh and dets sorted slab by slab (slab form)
     uint64_t used = 0;
-    DevBuf rr, det, dets, lamv, lamh;
-    int64_t n_rr = 0, n_det = 0, n_dets = 0, n_lamv = 0, n_lamh = 0;
+    ItemTable det, dets, lamv, lamh;
     std::vector<int64_t> off_lamv, off_lamh, off_dets;   // slab form: first item of each slab (+ end)
 };
-constexpr int NITEMSETS = 8;
+struct RrItemSet {
+    int64_t nc = -1;
+    int L = -1;
+    uint64_t used = 0;
+    ItemTable rr;
+};
 ItemSet g_items[NITEMSETS];
+RrItemSet g_rr_items[NITEMSETS];
 uint64_t g_items_clock = 0;
 
 // Euclidean distance form: 0 = automatic (MFMA Gram + exact recheck for fp32
@@ -276,9 +289,13 @@ int init_ctx() {
                 *b = DevBuf();
             }
             for (ItemSet &s : g_items) {
-                for (DevBuf *b : {&s.rr, &s.det, &s.dets, &s.lamv, &s.lamh})
-                    if (b->p) (void)hipFree(b->p);
+                for (ItemTable *t : {&s.det, &s.dets, &s.lamv, &s.lamh})
+                    if (t->buf.p) (void)hipFree(t->buf.p);
                 s = ItemSet();
+            }
+            for (RrItemSet &s : g_rr_items) {
+                if (s.rr.buf.p) (void)hipFree(s.rr.buf.p);
+                s = RrItemSet();
             }
             g_ctx.items_rr = g_ctx.items_det = g_ctx.items_dets = g_ctx.items_lamv = g_ctx.items_lamh = DevBuf();
             if (g_order.done) (void)hipEventSynchronize(g_order.done);
@@ -640,20 +657,69 @@ int finish_group(bool lam, bool det, bool split, int64_t nc, int nt, int L, int 
 //   k_det: (strip b, step segment q) over steps 0 .. N_c - (1 + 64b) - 1
 void select_items(const ItemSet &s) {
     Ctx &c = g_ctx;
-    c.items_rr = s.rr;
-    c.items_det = s.det;
-    c.items_dets = s.dets;
-    c.items_lamv = s.lamv;
-    c.items_lamh = s.lamh;
-    c.n_items_rr = s.n_rr;
-    c.n_items_det = s.n_det;
-    c.n_items_dets = s.n_dets;
-    c.n_items_lamv = s.n_lamv;
-    c.n_items_lamh = s.n_lamh;
+    c.items_det = s.det.buf;
+    c.items_dets = s.dets.buf;
+    c.items_lamv = s.lamv.buf;
+    c.items_lamh = s.lamh.buf;
+    c.n_items_det = s.det.n;
+    c.n_items_dets = s.dets.n;
+    c.n_items_lamv = s.lamv.n;
+    c.n_items_lamh = s.lamh.n;
     c.nslabs = s.slab ? (int)s.off_lamv.size() - 1 : 0;
     c.slab_lamv = s.slab ? s.off_lamv.data() : nullptr;
     c.slab_lamh = s.slab ? s.off_lamh.data() : nullptr;
     c.slab_dets = s.slab ? s.off_dets.data() : nullptr;
+}
+
+// (steps, item) lists; each table is sorted by decreasing size so that the
+// persistent waves take the long items first.
+typedef std::vector<std::pair<int64_t, int2>> ItemList;
+void add_segments(ItemList &v, int64_t b, int64_t len, int L) {
+    for (int64_t q = 0; q * L < len; q++) v.push_back({std::min<int64_t>(L, len - q * L), make_int2((int)b, (int)q)});
+}
+
+int upload_items(const ItemList &v, ItemTable &t, hipStream_t st) {
+    std::vector<int2> it(v.size());
+    for (size_t i = 0; i < v.size(); i++) it[i] = v[i].second;
+    int e;
+    if ((e = ensure(t.buf, std::max<size_t>(it.size(), 1) * sizeof(int2)))) return e;
+    // ordered on the call's stream: after the queued kernels that may
+    // still read the entry's previous tables, before those of this block
+    if ((e = stage_upload(t.buf.p, it.data(), it.size() * sizeof(int2), st))) return e;
+    t.n = (int64_t)it.size();
+    return E_OK;
+}
+
+void sort_by_size(ItemList &v) {
+    std::stable_sort(v.begin(), v.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
+}
+
+// The table of RR without LAM: rows that can be <= a column of the band.
+int build_rr_items(int64_t nc, int L, hipStream_t st) {
+    RrItemSet *slot = &g_rr_items[0];
+    for (RrItemSet &s : g_rr_items) {
+        if (s.nc == nc && s.L == L) {
+            slot = &s;
+            break;
+        }
+        if (s.used < slot->used) slot = &s;
+    }
+    RrItemSet &S = *slot;
+    if (S.nc != nc || S.L != L) {
+        ItemList rr;
+        const int64_t nb = (nc + rqa::WAVE - 1) / rqa::WAVE;
+        for (int64_t b = 0; b < nb; b++) add_segments(rr, b, std::min<int64_t>((b + 1) * rqa::WAVE, nc), L);
+        sort_by_size(rr);
+        S.nc = -1;
+        const int e = upload_items(rr, S.rr, st);
+        if (e) return e;
+        S.nc = nc;
+        S.L = L;
+    }
+    S.used = ++g_items_clock;
+    g_ctx.items_rr = S.rr.buf;
+    g_ctx.n_items_rr = S.rr.n;
+    return E_OK;
 }
 
 // Work-item tables of segment length L.  Slab form: the split passes' tables
@@ -672,61 +738,44 @@ int build_items(int64_t nc, int L, bool slab, hipStream_t st) {
         if (s.used < slot->used) slot = &s;
     }
     ItemSet &S = *slot;
-    // (item, steps) lists; each table is sorted by decreasing size so that the
-    // persistent waves take the long items first
-    std::vector<std::pair<int64_t, int2>> rr, det, dets, lamv, lamh;
+    ItemList det, dets, lamv, lamh;
     const int64_t nb = (nc + rqa::WAVE - 1) / rqa::WAVE;
-    auto seg = [&](std::vector<std::pair<int64_t, int2>> &v, int64_t b, int64_t len) {
-        for (int64_t q = 0; q * L < len; q++)
-            v.push_back({std::min<int64_t>(L, len - q * L), make_int2((int)b, (int)q)});
-    };
     for (int64_t b = 0; b < nb; b++) {
         const int64_t V = std::min<int64_t>((b + 1) * rqa::WAVE, nc);
-        seg(rr, b, V);          // rows that can be <= a column of the band
-        seg(lamv, b, V);        // split LAM: rows [0, V) of the band's columns
-        seg(lamh, b, nc - V);   // split LAM: columns [V, nc) of the band's rows
+        add_segments(lamv, b, V, L);        // split LAM: rows [0, V) of the band's columns
+        add_segments(lamh, b, nc - V, L);   // split LAM: columns [V, nc) of the band's rows
     }
     const int64_t nstrips = (nc - 1 + rqa::WAVE - 1) / rqa::WAVE;
-    for (int64_t b = 0; b < nstrips; b++) seg(det, b, nc - (1 + b * rqa::WAVE));
+    for (int64_t b = 0; b < nstrips; b++) add_segments(det, b, nc - (1 + b * rqa::WAVE), L);
     // k_det_scan: groups of WAVES strips, segments of the group's longest strip
     const int64_t ngroups = (nc - 1 + rqa::WG - 1) / rqa::WG;
-    for (int64_t g = 0; g < ngroups; g++) seg(dets, g, nc - (1 + g * rqa::WG));
-    int e;
+    for (int64_t g = 0; g < ngroups; g++) add_segments(dets, g, nc - (1 + g * rqa::WG), L);
     const int64_t nsl = (nc + L - 1) / L;
-    // slab of an item: -1 = not a slab-ordered table
-    auto upload = [&](std::vector<std::pair<int64_t, int2>> &v, DevBuf &buf, int64_t &n, int kind = -1,
-                      std::vector<int64_t> *off = nullptr) -> int {
-        auto slab_of = [&](const int2 &x) -> int64_t {
-            return kind == 1 ? ((int64_t)x.x * rqa::WAVE) / L : (int64_t)x.y;   // lamh: the row band's slab
-        };
-        if (off) {
-            std::stable_sort(v.begin(), v.end(), [&](const auto &x, const auto &y) {
-                const int64_t sx = slab_of(x.second), sy = slab_of(y.second);
-                return sx != sy ? sx < sy : x.first > y.first;
-            });
-            off->assign((size_t)nsl + 1, 0);
-            for (const auto &x : v) (*off)[(size_t)slab_of(x.second) + 1]++;
-            for (int64_t k = 0; k < nsl; k++) (*off)[(size_t)k + 1] += (*off)[(size_t)k];
-        } else {
-            std::stable_sort(v.begin(), v.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
-        }
-        std::vector<int2> it(v.size());
-        for (size_t i = 0; i < v.size(); i++) it[i] = v[i].second;
-        int e2;
-        if ((e2 = ensure(buf, std::max<size_t>(it.size(), 1) * sizeof(int2)))) return e2;
-        // ordered on the call's stream: after the queued kernels that may
-        // still read the entry's previous tables, before those of this block
-        if ((e2 = stage_upload(buf.p, it.data(), it.size() * sizeof(int2), st))) return e2;
-        n = (int64_t)it.size();
-        return E_OK;
+    // by slab, then by size; lamh: the row band's slab, else the segment's number
+    auto by_slab = [&](ItemList &v, bool band, std::vector<int64_t> &off) {
+        auto slab_of = [&](const int2 &x) -> int64_t { return band ? ((int64_t)x.x * rqa::WAVE) / L : (int64_t)x.y; };
+        std::stable_sort(v.begin(), v.end(), [&](const auto &x, const auto &y) {
+            const int64_t sx = slab_of(x.second), sy = slab_of(y.second);
+            return sx != sy ? sx < sy : x.first > y.first;
+        });
+        off.assign((size_t)nsl + 1, 0);
+        for (const auto &x : v) off[(size_t)slab_of(x.second) + 1]++;
+        for (int64_t k = 0; k < nsl; k++) off[(size_t)k + 1] += off[(size_t)k];
     };
     S.nc = -1;
-    if ((e = upload(rr, S.rr, S.n_rr))) return e;
-    if ((e = upload(det, S.det, S.n_det))) return e;
-    if ((e = upload(dets, S.dets, S.n_dets, 0, slab ? &S.off_dets : nullptr))) return e;
-    if ((e = upload(lamv, S.lamv, S.n_lamv, 0, slab ? &S.off_lamv : nullptr))) return e;
-    if ((e = upload(lamh, S.lamh, S.n_lamh, 1, slab ? &S.off_lamh : nullptr))) return e;
-    if (!slab) S.off_dets.clear(), S.off_lamv.clear(), S.off_lamh.clear();
+    sort_by_size(det);
+    if (slab) {
+        by_slab(dets, false, S.off_dets);
+        by_slab(lamv, false, S.off_lamv);
+        by_slab(lamh, true, S.off_lamh);
+    } else {
+        for (ItemList *v : {&dets, &lamv, &lamh}) sort_by_size(*v);
+        S.off_dets.clear(), S.off_lamv.clear(), S.off_lamh.clear();
+    }
+    int e;
+    if ((e = upload_items(det, S.det, st)) || (e = upload_items(dets, S.dets, st)) ||
+        (e = upload_items(lamv, S.lamv, st)) || (e = upload_items(lamh, S.lamh, st)))
+        return e;
     S.nc = nc;
     S.L = L;
     S.slab = slab;
@@ -1354,7 +1403,8 @@ int run_block(const F *dx, size_t n, int tau, int emb, const F *thr, int T, cons
             c.blk_slab = true;
         }
     }
-    if ((e = build_items(nc, c.blk_L, c.blk_slab, st))) return e;
+    if (d_rr && !d_lam && (e = build_rr_items(nc, c.blk_L, st))) return e;
+    if ((d_det || d_lam) && (e = build_items(nc, c.blk_L, c.blk_slab, st))) return e;
     if (use_mfma<F>(dist, emb, tau) && ngroups > 0) {
         if ((e = ensure(c.nrm, ((size_t)nc + 2 * rqa::WAVE) * sizeof(float)))) return e;
         if ((e = ensure(c.nmax, 256))) return e;
@@ -1582,7 +1632,7 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
     if ((e = call.err) || (e = upload_series(d_in, n, true, st))) return e;
     Ctx &c = g_ctx;
     const int64_t nc = (int64_t)n - (int64_t)(emb - 1) * tau;
-    if ((e = build_items(nc, seg_len_for(nc), false, st))) return e;
+    if ((e = build_rr_items(nc, seg_len_for(nc), st))) return e;
     if ((e = ensure(c.counts, std::max<size_t>(64, (size_t)T) * sizeof(unsigned long long)))) return e;
     unsigned long long *d_counts = (unsigned long long *)c.counts.p;
     fill_zero(d_counts, (size_t)T, st);
