@@ -1,7 +1,9 @@
 // rqa_bits.hpp -- word-level pieces of the line scan: decision words from
 // packed threshold ranks, and run extraction from a 32-step word.  Plain
 // integer code, compiled into the kernels and, unchanged, into the host unit
-// test of the line scan (tests/test_line_scan_bits.py).
+// tests of the line scan (tests/test_line_scan_run.py drives consume_word(), the
+// kernels' form; test_line_scan_bits.py and test_line_scan_word.py consume(), the
+// form it is compared with).
 //
 // Conventions.  A lane walks one sequence (a column for LAM, a diagonal for
 // DET) in blocks of 32 steps.  For each step the engine has a rank
@@ -26,10 +28,7 @@ constexpr int LCAP = 128;              // run lengths < LCAP go to the workgroup
 // a word) is positive as a signed integer and an all-ones word stands apart
 // from it.
 constexpr uint32_t PRE = 0x40000000u;
-// Spare bins after each row of an LDS run histogram: a lane adds one there for
-// a word whose carried run counts nothing (none closes, it is empty, or it
-// goes to the slow path), so that the wave's adds that count nothing spread
-// over NSPARE addresses instead of meeting on one.
+// Spare bins of consume(), for the words whose carried run counts nothing.
 constexpr int NSPARE = 16;
 
 // Position of the lowest / highest set bit (as the hardware's find-first-bit
@@ -162,7 +161,8 @@ RQA_HD void inner_runs(uint32_t mid, uint32_t nw, Inner &&inner) {
     }
 }
 
-// One 32-step word of one threshold.  nw: bit u set = step u not recurrent
+// One 32-step word of one threshold, in the form the host tests compare with
+// the kernels' (consume_word, below).  nw: bit u set = step u not recurrent
 // (bit 0 = oldest).  run: recurrent steps carried in from earlier words, with
 // PRE added while the segment's first run is open.  Counting goes through
 // three callbacks:
@@ -174,11 +174,11 @@ RQA_HD void inner_runs(uint32_t mid, uint32_t nw, Inner &&inner) {
 //   inner(len): a run strictly inside the word, 1 <= len <= 30;
 //   slow(first): the carried run when it is >= CAP long or is the segment's
 //     first run (first >= PRE: its length is first - PRE, 0 included).
-// CAP (at least 32) is the caller's LDS histogram size: LCAP for the large-N
-// kernels.  No select or compare is spent on "does a run close": for nw == 0
-// both find-first-bit results are all ones, so the saturating sum is all
-// ones (a spare bin, and negative as a signed integer, so not slow) and the
-// new carry min(run + 32, tail) is run + 32.
+// CAP (at least 32) is the caller's LDS histogram size.  No select or compare
+// is spent on "does a run close": for nw == 0 both find-first-bit results are
+// all ones, so the saturating sum is all ones (a spare bin, and negative as a
+// signed integer, so not slow) and the new carry min(run + 32, tail) is
+// run + 32.
 template <uint32_t CAP = LCAP, class First, class Inner, class Slow>
 RQA_HD void consume(uint32_t nw, uint32_t &run, uint32_t spare, First &&first_bin, Inner &&inner, Slow &&slow) {
     static_assert(CAP >= 32, "inner runs (up to 30 steps) always take the histogram");
@@ -192,12 +192,12 @@ RQA_HD void consume(uint32_t nw, uint32_t &run, uint32_t spare, First &&first_bi
     run = umin(run + 32u, tail);
 }
 
-// The same with the carried run counted only where one closes (first(len), 1
-// <= len < CAP): a compare in the place of the minimum, and no add at all from
-// the lanes that have nothing to count.  In the large-N scans' LDS histograms
-// those adds met four to eight on a spare bin, one after the other: without
-// them, 20 thresholds, N = 131,072, k_lam_hscan takes 3.7 instead of 4.2 ms and
-// k_det_scan 5.1 instead of 5.8.  take(mid) may count and clear some of the
+// The kernels' form: the carried run is counted only where one closes
+// (first(len), 1 <= len < CAP): a compare in the place of consume()'s minimum,
+// and no add at all from the lanes that have nothing to count.  In the large-N
+// scans' LDS histograms those adds met four to eight on a spare bin, one after
+// the other: without them, 20 thresholds, N = 131,072, k_lam_hscan takes 3.7
+// instead of 4.2 ms and k_det_scan 5.1 instead of 5.8.  take(mid) may count and clear some of the
 // word's inner runs (mid: their steps) before the loop reads the rest.
 template <uint32_t CAP, class First, class Take, class Inner, class Slow>
 RQA_HD void consume_word(uint32_t nw, uint32_t &run, First &&first_run, Take &&take, Inner &&inner, Slow &&slow) {

@@ -208,7 +208,7 @@ __device__ __forceinline__ void flush_hist(const uint32_t *lh, const Sink &K, in
     }
 }
 
-// The slow path of consume(): the segment's first run goes to the carry slot
+// The slow path of consume_word(): the segment's first run goes to the carry slot
 // (for the stitch), runs of LCAP or more to the private or result bins.  A
 // run longer than the sequence would be an engine bug and is dropped rather
 // than written out of bounds (the parity tests would then fail on the count).
@@ -1692,19 +1692,6 @@ __device__ __forceinline__ F exact_sqdist(const F *__restrict__ x, int64_t i, in
         }
     }
     return s;
-}
-
-// Wave-wide exclusive prefix sum of a small per-lane count.
-__device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t &total) {
-    const int lane = threadIdx.x & (WAVE - 1);
-    uint32_t inc = v;
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) {
-        const uint32_t o = __shfl_up(inc, off);
-        if (lane >= off) inc += o;
-    }
-    total = __shfl(inc, WAVE - 1);
-    return inc - v;
 }
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
