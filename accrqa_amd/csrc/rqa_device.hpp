@@ -52,10 +52,12 @@ constexpr int WG = 256;            // threads per workgroup (4 waves)
 constexpr int WAVES = WG / WAVE;
 // k_lam, fp32 up to 16 thresholds: 4 waves per SIMD (128 VGPRs, a
 // few bytes spilled) instead of the compiler's 3 (measured: 61.8 -> 56.0 ms
-// on the default workload); the other instantiations keep what their
-// registers give (1 = no minimum).
+// on the default workload; maximal norm, a call at N = 30,000 with 6 to 16
+// thresholds 2-3 % less, at 9,000 1-2 % more); the other instantiations keep what
+// their registers give (1 = no minimum), and so does the maximal norm up to 4
+// thresholds (65,000: 1-3 % a call less without the minimum).
 #define RQA_WPE_LAM(F, NORM, TG) \
-    __attribute__((amdgpu_waves_per_eu((sizeof(F) == 4 && (TG) <= 16) ? 4 : 1)))
+    __attribute__((amdgpu_waves_per_eu((sizeof(F) == 4 && (TG) <= 16 && ((NORM) == 1 || (TG) > 4)) ? 4 : 1)))
 // k_lam_mx, k_det_mx: three waves per SIMD with the line scan (168 VGPRs for
 // 16 thresholds, no spills; left to itself the compiler takes a few registers
 // more and halves that), four without it (the LDS allows four workgroups).
