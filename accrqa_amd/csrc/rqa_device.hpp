@@ -1171,13 +1171,11 @@ __global__ __launch_bounds__(S) void k_rp_sq(const F *__restrict__ x, int64_t nc
                     for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xk[k]);
                 }
             }
-            F xv = m > RPK ? xj[(int64_t)RPK * tau] : F(0);
-            for (int k = RPK; k < m; k++) {   // the next dimension's sample is under way
-                const F xn = xj[(int64_t)(k + 1 < m ? k + 1 : k) * tau];
+            for (int k = RPK; k < m; k++) {
+                const F xv = xj[(int64_t)k * tau];
                 const F *xr = x + i0 + (int64_t)k * tau;
 #pragma unroll
                 for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xv);
-                xv = xn;
             }
 #pragma unroll
             for (int u = BLK - 1; u >= 0; u--) push_le(w, s[u], bound);
@@ -1275,13 +1273,11 @@ __global__ __launch_bounds__(WG) void k_rp_row(const F *__restrict__ x, int64_t 
                     for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xk[k]);
                 }
             }
-            F xv = m > RPK ? xj[(int64_t)RPK * tau] : F(0);
-            for (int k = RPK; k < m; k++) {   // the next dimension's sample is under way
-                const F xn = xj[(int64_t)(k + 1 < m ? k + 1 : k) * tau];
+            for (int k = RPK; k < m; k++) {
+                const F xv = xj[(int64_t)k * tau];
                 const F *xr = x + i0 + (int64_t)k * tau;
 #pragma unroll
                 for (int u = 0; u < BLK; u++) s[u] = dim_step<NORM>(s[u], xr[u], xv);
-                xv = xn;
             }
             uint32_t w = 0u;
 #pragma unroll

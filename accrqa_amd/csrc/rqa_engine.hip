@@ -1669,9 +1669,10 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
 // form, fp32 and Euclidean unless said):
 //   SMALL  blocks of 32 x 256, every element: enough workgroups for a small
 //          plot (1,500, m = 3: 11.6, 64-squares 14.2, k_rp4 12.7), with few
-//          dimensions also a larger one (3,600, m = 3: 15.0, 64-squares 15.5;
-//          m = 5: 16.6 and 16.5; maximal, m = 8: 20.1 and 18.5; with one
-//          dimension: 11,000: 31, 64-squares 37, k_rp4 33)
+//          dimensions also a larger one (3,073, m = 5: 14.8, 64-squares 16.4;
+//          3,600: 16.6 and 16.5; 4,097, m = 3: 16.5 and 17.1; 4,501: 17.9 and
+//          16.7; maximal, m = 8, 3,600: 20.1 and 18.5; with one dimension:
+//          11,000: 31, 64-squares 37, k_rp4 33)
 //   SQ64   64-squares, mirrored: while the plot fits the 256 MB last-level
 //          cache its short mirrored runs merge there (12,000, m = 3: 35,
 //          256-squares 43, rows 45; 20,000: 146, 134, 105).  More than 32
@@ -1695,7 +1696,7 @@ int device_fp64_diag(const float *d_in, size_t n, int tau, int emb, const float 
 enum { RP_SMALL, RP_SQ64, RP_SQ256, RP_ROWS };
 int rp_shape(int64_t nc, const void *out, int m, bool mx, bool cheap) {
     if (m == 1) return nc <= 13312 ? RP_SMALL : RP_ROWS;
-    if (nc <= 3072 || (nc <= 4096 && m <= 3)) return RP_SMALL;
+    if (nc <= 3072 || (nc <= 3328 && m <= 8) || (nc <= 4224 && m <= 3)) return RP_SMALL;
     if (mx && m > 32) return RP_SQ64;
     if (nc <= (mx && m > 16 ? 12288 : 16384)) return RP_SQ64;
     if (nc % 128 == 0 && (uintptr_t)out % 128 == 0) return RP_SQ256;
@@ -1705,14 +1706,14 @@ int rp_shape(int64_t nc, const void *out, int m, bool mx, bool cheap) {
 // Small plots in the exact form that stay with one store per decision: fp64
 // with k_rp4's waves of 8 rows, whose chains are a quarter as long as the
 // blocks' of 32 (500: 4.0 us in the kernel at m = 3, 4.4 in blocks; maximal,
-// m = 16: a call 13.3 and 15.9; 2,300, m = 32, Euclidean: 29.8 and 30.5), and
-// odd sizes in fp32 with many dimensions of the maximal norm (1,250, m = 32:
-// 18.3 and 19.4).
+// m = 16: a call 13.3 and 15.9; 2,300: 19.5 and 21.1; Euclidean, 2,000, m = 24:
+// 20.8 and 20.5), and odd sizes in fp32 with many dimensions (1,250, maximal,
+// m = 32: 18.3 and 19.4; Euclidean, m = 16, tau = 8: 14.9 and 15.6).
 template <typename F>
 bool rp_direct(int64_t nc, const void *out, int m, int dist) {
     if (sizeof(F) == 8)
-        return nc % 4 == 0 && (uintptr_t)out % 4 == 0 && (nc <= 1024 || (nc <= 3072 && m >= (dist == 1 ? 16 : 8)));
-    return dist == 2 && m >= 16 && nc % 4 != 0 && nc <= 1536;
+        return nc % 4 == 0 && (uintptr_t)out % 4 == 0 && (nc <= 1024 || (dist == 2 && m >= 8 && nc <= 3072));
+    return m >= 16 && nc % 4 != 0 && nc <= 1536;
 }
 
 unsigned rp_grid(int64_t nc, int64_t S) { return (unsigned)rqa::rp_items((nc + S - 1) / S); }

@@ -89,10 +89,11 @@ def test_row_ends(nc, m, dist, tail):
     (2049, 1, 8, 2, np.float32), (3071, 1, 9, 2, np.float64), (3072, 1, 8, 2, np.float64), (3072, 1, 8, 2, np.float32),
     (3072, 1, 7, 2, np.float64), (3072, 1, 16, 1, np.float64), (3072, 1, 15, 1, np.float64), (1024, 1, 1, 1, np.float64),
     (1028, 1, 2, 1, np.float64), (1022, 1, 8, 1, np.float64), (1535, 1, 16, 2, np.float32), (1537, 1, 16, 2, np.float32),
-    (1535, 1, 15, 2, np.float32), (2048, 1, 32, 1, np.float32), (2047, 1, 33, 1, np.float32), (4096, 1, 3, 2, np.float32),
+    (1535, 1, 15, 2, np.float32), (1535, 8, 16, 1, np.float32), (2048, 1, 32, 1, np.float32), (2047, 1, 33, 1, np.float32), (4096, 1, 3, 2, np.float32),
     (13312, 1, 1, 1, np.float32),
     # rows of one dimension, 64-squares
-    (13313, 1, 1, 2, np.float32), (3073, 1, 4, 2, np.float32), (4097, 1, 3, 2, np.float32), (4671, 2, 16, 1, np.float32), (4609, 3, 32, 1, np.float32),
+    (13313, 1, 1, 2, np.float32), (3328, 1, 8, 2, np.float32), (3329, 1, 8, 2, np.float32), (4224, 1, 3, 2, np.float32),
+    (4225, 1, 3, 2, np.float32), (4671, 2, 16, 1, np.float32), (4609, 3, 32, 1, np.float32),
     (4609, 1, 48, 1, np.float32), (4673, 1, 97, 1, np.float32), (4609, 2, 3, 1, np.float64), (16384, 1, 16, 1, np.float32),
     (12288, 1, 17, 1, np.float32), (16512, 1, 33, 1, np.float32),
     (16385, 1, 3, 2, np.float64), (45057, 1, 16, 1, np.float32)])
