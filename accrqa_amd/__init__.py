@@ -145,9 +145,10 @@ FORM_AUTO, FORM_EXACT, FORM_MFMA = 0, 1, 2
 
 def set_form(form):
     """Euclidean distance form: FORM_AUTO (MFMA Gram + exact recheck for
-    m >= 8, m >= 4 for plots of bytes with N_c > 16384), FORM_EXACT (exact VALU sums only) or FORM_MFMA (MFMA form wherever
-    it applies: fp32 input, and fp64 input in the LAM pass with the Gram of
-    the series rounded to fp32 and an fp64 recheck).  The Gram runs on FP16
+    m >= 8, m >= 4 for plots of bytes with N_c > 16384), FORM_EXACT (exact VALU
+    sums only) or FORM_MFMA (MFMA form wherever it applies: fp32 input, and fp64
+    input in RR, DET and LAM with the Gram of the series rounded to fp32 and an
+    fp64 recheck).  The Gram runs on FP16
     matrix cores with each sample split into two halves (hi/lo).  Results are identical; only
     speed differs."""
     e = load().accrqa_amd_set_form(int(form))

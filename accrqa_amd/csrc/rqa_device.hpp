@@ -64,9 +64,10 @@ constexpr int WAVES = WG / WAVE;
 #ifndef RQA_WPE_MX
 #define RQA_WPE_MX(scan) __attribute__((amdgpu_waves_per_eu((scan) ? 3 : 4)))
 #endif
-// The tile scans up to 16 thresholds: 7 waves per SIMD (<= 73 VGPRs), one
-// or two more than the compiler's own choice (measured on the default
-// workload: -0.8 ms for each LAM scan, -1.9 ms for k_det_scan).  At 32
+// The tile scans up to 24 thresholds: 7 waves per SIMD (<= 73 VGPRs; at 24
+// k_det_scan's LDS leaves it five, with 91), one or two more than the compiler's
+// own choice (measured on the default workload: -0.8 ms for each LAM scan,
+// -1.9 ms for k_det_scan).  At 32
 // thresholds the column and row scans take 6 (80 VGPRs, a few spilled; 3 %
 // off the million-sample call) and k_det_scan keeps what its registers give.
 #define RQA_WPE_SCAN(tg, n, n32) __attribute__((amdgpu_waves_per_eu((tg) == 32 ? (n32) : (n))))
@@ -502,7 +503,11 @@ __global__ __launch_bounds__(WG) RQA_WPE_LAM(F, NORM, TG) void k_lam(const F *__
     const int64_t nbands = (nc + WAVE - 1) / WAVE;
     const int64_t nitems = W.items ? W.nitems : nbands * W.nseg;
     const size_t cstride = (size_t)W.cseg * nc;   // carry stride between thresholds
-    constexpr int MJ = 4;  // column samples kept in registers (16 cost a wave per SIMD and served few calls)
+    // Column samples kept in registers.  Against sixteen (eight in fp64), a call in
+    // this form: maximal norm, N = 65,000, m = 8, 12 thresholds 4.01 -> 3.92 ms, 32
+    // thresholds 6.71 -> 6.06; Euclidean, m = 6, 32 thresholds 10.5 -> 9.2; at most
+    // 4 % more at N = 9,000 with 12 or more dimensions and 17 to 24 thresholds.
+    constexpr int MJ = 4;
 
     for (int64_t item = (int64_t)blockIdx.x * WAVES + wave; item < nitems; item += (int64_t)gridDim.x * WAVES) {
         int64_t band;

@@ -4,16 +4,19 @@
 // One call handles one (tau, emb) block for all thresholds: thresholds are
 // turned into exact comparison bounds, sorted, split into groups of 4/8/16/24/32
 // (one pass over the pairs per group), and each group runs on one HIP stream
-//   RR alone:   k_rr -> k_rr_out
+//   RR alone:   k_rr | k_rr_mx -> k_rr_out
 //   LAM:        k_lam | k_lam_mx (column pass; keeps the rank tiles when they
 //               fit, and then leaves the column runs to k_lam_vscan in the
 //               MFMA form) [-> k_lam_hscan] -> k_stitch -> k_finalize, RR from
-//               its histogram -> k_rr_out
-//   DET:        k_det_scan (from the tiles) | k_det | k_det_mx -> k_stitch
-//               -> k_finalize
-// (k_lam_mx / k_det_mx: MFMA Gram form, with k_norms and k_mx_lut first).  Device buffers live in a per-process context that grows
-// on demand and is reused across calls (the reference allocates and frees per
-// call, src/AccRQA-GPU-HST.cu:1855-1945).
+//               its histogram
+//   DET:        k_det_scan (from the LAM pass's tiles, beside its scans; asked
+//               alone in the MFMA form, from a k_lam_mx pass that only ranks)
+//               | k_det | k_det_mx -> k_stitch -> k_finalize
+// LAM and DET asked together end in one k_stitch and one k_finalize (k_lam_mx,
+// k_rr_mx, k_det_mx: MFMA Gram form, with k_norms and k_mx_lut first).  Device
+// buffers live in a per-process context that grows on demand and is reused
+// across calls (the reference allocates and frees per call,
+// src/AccRQA-GPU-HST.cu:1855-1945).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -93,9 +96,9 @@ ItemSet g_items[NITEMSETS];
 RrItemSet g_rr_items[NITEMSETS];
 uint64_t g_items_clock = 0;
 
-// Euclidean distance form: 0 = automatic (MFMA Gram + exact recheck for fp32
-// input with m >= 8, exact VALU sums otherwise), 1 = exact VALU sums only,
-// 2 = MFMA + recheck wherever it applies (fp32 input, Euclidean norm).
+// Euclidean distance form: 0 = automatic (MFMA Gram + exact recheck with
+// m >= 8, exact VALU sums otherwise), 1 = exact VALU sums only, 2 = MFMA +
+// recheck wherever it applies (use_mfma).
 int g_form = 0;
 
 // LAM/DET split through kept rank tiles: 0 = when the tiles fit, 1 = never.
@@ -140,8 +143,9 @@ int g_scan_waves = 7;
 // order into the context's mxstats buffer (3 u64).
 bool g_mxstats = false;
 
-// MFMA form for F = float and, in the LAM pass, F = double (hi/lo Gram of the
-// series rounded to fp32, exact re-decision in fp64); the direct DET kernel is fp32-only.
+// MFMA form for F = float and for F = double (hi/lo Gram of the series rounded
+// to fp32, exact re-decision in fp64; the LAM pass, RR alone and DET alone from
+// the tiles); the direct DET kernel and the plot kernels are fp32-only.
 template <typename F>
 bool use_mfma(int dist, int m, int tau) {
     if (dist != 1) return false;
@@ -536,7 +540,11 @@ int64_t seg_by_items(int64_t nc) {
 // steps and the items' 65,536 alone, and so: N = 700: 165 / 168, 117 / 146;
 // 3,000: 173 / 178, 151 / 179; 16,000: 416 / 414, 388 / 343; 32,000: 1100 / 971,
 // 1009 / 769; 65,000: 3731 / 2376, 3720 / 2199.  Half and twice these lengths were
-// slower at most of the sizes (16,000, m = 16, half: 498).
+// slower at most of the sizes (16,000, m = 16, half: 498).  Neutral from 7,000 to
+// 9,000, where both rules cut nearly alike, and not everywhere a gain: with 20
+// thresholds, m = 3, 5,000: 288 and 308, 10,000: 623 and 679; DET, fp64, m = 3,
+// 10,000: 182 and 199; RR, DET and LAM in one call with 3 thresholds, m = 16, 1,500:
+// 95 and 100, 5,000: 120 and 123.
 int seg_len_for(int64_t nc) {
     const int64_t nseg = nc > 16384 && nc <= 49152 ? 40 : 32;
     return seg_of(std::max(seg_by_items(nc), std::max<int64_t>((nc + nseg - 1) / nseg, 64)));

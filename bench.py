@@ -100,10 +100,10 @@ def tile_store_bytes(nc):
 # (FETCH_SIZE reads 0.5 GiB for it: x2.0; WRITE_SIZE 1 GiB: x1.0).
 _TRAFFIC_SRC = "profiles/ar1_m16_traffic.md"
 MEASURED_TRAFFIC = {
-    ("ar1_m16", "k_lam_mx"): (2.0 * 0.9967e9 + 34.373e9, _TRAFFIC_SRC),
-    ("ar1_m16", "k_lam_vscan"): (2.0 * 17.305e9 + 5.311e9, _TRAFFIC_SRC),
-    ("ar1_m16", "k_lam_hscan"): (2.0 * 17.287e9 + 5.291e9, _TRAFFIC_SRC),
-    ("ar1_m16", "k_det_scan"): (2.0 * 25.343e9 + 4.015e9, _TRAFFIC_SRC),
+    ("ar1_m16", "k_lam_mx"): (2.0 * 1.0121e9 + 34.373e9, _TRAFFIC_SRC),
+    ("ar1_m16", "k_lam_vscan"): (2.0 * 17.296e9 + 1.679e9, _TRAFFIC_SRC),
+    ("ar1_m16", "k_lam_hscan"): (2.0 * 17.287e9 + 2.617e9, _TRAFFIC_SRC),
+    ("ar1_m16", "k_det_scan"): (2.0 * 25.333e9 + 3.211e9, _TRAFFIC_SRC),
 }
 
 
@@ -114,11 +114,11 @@ MEASURED_TRAFFIC = {
 # v_bitop3 and 1.87 for FP32 adds.
 _ISSUE_SRC = "profiles/ar1_m16_instruction_mix.md"
 MEASURED_VALU = {
-    ("ar1_m16", "k_lam_vscan"): 7.029e9,
-    ("ar1_m16", "k_lam_hscan"): 7.298e9,
-    ("ar1_m16", "k_det_scan"): 7.122e9,
-    ("ar1_m16", "k_lam_mx"): 6.634e9,
-    ("ar1_m16", "k_lam"): 3.921e10,
+    ("ar1_m16", "k_lam_vscan"): 7.426e9,
+    ("ar1_m16", "k_lam_hscan"): 7.648e9,
+    ("ar1_m16", "k_det_scan"): 7.525e9,
+    ("ar1_m16", "k_lam_mx"): 6.095e9,
+    ("ar1_m16", "k_lam"): 3.894e10,
 }
 CU_COUNT, CLOCK_GHZ = 256, 2.4
 

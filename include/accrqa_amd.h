@@ -194,9 +194,11 @@ int accrqa_amd_rp_device_f64(const double *d_input, size_t data_size, int tau, i
 
 /* Form of the Euclidean distance (no counterpart in the reference, which has
  * one form per platform).  0 = automatic: the MFMA form for emb >= 8 (emb >= 4
- * for plots of bytes with N_c > 16384), exact VALU sums otherwise; 1 = exact VALU sums only; 2 = MFMA form wherever it
- * applies (Euclidean norm; fp32 input, and fp64 input in the LAM pass, whose
- * Gram then runs on the series rounded to fp32).  The MFMA form computes
+ * for plots of bytes with N_c > 16384), exact VALU sums otherwise; 1 = exact
+ * VALU sums only; 2 = MFMA form wherever it applies (Euclidean norm, a window
+ * (emb - 1) tau <= 96; fp32 input, and fp64 input in RR, DET and LAM, whose Gram
+ * then runs on the series rounded to fp32; not DET alone of fp64 input without
+ * the rank tiles, nor fp64 plots).  The MFMA form computes
  * |x_i|^2 + |x_j|^2 - 2 x_i.x_j with the Gram tile on FP16 matrix cores
  * (each scaled sample split into two halves, hi/lo) and
  * re-decides every pair within a rigorous error bound of a threshold in the
